@@ -5,15 +5,19 @@
 // The attention backward leaves dy (the gradient of the normalized, unrotated
 // rows, in the caller's dq / dk buffer and dtype, as the unfused path holds
 // it); norm_bwd_kernel turns it into dx in place and writes one fp32 partial
-// of dw per workgroup; norm_dw_reduce_kernel sums the partials in a fixed
-// order (no atomics: the result does not depend on scheduling).
+// of dw per workgroup; norm_dw_reduce_kernel sums the partials of both sides
+// in a fixed order (no atomics: the result does not depend on scheduling).
 // norm_rows_kernel writes the normalized rows themselves, for the backward
 // kernels that read q / k rows directly instead of through the MFMA path's
 // operand images.
 //
 // Row layout: a group of D/8 lanes holds one row, 8 elements per lane
 // (16-byte loads at 16-bit dtypes); a wave covers 512/D rows at a time and a
-// workgroup of 4 waves kNormRows rows of one (sequence, head).
+// workgroup of 4 waves kNormRows rows of one (sequence, head), all of whose
+// loads are issued before the first row's reductions. The kernel is bound by
+// HBM where the grid fills the GPU and by one round trip to it where it does
+// not: 256 rows one after the other took 28.6 us for the k rows of B=2, T=4096,
+// 8 heads, D=128 bf16 (256 workgroups, 50 MB) whatever their number.
 
 #include "common.h"
 #include "launch.h"
@@ -22,7 +26,7 @@
 namespace goda {
 namespace {
 
-constexpr int kNormRows = 256;  // rows per workgroup
+constexpr int kNormRows = 64;  // rows per workgroup
 
 template <typename T, int D>
 struct NormGeom {
@@ -67,46 +71,54 @@ __global__ void __launch_bounds__(256) norm_rows_kernel(const goda_prefill_args 
     g[e] = 1.f + n.w[c + e];
     acc[e] = 0.f;
   }
-  const int first = blockIdx.x * kNormRows;
-  // The row loop is uniform over the workgroup: every lane of a row group
-  // takes part in its reductions (rows past the sequence load zeros).
-  for (int r = first + wave * NG::RPW + sub; r < first + kNormRows; r += 4 * NG::RPW) {
-    const bool ok = r < len;
-    const int64_t row = row0 + r;
-    const T* xp = reinterpret_cast<const T*>(n.x) + (varlen ? 0 : (int64_t)b * n.x_sb) + row * n.x_st + (int64_t)h * n.x_sh + c;
-    T* yp = reinterpret_cast<T*>(n.y) + (varlen ? 0 : (int64_t)b * n.y_sb) + row * n.y_st + (int64_t)h * n.y_sh + c;
-    v8 xv = {};
-    if (ok) xv = ld_vec<v8>(xp);
+  // Every lane of a row group takes part in its reductions (rows past the
+  // sequence load zeros).
+  constexpr int STEPS = kNormRows / NG::SLOTS;
+  static_assert(kNormRows % NG::SLOTS == 0, "whole rounds of the row groups");
+  const int first = blockIdx.x * kNormRows + wave * NG::RPW + sub;
+  const T* xb = reinterpret_cast<const T*>(n.x) + (varlen ? 0 : (int64_t)b * n.x_sb) + (int64_t)h * n.x_sh + c;
+  T* yb = reinterpret_cast<T*>(n.y) + (varlen ? 0 : (int64_t)b * n.y_sb) + (int64_t)h * n.y_sh + c;
+  v8 xv[STEPS], dv[STEPS];
+#pragma unroll
+  for (int k = 0; k < STEPS; ++k) {
+    const int r = first + k * NG::SLOTS;
+    xv[k] = dv[k] = v8{};
+    if (r < len) {
+      xv[k] = ld_stream<v8>(xb + (row0 + r) * n.x_st);
+      if (BWD) dv[k] = ld_stream<v8>(yb + (row0 + r) * n.y_st);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < STEPS; ++k) {
+    const int r = first + k * NG::SLOTS;
+    T* yp = yb + (row0 + r) * n.y_st;
     float x[8];
     float ss = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      x[e] = (float)xv[e];
+      x[e] = (float)xv[k][e];
       ss = fmaf(x[e], x[e], ss);
     }
     const float rs = rms_scale(lane_group_sum<NG::LPR>(ss), D, n.eps);
+    v8 out;
     if (!BWD) {
-      v8 out;
 #pragma unroll
       for (int e = 0; e < 8; ++e) out[e] = (T)(x[e] * rs * g[e]);
-      if (ok) st_vec<v8>(yp, out);
+      if (r < len) st_vec<v8>(yp, out);
       continue;
     }
-    v8 dv = {};
-    if (ok) dv = ld_vec<v8>(yp);
     float dy[8], t = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      dy[e] = (float)dv[e];
+      dy[e] = (float)dv[k][e];
       x[e] *= rs;  // x^
       t = fmaf(x[e] * g[e], dy[e], t);
       acc[e] = fmaf(x[e], dy[e], acc[e]);
     }
     const float m = lane_group_sum<NG::LPR>(t) / (float)D;
-    v8 out;
 #pragma unroll
     for (int e = 0; e < 8; ++e) out[e] = (T)(rs * (g[e] * dy[e] - x[e] * m));
-    if (ok) st_vec<v8>(yp, out);
+    if (r < len) st_vec<v8>(yp, out);
   }
   if (!BWD) return;
   // dw partial of this workgroup: row groups in slots, summed in slot order.
@@ -123,13 +135,44 @@ __global__ void __launch_bounds__(256) norm_rows_kernel(const goda_prefill_args 
   }
 }
 
-__global__ void __launch_bounds__(256) norm_dw_reduce_kernel(const float* part, int64_t nparts, int d_model,
-                                                             float* dw) {
-  const int d = blockIdx.x * 256 + threadIdx.x;
-  if (d >= d_model) return;
-  float s = 0.f;
-  for (int64_t k = 0; k < nparts; ++k) s += part[k * d_model + d];
-  dw[d] = s;
+// The partials of one norm weight: dw[d] = sum over k < n of part[k][d].
+struct DwSum {
+  const float* part;
+  int64_t n;
+  float* dw;  // nullptr: this side is not wanted
+};
+
+// A workgroup sums 16 columns of one side (blockIdx.y): 64 rows of 4 lanes
+// take every 64th partial, four in flight, and meet in LDS in row order. One
+// thread per column over all partials was a serial chain of loads in a single
+// workgroup: 232 us for the 1024 partials of B=2, T=4096, 32 heads, D=128
+// (a training pass at that size, 8 KV heads, bf16, with this reduction and 64
+// rows per workgroup above: 1558 -> 1256 us).
+constexpr int kDwCols = 16, kDwRows = 64;
+__global__ void __launch_bounds__(256) norm_dw_reduce_kernel(const DwSum q, const DwSum k, int head_dim) {
+  const DwSum u = blockIdx.y == 0 ? q : k;
+  if (!u.dw) return;  // (the whole workgroup)
+  const int row = threadIdx.x >> 2, c = 4 * (threadIdx.x & 3);
+  const int d = blockIdx.x * kDwCols + c;
+  f32x4 s = {};
+#pragma unroll 4
+  for (int64_t i = row; i < u.n; i += kDwRows) s += ld_vec<f32x4>(u.part + i * head_dim + d);
+  __shared__ __align__(16) float sums[kDwRows][kDwCols];
+  st_vec<f32x4>(&sums[row][c], s);
+  __syncthreads();
+  if (threadIdx.x < kDwCols) {
+    float t = 0.f;
+#pragma unroll 8
+    for (int r = 0; r < kDwRows; ++r) t += sums[r][threadIdx.x];
+    u.dw[blockIdx.x * kDwCols + threadIdx.x] = t;
+  }
+}
+
+hipError_t launch_dw_reduce(const DwSum& q, const DwSum& k, int head_dim, hipStream_t s) {
+  if (!q.dw && !k.dw) return hipSuccess;
+  // head_dim is 64, 128 or 256: whole column blocks
+  norm_dw_reduce_kernel<<<dim3(head_dim / kDwCols, 2), 256, 0, s>>>(q, k, head_dim);
+  return hipGetLastError();
 }
 
 template <typename T, int D>
@@ -197,19 +240,15 @@ hipError_t launch_norm_rows(const goda_prefill_args& a, bool q_side, void* dst, 
 }
 
 hipError_t zero_norm_dw(const goda_prefill_args& a, const goda_prefill_grads& g, hipStream_t s) {
-  for (int side = 0; side < 2; ++side) {
-    const float* w = side == 0 ? a.q_norm_weight : a.k_norm_weight;
-    float* dw = side == 0 ? g.dq_norm_weight : g.dk_norm_weight;
-    if (!w || !dw) continue;
-    norm_dw_reduce_kernel<<<(a.head_dim + 255) / 256, 256, 0, s>>>(nullptr, 0, a.head_dim, dw);  // sums nothing: 0
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
+  // sums of nothing: 0
+  const DwSum q{nullptr, 0, a.q_norm_weight ? g.dq_norm_weight : nullptr};
+  const DwSum k{nullptr, 0, a.k_norm_weight ? g.dk_norm_weight : nullptr};
+  return launch_dw_reduce(q, k, a.head_dim, s);
 }
 
 hipError_t launch_norm_bwd(const goda_prefill_args& a, const goda_prefill_grads& g, float* part, hipStream_t s) {
   hipError_t e;
+  DwSum sum[2] = {};
   for (int side = 0; side < 2; ++side) {
     const bool q_side = side == 0;
     const float* w = q_side ? a.q_norm_weight : a.k_norm_weight;
@@ -232,14 +271,10 @@ hipError_t launch_norm_bwd(const goda_prefill_args& a, const goda_prefill_grads&
     n.q_side = q_side;
     if ((e = launch_rows_any(a, n, true, seqlen, s)) != hipSuccess) return e;
     const int64_t np = parts(seqlen, heads, a.batch);
-    float* dw = q_side ? g.dq_norm_weight : g.dk_norm_weight;
-    if (dw) {  // np == 0 writes zeros
-      norm_dw_reduce_kernel<<<(a.head_dim + 255) / 256, 256, 0, s>>>(part, np, a.head_dim, dw);
-      if ((e = hipGetLastError()) != hipSuccess) return e;
-    }
+    sum[side] = DwSum{part, np, q_side ? g.dq_norm_weight : g.dk_norm_weight};
     part += np * a.head_dim;
   }
-  return hipSuccess;
+  return launch_dw_reduce(sum[0], sum[1], a.head_dim, s);
 }
 
 }  // namespace goda

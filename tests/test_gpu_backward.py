@@ -446,3 +446,11 @@ def test_backward_fused_qk_norm_weight_gradients_are_deterministic():
     again = ops.attention_prefill_bwd(qg, kg, vg, o, lse, d_o.to(DEV), **kw)
     for a_, b_ in zip(grads[3:], again[3:]):
         assert torch.equal(a_, b_)
+
+
+@pytest.mark.parametrize("b,t,hq,hkv", [(1, 1, 1, 1), (1, 63, 2, 1), (1, 65, 33, 1), (3, 129, 32, 8)])
+@pytest.mark.parametrize("d", [64, 256])
+def test_backward_fused_qk_norm_partial_sums(b, t, hq, hkv, d):
+    """The rows of a norm workgroup (64) and the partials of a reduction round
+    (64), one less, one more and several rounds, on both sides."""
+    _norm_case(b, t, t, hq, hkv, d, torch.bfloat16, rope=False, seed=53)
