@@ -104,6 +104,11 @@ goda::PrefillParams make_prefill_params(const goda_prefill_args* a) {
   return p;
 }
 
+int64_t prefill_workspace_bytes(const goda_prefill_args& a) {
+  if (goda::prefill_f32_streams(a)) return goda::prefill_f32_workspace_bytes(a);
+  return goda::prefill_mfma_supported(a) ? goda::prefill_mfma_workspace_bytes(a) : 0;
+}
+
 // Checks of goda_attn_decode / goda_attn_decode_noalloc (everything but the
 // workspace); returns GODA_OK or a failure status.
 int32_t check_decode(const goda_decode_args* a) {
@@ -164,8 +169,7 @@ const char* goda_attn_last_error(void) { return g_last_error.c_str(); }
 int64_t goda_attn_prefill_workspace_size(const goda_prefill_args* a) {
   const int32_t st = check_prefill(a, false);
   if (st != GODA_OK) return st;
-  if (goda::prefill_mfma_supported(*a)) return goda::prefill_mfma_workspace_bytes(*a);
-  return 0;
+  return prefill_workspace_bytes(*a);
 }
 
 int32_t goda_attn_prefill_fwd(const goda_prefill_args* a, void* stream) {
@@ -174,13 +178,15 @@ int32_t goda_attn_prefill_fwd(const goda_prefill_args* a, void* stream) {
   if (a->batch == 0 || a->seqlen_q == 0) return ok();
   goda::PrefillParams p = make_prefill_params(a);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (goda::prefill_mfma_supported(*a)) {
-    const int64_t need = goda::prefill_mfma_workspace_bytes(*a);
-    if (need > 0 && (!a->workspace || a->workspace_bytes < need))
-      return fail(GODA_ERR_WORKSPACE, "prefill: workspace of %lld bytes needed, %lld given",
-                  (long long)need, (long long)a->workspace_bytes);
-    return hip_status(goda::launch_prefill_mfma(p, s), "prefill_fwd");
+  const int64_t need = prefill_workspace_bytes(*a);
+  if (need > 0 && (!a->workspace || a->workspace_bytes < need)) {
+    // (fp32 at head_dim 256 also runs without a workspace, on the vector ALUs)
+    if (!goda::prefill_mfma_supported(*a)) return hip_status(goda::launch_prefill_generic(p, s), "prefill_fwd");
+    return fail(GODA_ERR_WORKSPACE, "prefill: workspace of %lld bytes needed, %lld given",
+                (long long)need, (long long)a->workspace_bytes);
   }
+  if (goda::prefill_f32_streams(*a)) return hip_status(goda::launch_prefill_f32(p, s), "prefill_fwd");
+  if (goda::prefill_mfma_supported(*a)) return hip_status(goda::launch_prefill_mfma(p, s), "prefill_fwd");
   return hip_status(goda::launch_prefill_generic(p, s), "prefill_fwd");
 }
 

@@ -21,6 +21,7 @@ struct PrefillParams {
   int qtiles;         // query tiles per (sequence, head slice) in the grid (MFMA path)
   int persist_slots;  // persistent grid: resident workgroups per XCD (0: one workgroup per item)
   int persist_pairs;  // persistent grid: (sequence, head slice) pairs per XCD
+  int key_split;      // fp32: waves of a workgroup sharing an item's key tiles
 };
 
 struct DecodeParams {
@@ -93,6 +94,18 @@ hipError_t launch_prefill_generic(const PrefillParams& p, hipStream_t s);
 bool prefill_mfma_supported(const goda_prefill_args& a);
 int64_t prefill_mfma_workspace_bytes(const goda_prefill_args& a);
 hipError_t launch_prefill_mfma(const PrefillParams& p, hipStream_t s);
+
+// fp32 prefill on the matrix cores with operands streamed from L2: head_dim
+// 256 (more than two key tiles), and 64 / 128 where the work is small.
+bool prefill_f32_streams(const goda_prefill_args& a);
+int64_t prefill_f32_workspace_bytes(const goda_prefill_args& a);
+hipError_t launch_prefill_f32(const PrefillParams& p, hipStream_t s);
+// Waves that share the key tiles of an fp32 item (32 query rows of one head):
+// enough that `items` fill the GPU, at most one per key tile.
+inline int f32_key_split(int64_t items, int ntiles_k) {
+  const int split = items <= 2048 ? 4 : items <= 4096 ? 2 : 1;
+  return ntiles_k < split ? (ntiles_k >= 2 ? 2 : 1) : split;
+}
 
 // Split-K decode (bf16 / fp16 / fp32).
 int64_t decode_slots(const goda_decode_args& a);

@@ -122,6 +122,29 @@ __device__ __forceinline__ void mfma_vgpr_drain(f32x16& x, f32x16& y) {
   asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" : "+v"(x), "+v"(y));
 }
 
+// Dispatch order of a grid of `units` x `nblk` workgroups whose work falls
+// with the block index (block 0: the earliest keys, or the last query tile,
+// which the most causal rows / keys reach). Unit after unit, the last unit's
+// heaviest block would start when little work is left (simulated makespan
+// 1.19-1.23x the ideal at the cfg2 shape); here units go in chunks of
+// kOrderChunk, heaviest block of every unit of the chunk first (1.0x).
+// Measured: cfg2-shape backward 13.5 -> 10.7 ms, cfg3 shape 9.2 -> 6.4 ms
+// (chunks of 8, 16 and 32 alike then; 4: 10.7 and 7.3 ms).
+// Chunks of 8: consecutive workgroups go round-robin to the 8 XCDs, so every
+// block of one unit runs on the same XCD and each XCD runs one unit at a
+// time. With the dk/dv walk that reads the same query tiles in every key
+// block of a unit, one unit per XCD halves the distinct tiles streaming
+// through each L2 (16: two units per XCD): cfg2-shape dk/dv 5.10 -> 4.89 ms,
+// dq 2.99 -> 2.89 ms.
+constexpr int kOrderChunk = 8;
+__device__ __forceinline__ void chunked_order(int lin, int nblk, int units, int& unit, int& blk) {
+  const int base = lin / (kOrderChunk * nblk) * kOrderChunk;
+  const int cc = min(kOrderChunk, units - base);
+  const int r = lin - base * nblk;
+  blk = r / cc;
+  unit = base + r % cc;
+}
+
 // Workgroup barrier for the tile rings. __syncthreads() would also wait for
 // every outstanding global access (vmcnt(0)), i.e. for the registers of the
 // tile being prefetched; a ring only needs this wave's LDS accesses retired.

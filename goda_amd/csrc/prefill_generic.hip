@@ -1,8 +1,7 @@
-// Generic prefill attention on the vector ALUs, fp32 arithmetic throughout.
-// The product path for fp32 at head_dim 256 (goda's default model dtype is
-// fp32, mint/nn/models.py:23), whose operands do not fit the matrix-core
-// kernel's register and LDS budgets; every other dtype / head_dim runs on
-// prefill_mfma.hip.
+// Generic prefill attention on the vector ALUs, fp32 arithmetic throughout,
+// with no pre-pass and no workspace: fp32 at head_dim 256 over at most two key
+// tiles (64 keys), or where the caller gives no workspace; everything else
+// runs on prefill_f32.hip or prefill_mfma.hip.
 //
 // Work split: one workgroup of 256 threads per (64-query block, query head,
 // sequence). Four threads share a query row; thread `part` owns head-dim

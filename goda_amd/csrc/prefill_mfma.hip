@@ -1152,7 +1152,7 @@ struct Config<T, 128> {
 };
 template <typename T>
 struct Config<T, 256> {
-  static_assert(sizeof(T) == 2, "fp32 at head_dim 256 takes the generic kernel");
+  static_assert(sizeof(T) == 2, "fp32 at head_dim 256 takes prefill_f32.hip");
   static constexpr int BKV = 32, NT = 1, WAVES = 8;
 };
 

@@ -2,12 +2,13 @@
 
 from __future__ import annotations
 
+import ctypes
 import math
 
 import pytest
 import torch
 
-from goda_amd import ops
+from goda_amd import _lib, ops
 from goda_amd import workloads as wl
 from oracle import attention as ref
 from tests.helpers import TOL, lse_err, max_err, report, rope_oracle, wave_block_rows
@@ -429,3 +430,48 @@ def test_cfg3_mqa_alibi_block_rows():
 
 def test_cfg5_varlen_prefill_block_rows():
     _check_prefill_workload(wl.CFG5.prefill, rows_per_seq=16)
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("b,tq,tk,hq,hkv,causal,window", [
+    (1, 1, 1, 1, 1, True, -1),  # one row, one key
+    (1, 31, 97, 3, 1, True, -1),  # a partial query tile over a partial fourth key tile
+    (2, 33, 33, 6, 2, True, -1),  # two query tiles, idle rows
+    (1, 160, 160, 5, 5, True, 32),  # windowed: two key tiles a query tile
+    (1, 70, 200, 4, 1, False, -1),
+    (1, 96, 40, 2, 1, True, -1),  # rows without a key
+    (2, 2081, 2081, 24, 8, True, -1),  # more than 3072 items: the LDS ring at D <= 128
+])
+def test_prefill_fp32_streamed(d, b, tq, tk, hq, hkv, causal, window):
+    """fp32 on streamed operands: the edges of its 32-row tiles, each way of
+    splitting an item's keys over a workgroup's waves, and both sides of the
+    rule that chooses it."""
+    rope = tq <= tk
+    if tq > 2048:
+        _run_rows(b, tq, tk, hq, hkv, d, causal)
+    else:
+        _run_case(b, tq, tk, hq, hkv, d, torch.float32, causal, seed=d + tq, window=window, rope=rope)
+
+
+def _run_rows(b, tq, tk, hq, hkv, d, causal):
+    """fp32 parity on the first and last row of every query tile."""
+    q, k, v = _rand((b, tq, hq, d), torch.float32, 1), _rand((b, tk, hkv, d), torch.float32, 2), _rand((b, tk, hkv, d), torch.float32, 3)
+    o = ops.attention_prefill(q.to(DEV), k.to(DEV), v.to(DEV), causal=causal)
+    rows = wave_block_rows(tq)
+    o_ref, _ = ref.attention_rows(q, k, v, rows, causal=causal)
+    assert max_err(o[:, rows.to(DEV)], o_ref) <= TOL[torch.float32]
+
+
+@pytest.mark.parametrize("tk", [64, 65, 200])
+def test_prefill_fp32_wide_without_workspace(tk):
+    """fp32 at head_dim 256: a call without a workspace gives the same result
+    (on the vector ALUs) as one with the workspace that the query asks for."""
+    q, k, v = _rand((2, tk, 4, 256), torch.float32, 1).to(DEV), _rand((2, tk, 2, 256), torch.float32, 2).to(DEV), _rand((2, tk, 2, 256), torch.float32, 3).to(DEV)
+    plan = ops.plan_prefill(q, k, v, causal=True)
+    want = plan().clone()
+    plan.args.workspace, plan.args.workspace_bytes = None, 0
+    plan.result.zero_()
+    got = plan()
+    torch.cuda.synchronize()
+    assert (_lib.load().goda_attn_prefill_workspace_size(ctypes.byref(plan.args)) > 0) == (tk > 64)
+    assert max_err(got, want) <= 1e-5
