@@ -215,8 +215,6 @@ int32_t goda_attn_prefill_bwd(const goda_prefill_args* a, const goda_prefill_gra
   p.g = *g;
   p.group = a->heads_q / a->heads_kv;
   p.scale_log2 = a->softmax_scale * 1.4426950408889634f;
-  p.delta_rows = (int64_t)a->batch * a->seqlen_q;
-  p.delta = reinterpret_cast<float*>(g->workspace);
   return hip_status(goda::launch_prefill_bwd(p, reinterpret_cast<hipStream_t>(stream)), "prefill_bwd");
 }
 

@@ -1,6 +1,6 @@
 // Backward of prefill attention on gfx950 matrix cores: bf16 / fp16 operands
-// at head_dim 64, 128 or 256, fp32 operands at head_dim 64 or 128 (fp32 at 256
-// takes the generic kernels of backward.hip); fp32 accumulation.
+// at head_dim 64, 128 or 256, fp32 accumulation (fp32 operands:
+// backward_f32.hip).
 // Same quantities as kernels_/flash_attn_gqa/cuda.py:6-246:
 //   P = exp(scale q k^T + bias - lse), dV = P^T dO, dP = dO V^T,
 //   dS = P * (dP - delta) with delta = rowsum(dO * O),
@@ -10,15 +10,12 @@
 //   1. pack_q_bwd_kernel: per (32-row query tile, query head, sequence),
 //      the row-major operand images of rotated q (prescaled) and of dO
 //      ("chunk-column-major" [D/8][32] 16-byte chunks, the A operand of a
-//      product over head_dim), plus the row statistics lse*log2(e) and
-//      delta; for fp32 also the transposed images ([32/8][D] chunks with the
-//      rows of each 16-row group in kPermKey order, the A operand of a
-//      product over rows). The 16-bit kernels read those operands out of the
-//      row-major images with transposing LDS reads (ds_read_b64_tr_b16).
+//      product over head_dim), plus the row statistics lse*log2(e) and delta.
+//      The operands of products over rows are read out of the same images
+//      with transposing LDS reads (ds_read_b64_tr_b16).
 //   2. pack_kv_bwd_kernel: per (32-key tile, KV head, sequence), the
-//      row-major images of rotated k and of v and, for fp32, the transposed
-//      image of k (the 16-bit dq kernels read k^T out of the row-major image
-//      with transposing LDS reads).
+//      row-major images of rotated k and of v (k^T likewise by transposing
+//      reads).
 //   3. bwd_dkv_mfma_kernel: one workgroup of 8 waves per 128 keys of a KV
 //      head, in pairs (two waves of one SIMD) that share 32 keys; the pair
 //      pins the k and v operands of its keys and walks the query tiles of
@@ -41,10 +38,9 @@
 //      dO operands of its 32 rows and walks the key tiles:
 //        S^T  [keys][rows] = K Q^T         A = k image,   B = q (registers)
 //        dP^T [keys][rows] = V dO^T        A = v image,   B = dO (registers)
-//        dQ^T [d][rows]   += K^T dS^T      A = K^T (image or transposing reads), B = dS^T (packed)
-// A packed accumulator becomes a B operand directly because the transposed
-// operands (fp32 images, or transposing reads of the row-major images) hold
-// their rows / keys in the accumulator's register order (kPermKey). With the
+//        dQ^T [d][rows]   += K^T dS^T      A = K^T (transposing reads), B = dS^T (packed)
+// A packed accumulator becomes a B operand directly because the transposing
+// reads hand out rows / keys in the accumulator's register order (kPermKey). With the
 // log-sum-exp known there is no online softmax.
 
 #include <algorithm>
@@ -60,57 +56,43 @@ constexpr int kQRows = 32;   // rows per query tile
 constexpr int kBKV = 32;     // keys per key tile
 // dq workgroup: two waves per SIMD, or one at head_dim 256 (q and dO operands
 // plus the dQ^T accumulator take ~350 registers there).
-template <typename T, int D>
+template <int D>
 struct DqShape {
-  static constexpr bool WIDE = D >= 256 || sizeof(T) == 4;
+  static constexpr bool WIDE = D >= 256;
   static constexpr int WAVES = WIDE ? 4 : 8;
   static constexpr int OCC = WIDE ? 1 : 2;
 };
 
-// Images are counted in 8-element chunks (16 bytes, or 32 for fp32).
-// The transposed q and dO images (QT, GT) exist only for fp32 operands, which
-// have no transposing LDS read; the 16-bit dk/dv kernels read those operands
-// out of the row-major images (tr_operand). Without them the dK accumulators
-// multiply the prescaled q image: dk = ln(2) * dK^T (kDkScale).
+// Images are counted in 8-element chunks of 16 bytes. The dK accumulators
+// multiply the prescaled q image (q * scale * log2(e)): dk = ln(2) * dK^T.
 template <typename T, int D>
 struct QImg {
   static constexpr int CHB = (int)sizeof(typename Vec<T>::v8);
   static constexpr int CH = D / 8 * kQRows;  // chunks of one image
-  static constexpr bool HAS_T = sizeof(T) == 4;
-  static constexpr int NIMG = HAS_T ? 4 : 2;
-  static constexpr int QA = 0, GA = CH, QT = 2 * CH, GT = 3 * CH;
+  static constexpr int NIMG = 2;
+  static constexpr int QA = 0, GA = CH;
   // Row-major images: chunk (c, r) (head-dim 8c..8c+7 of row r) at
-  // c*32 + (r ^ SWZ*(c%2)). Without the transposed images, a transposing read
+  // c*32 + (r ^ SWZ*(c%2)). A transposing read
   // of 16 lanes covers rows r..r+3 of two adjacent chunk columns, 512 bytes
   // apart (the same LDS banks); swapping the 4-row halves of every odd column
   // puts them on disjoint banks. A 32-row column read stays one contiguous
   // 512-byte block.
-  static constexpr int SWZ = HAS_T ? 0 : 4;
+  static constexpr int SWZ = 4;
   static constexpr int STAT = NIMG * CH;     // lse2[32] then delta[32]: 256 bytes
   static constexpr int STAT_CH = 256 / CHB;
   static constexpr int CHUNKS = NIMG * CH + STAT_CH;
   static constexpr int64_t BYTES = (int64_t)CHUNKS * CHB;
 };
 
-// Key-side images: row-major k and v (with the query images' odd-column
-// swizzle) and, for fp32 only, the transposed k; the 16-bit dq kernels read
-// k^T out of the row-major image.
-// Factor from the dK^T accumulators to dk: against the prescaled q image
-// (q * scale * log2(e)) it is ln(2), against the unscaled transposed image
-// the softmax scale.
-template <typename T, int D>
-__device__ __forceinline__ float dk_scale(const goda_prefill_args& a) {
-  return QImg<T, D>::HAS_T ? a.softmax_scale : kLn2;
-}
-
+// Key-side images: row-major k and v, with the query images' odd-column
+// swizzle.
 template <typename T, int D>
 struct KVImg {
   static constexpr int CHB = (int)sizeof(typename Vec<T>::v8);
   static constexpr int CH = D / 8 * kBKV;
-  static constexpr bool HAS_T = sizeof(T) == 4;
-  static constexpr int NIMG = HAS_T ? 3 : 2;
-  static constexpr int SWZ = HAS_T ? 0 : 4;
-  static constexpr int KA = 0, VA = CH, KT = 2 * CH;
+  static constexpr int NIMG = 2;
+  static constexpr int SWZ = 4;
+  static constexpr int KA = 0, VA = CH;
   static constexpr int CHUNKS = NIMG * CH;
   static constexpr int64_t BYTES = (int64_t)CHUNKS * CHB;
 };
@@ -146,15 +128,6 @@ __device__ __forceinline__ int64_t kv_tile_index(int b, int j, int hk, int ntk, 
   return ((int64_t)b * ntk + j) * heads_kv + hk;
 }
 
-// Stored dS tiles: key tiles held before query tile qt of a sequence. With
-// `tri`, query tile q holds min(ntk, q + c + 1) key tiles (a causal sequence
-// whose keys run c tiles past its queries), else ntk.
-__host__ __device__ __forceinline__ int64_t ds_row_off(int qt, int ntk, int c, bool tri) {
-  if (!tri) return (int64_t)qt * ntk;
-  const int m = ntk - c > 0 ? ntk - c : 0;  // tiles below m are not yet full
-  const int q1 = qt < m ? qt : m;
-  return (int64_t)q1 * (q1 - 1) / 2 + (int64_t)q1 * (c + 1) + (int64_t)(qt - q1) * ntk;
-}
 // Byte offset of dS tile (sequence b, query tile qt, key tile kt, query head
 // hq). A stored tile (32 query rows x 32 keys, 2 KB) holds the B operands of
 // the dq product over its keys: 16 bytes per (k-step s, lane half h, row) at
@@ -264,8 +237,7 @@ __global__ void __launch_bounds__(256) pack_q_bwd_kernel(const BwdParams p) {
   if (i0 >= g.lq) return;
   const bool varlen = a.cu_seqlens_q != nullptr;
   const int diag = g.lk - g.lq;
-  __shared__ __align__(16) T qrows[kQRows][D + 8];   // q for the transposed image (dK; fp32 only)
-  __shared__ __align__(16) T qsrows[kQRows][D + 8];  // q * scale * log2(e) for the row-major one (S)
+  __shared__ __align__(16) T qsrows[kQRows][D + 8];  // q * scale * log2(e)
   __shared__ __align__(16) T grows[kQRows][D + 8];
   const int tid = threadIdx.x;
   constexpr int HALF8 = D / 16;
@@ -288,10 +260,6 @@ __global__ void __launch_bounds__(256) pack_q_bwd_kernel(const BwdParams p) {
     v8 qs1, qs2;
     norm_rope_row<T, D, HALF8>(q1, q2, c, a.q_norm_weight, a.norm_eps, i < g.lq && a.rope_q,
                                i < g.lq ? rope_qpos(a, diag, i) : 0, a, p.scale_log2, &qs1, &qs2);
-    if constexpr (QI::HAS_T) {
-      st_vec<v8>(&qrows[r][c], q1);
-      st_vec<v8>(&qrows[r][c + D / 2], q2);
-    }
     st_vec<v8>(&qsrows[r][c], qs1);
     st_vec<v8>(&qsrows[r][c + D / 2], qs2);
     st_vec<v8>(&grows[r][c], g1);
@@ -307,22 +275,6 @@ __global__ void __launch_bounds__(256) pack_q_bwd_kernel(const BwdParams p) {
     const int at = c * kQRows + (r ^ (QI::SWZ * (c & 1)));
     img[QI::QA + at] = ld_vec<v8>(&qsrows[r][8 * c]);
     img[QI::GA + at] = ld_vec<v8>(&grows[r][8 * c]);
-  }
-  // transposed images: chunk (kc, d) at kc*D + d holds rows
-  // 16*(kc/2) + kPermKey(8*(kc%2) + e)
-  if constexpr (QI::HAS_T)
-  for (int idx = tid; idx < QI::CH; idx += 256) {
-    const int kc = idx / D, d = idx % D;
-    const int r0 = 16 * (kc / 2);
-    v8 tq, tg;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int r = r0 + kPermKey(8 * (kc % 2) + e);
-      tq[e] = qrows[r][d];
-      tg[e] = grows[r][d];
-    }
-    img[QI::QT + idx] = tq;
-    img[QI::GT + idx] = tg;
   }
   // row statistics: 8 threads per row
   {
@@ -401,15 +353,6 @@ __global__ void __launch_bounds__(256) pack_kv_bwd_kernel(const BwdParams p) {
     const int at = c * kBKV + (r ^ (KI::SWZ * (c & 1)));
     img[KI::KA + at] = ld_vec<v8>(&krows[r][8 * c]);
     img[KI::VA + at] = ld_vec<v8>(&vrows[r][8 * c]);
-  }
-  if constexpr (KI::HAS_T)
-  for (int idx = tid; idx < KI::CH; idx += 256) {
-    const int kc = idx / D, d = idx % D;
-    const int r0 = 16 * (kc / 2);
-    v8 t;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) t[e] = krows[r0 + kPermKey(8 * (kc % 2) + e)][d];
-    img[KI::KT + idx] = t;
   }
 }
 
@@ -539,7 +482,7 @@ __global__ void __launch_bounds__(kWavesKv * 64, 1) bwd_dkv_mfma_kernel(const Bw
   typedef KVImg<T, D> KI;
   constexpr int KS = D / 16;  // k-steps over head_dim
   constexpr int MD = D / 32;  // 32-wide head_dim tiles of dK^T / dV^T
-  static_assert(!QI::HAS_T && sizeof(T) == 2, "B's operands come from transposing reads of 16-bit images");
+  static_assert(sizeof(T) == 2, "B's operands come from transposing reads of 16-bit images");
   constexpr int LOADS = QI::NIMG * QI::CH / (kWavesKv * 64);
   static_assert(QI::NIMG * QI::CH % (kWavesKv * 64) == 0, "tile must split over the waves");
   extern __shared__ __align__(16) unsigned char smem[];
@@ -793,7 +736,7 @@ __global__ void __launch_bounds__(kWavesKv * 64, 1) bwd_dkv_mfma_kernel(const Bw
   // which holds q * scale * log2(e): dk = scale * (dS^T q) = ln(2) * dK^T.
 #pragma unroll
   for (int md = 0; md < MD / 2; ++md) {
-    f32x16 x1 = dk[md] * dk_scale<T, D>(a), x2 = dk[md + MD / 2] * dk_scale<T, D>(a);
+    f32x16 x1 = dk[md] * kLn2, x2 = dk[md + MD / 2] * kLn2;
     if (rot) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
@@ -822,8 +765,6 @@ __global__ void __launch_bounds__(kWavesKv * 64, 1) bwd_dkv_mfma_kernel(const Bw
 // (key block, hk * nsplit + split) walks its share of the (query head, query
 // tile) pairs; with nsplit > 1 it writes fp32 partials.
 constexpr int kWavesWide = 4;
-constexpr int kWideParts = 4;
-
 
 template <typename T, int D, bool ALIBI, bool MASK, bool DS>
 __global__ void __launch_bounds__(kWavesWide * 64, 1) bwd_dkv_wide_kernel(const BwdParams p) {
@@ -839,8 +780,7 @@ __global__ void __launch_bounds__(kWavesWide * 64, 1) bwd_dkv_wide_kernel(const 
   constexpr int MD = D / 32;
   constexpr int NTH = kWavesWide * 64;
   constexpr int LOADS = QI::NIMG * QI::CH / NTH;
-  constexpr int PART = LOADS / kWideParts;
-  static_assert(QI::NIMG * QI::CH % (NTH * kWideParts) == 0, "tile must split over the threads and parts");
+  static_assert(QI::NIMG * QI::CH % NTH == 0, "tile must split over the threads");
   extern __shared__ __align__(16) unsigned char smem[];
 
   const goda_prefill_args& a = p.a;
@@ -894,43 +834,27 @@ __global__ void __launch_bounds__(kWavesWide * 64, 1) bwd_dkv_wide_kernel(const 
   const int it0 = (int)((int64_t)n * split / p.nsplit);
   const int it1 = (int)((int64_t)n * (split + 1) / p.nsplit);
 
-  v8 stg[PART];
-  v8 stg_stat;
   auto src_of = [&](const QWalk& w) {
     const int64_t t = q_tile_index(b, qt_lo + w.q, hk * p.group + w.h, p.ntq, a.heads_q);
     return reinterpret_cast<const v8*>(p.qimg + t * QI::BYTES);
   };
-  auto load_part = [&](const v8* src, int part) {
-#pragma unroll
-    for (int i = 0; i < PART; ++i) stg[i] = src[tid + (part * PART + i) * NTH];
-    if (part == 0 && tid < QI::STAT_CH) stg_stat = src[QI::STAT + tid];
-  };
-  auto store_part = [&](int it, int part) {
-    v8* dst = reinterpret_cast<v8*>(smem + (it % 2) * QI::BYTES);
-#pragma unroll
-    for (int i = 0; i < PART; ++i) dst[tid + (part * PART + i) * NTH] = stg[i];
-    if (part == 0 && tid < QI::STAT_CH) dst[QI::STAT + tid] = stg_stat;
-  };
 
-  // 16-bit tiles move by direct global->LDS loads instead (dma_blocks): wave w
+  // Tiles move by direct global->LDS loads (dma_blocks): wave w
   // copies chunks [w LOADS 64, (w + 1) LOADS 64) of the image to the same
   // offsets of the stage, and wave 0's lanes below STAT_CH the statistics.
   // Tile it + 1 lands in stage (it + 1) % 2 during interval it (the barrier
   // opening the interval ends every read of tile it - 1 there), its blocks
   // issued between the score products; the barrier closing the interval
-  // waits for the copies (vmcnt(0)). fp32 images
-  // (32-byte chunks) are staged through registers, in parts between the
-  // product phases.
-  constexpr bool DMA = sizeof(T) == 2;
+  // waits for the copies (vmcnt(0)).
   static_assert(QI::STAT_CH <= 64, "statistics fit one wave's copy");
-  static_assert(!DMA || 2 * LOADS + 1 < 2 * KS, "every copy block issues between score products");
+  static_assert(2 * LOADS + 1 < 2 * KS, "every copy block issues between score products");
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   const unsigned lane_off = (unsigned)((wave_u * LOADS * 64 + lane) * 16);
   const unsigned stat_off = (unsigned)((QI::STAT + lane) * 16);
   auto tile_dma = [&](const QWalk& w, int it) {
     const unsigned long long base = (unsigned long long)(uintptr_t)src_of(w);
     const unsigned lds = (unsigned)(uintptr_t)(smem + (it % 2) * QI::BYTES);
-    dma_span<DMA ? LOADS : 1>(lds + (unsigned)(wave_u * LOADS * 64 * 16), lane_off, base);
+    dma_span<LOADS>(lds + (unsigned)(wave_u * LOADS * 64 * 16), lane_off, base);
     if (wave_u == 0 && lane < QI::STAT_CH) dma_blocks<1>(lds + QI::STAT * 16, stat_off, base);
   };
 
@@ -940,31 +864,18 @@ __global__ void __launch_bounds__(kWavesWide * 64, 1) bwd_dkv_wide_kernel(const 
   // for every access of the wave) does not wait on fresh stores; the last
   // tile's after the loop. A tile with no slot (no key visible to its rows)
   // goes to a sink nobody reads.
-  constexpr bool kStoreDs = DS && sizeof(T) == 2;
+  constexpr bool kStoreDs = DS;
   static_assert(!kStoreDs || 2 * KS >= 32, "a store after every other score product");
   v8 dsp0{}, dsp1{};
   unsigned char* dsp_tile = kStoreDs ? p.ds + p.ds_sink : nullptr;
   const int ds_lane = (2 * (l32 >> 4) + ((l32 >> 2) & 1)) * 512 + 2 * ((l32 & 3) + 4 * ((l32 >> 3) & 1)) + 64 * hi;
   QWalk cu(it0, nq), nw(it0, nq);
-  if constexpr (DMA) {
-    if (it0 < it1) tile_dma(cu, it0);
-    dma_ring_barrier<0>();
-  } else {
-    if (it0 < it1) {
-      const v8* src = src_of(cu);
-#pragma unroll
-      for (int part = 0; part < kWideParts; ++part) {
-        load_part(src, part);
-        store_part(it0, part);
-      }
-    }
-    ring_barrier();
-  }
+  if (it0 < it1) tile_dma(cu, it0);
+  dma_ring_barrier<0>();
   for (int it = it0; it < it1; ++it) {
     // The next tile is staged into the other stage (on the last tile: this
     // tile again, into a stage nobody reads), so the loop body is branch-free.
     if (it + 1 < it1) nw.next();
-    const v8* nsrc = src_of(nw);
     const int hq = hk * p.group + cu.h;
     const int qt = qt_lo + cu.q;
     const int q0 = qt * kQRows;
@@ -972,19 +883,7 @@ __global__ void __launch_bounds__(kWavesWide * 64, 1) bwd_dkv_wide_kernel(const 
     const float slope2 = ALIBI ? a.alibi_slopes[hq] * kLog2e : 0.f;
     const v8* st = reinterpret_cast<const v8*>(smem + (it % 2) * QI::BYTES);
     const float* stat = reinterpret_cast<const float*>(st + QI::STAT);
-    auto store_next = [&](int part) {
-      if constexpr (!DMA) {
-        v8* dst = reinterpret_cast<v8*>(smem + ((it + 1) % 2) * QI::BYTES);
-#pragma unroll
-        for (int i = 0; i < PART; ++i) dst[tid + (part * PART + i) * NTH] = stg[i];
-        if (part == 0 && tid < QI::STAT_CH) dst[QI::STAT + tid] = stg_stat;
-      }
-    };
-    auto next_part = [&](int part) {
-      if constexpr (!DMA) load_part(nsrc, part);
-    };
 
-    next_part(0);
     // The caller's mask bits of this key for the tile's 32 rows.
     uint32_t mword = 0;
     if (MASK && key < g.lk)
@@ -1006,24 +905,16 @@ __global__ void __launch_bounds__(kWavesWide * 64, 1) bwd_dkv_wide_kernel(const 
       }
     }
     // One wave per SIMD: nothing else hides a product's LDS operand latency,
-    // so the reads run WL products ahead. 16-bit: S and dP stay in VGPRs
+    // so the reads run WL products ahead. S and dP stay in VGPRs
     // (mfma32_vgpr), where the VALU fills and reads them.
-    constexpr bool SV = sizeof(T) == 2;
-    if constexpr (SV) mfma_vgpr_fill(s, dp);
+    mfma_vgpr_fill(s, dp);
     prefetched_products<2 * KS, WL, v8>(
         [&](int j) { return st[((j & 1) ? QI::GA : QI::QA) + (2 * (j >> 1) + hi) * kQRows + (l32 ^ (QI::SWZ * hi))]; },
         [&](int j, const v8& o) {
-          if constexpr (SV) {
-            if (j & 1)
-              mfma32_vgpr(o, vf[j >> 1], dp);
-            else
-              mfma32_vgpr(o, kf[j >> 1], s);
-          } else {
-            if (j & 1)
-              dp = mfma32(o, vf[j >> 1], dp);
-            else
-              s = mfma32(o, kf[j >> 1], s);
-          }
+          if (j & 1)
+            mfma32_vgpr(o, vf[j >> 1], dp);
+          else
+            mfma32_vgpr(o, kf[j >> 1], s);
         },
         [&](int j) {
           // The next tile's copies, one block after every other product, so
@@ -1033,17 +924,15 @@ __global__ void __launch_bounds__(kWavesWide * 64, 1) bwd_dkv_wide_kernel(const 
           // clocks a step; cfg3-shape backward kernels -9% in a same-box
           // A/B). On the last tile nw is this tile again: its copy lands in
           // the stage nobody reads, and the loop stays branch-free.
-          if constexpr (DMA) {
-            if ((j & 1) && (j >> 1) < LOADS) {
-              const int k = j >> 1;
-              const unsigned lds = (unsigned)(uintptr_t)(smem + ((it + 1) % 2) * QI::BYTES);
-              dma_blocks<1>(lds + (unsigned)((wave_u * LOADS + k) * 1024), lane_off,
-                            (unsigned long long)(uintptr_t)src_of(nw) + k * 1024);
-            }
-            if (j == 2 * LOADS + 1 && wave_u == 0 && lane < QI::STAT_CH)
-              dma_blocks<1>((unsigned)(uintptr_t)(smem + ((it + 1) % 2) * QI::BYTES) + QI::STAT * 16, stat_off,
-                            (unsigned long long)(uintptr_t)src_of(nw));
+          if ((j & 1) && (j >> 1) < LOADS) {
+            const int k = j >> 1;
+            const unsigned lds = (unsigned)(uintptr_t)(smem + ((it + 1) % 2) * QI::BYTES);
+            dma_blocks<1>(lds + (unsigned)((wave_u * LOADS + k) * 1024), lane_off,
+                          (unsigned long long)(uintptr_t)src_of(nw) + k * 1024);
           }
+          if (j == 2 * LOADS + 1 && wave_u == 0 && lane < QI::STAT_CH)
+            dma_blocks<1>((unsigned)(uintptr_t)(smem + ((it + 1) % 2) * QI::BYTES) + QI::STAT * 16, stat_off,
+                          (unsigned long long)(uintptr_t)src_of(nw));
           if constexpr (kStoreDs) {
             if (!(j & 1)) {
               const int r = j >> 1;
@@ -1051,9 +940,7 @@ __global__ void __launch_bounds__(kWavesWide * 64, 1) bwd_dkv_wide_kernel(const 
             }
           }
         });
-    if constexpr (SV) mfma_vgpr_drain(s, dp);
-    store_next(0);
-    next_part(1);
+    mfma_vgpr_drain(s, dp);
 
     // P and dS; visibility as a range of the register's row offset.
     int lo_lim = -1, hi_lim = g.lq - 1 - rel;
@@ -1078,8 +965,6 @@ __global__ void __launch_bounds__(kWavesWide * 64, 1) bwd_dkv_wide_kernel(const 
         ds[r] = keep_if_bit(ds[r], vis, off, 0.f);
       }
     }
-    store_next(1);
-    next_part(2);
     const v8 pp0 = pack8<v8, T>(pr), pp1 = pack8<v8, T>(pr + 8);
     const v8 d0 = pack8<v8, T>(ds), d1 = pack8<v8, T>(ds + 8);
     // this tile's dS and its slot (every tile a causal query tile can see;
@@ -1092,27 +977,15 @@ __global__ void __launch_bounds__(kWavesWide * 64, 1) bwd_dkv_wide_kernel(const 
     }
     prefetched_products<2 * MD, WL, v8>(
         [&](int j) {
-          if constexpr (QI::HAS_T)
-            return st[QI::GT + (2 * (j & 1) + hi) * D + 32 * (j >> 1) + l32];
-          else
-            return tr_operand<v8>(reinterpret_cast<const unsigned char*>(st + QI::GA), lane, j & 1, j >> 1);
+          return tr_operand<v8>(reinterpret_cast<const unsigned char*>(st + QI::GA), lane, j & 1, j >> 1);
         },
         [&](int j, const v8& o) { dv[j >> 1] = mfma32(o, (j & 1) ? pp1 : pp0, dv[j >> 1]); });
-    store_next(2);
-    next_part(3);
     prefetched_products<2 * MD, WL, v8>(
         [&](int j) {
-          if constexpr (QI::HAS_T)
-            return st[QI::QT + (2 * (j & 1) + hi) * D + 32 * (j >> 1) + l32];
-          else
-            return tr_operand<v8>(reinterpret_cast<const unsigned char*>(st + QI::QA), lane, j & 1, j >> 1);
+          return tr_operand<v8>(reinterpret_cast<const unsigned char*>(st + QI::QA), lane, j & 1, j >> 1);
         },
         [&](int j, const v8& o) { dk[j >> 1] = mfma32(o, (j & 1) ? d1 : d0, dk[j >> 1]); });
-    store_next(3);
-    if constexpr (DMA)
-      dma_ring_barrier<0>();
-    else
-      ring_barrier();
+    dma_ring_barrier<0>();
   }
 
   if constexpr (kStoreDs) {
@@ -1154,7 +1027,7 @@ __global__ void __launch_bounds__(kWavesWide * 64, 1) bwd_dkv_wide_kernel(const 
   const int pos = a.rope_k_offset + key;
   // dk: one pair of head-dim blocks (md, md + MD/2: the rotation's partners)
   // at a time, scaled and rotated back.
-  const float dks = dk_scale<T, D>(a);
+  const float dks = kLn2;
 #pragma unroll
   for (int md = 0; md < MD / 2; ++md) {
     f32x16 x1 = dk[md] * dks, x2 = dk[md + MD / 2] * dks;
@@ -1201,8 +1074,8 @@ __global__ void __launch_bounds__(256) bwd_dkv_reduce_kernel(const BwdParams p) 
     v1 += ld_vec<f32x4>(pv + d0);
     v2 += ld_vec<f32x4>(pv + d0 + D / 2);
   }
-  k1 *= dk_scale<T, D>(a);
-  k2 *= dk_scale<T, D>(a);
+  k1 *= kLn2;
+  k2 *= kLn2;
   if (a.rope_k && key < g.lk) {
     const int pos = a.rope_k_offset + key;
     const f32x4 cs = ld_vec<f32x4>(a.rope_cos + (int64_t)pos * (D / 2) + d0);
@@ -1226,8 +1099,8 @@ __global__ void __launch_bounds__(256) bwd_dkv_reduce_kernel(const BwdParams p) 
 // 4. dq
 // ---------------------------------------------------------------------------
 template <typename T, int D, bool ALIBI, bool MASK>
-__global__ void __launch_bounds__((DqShape<T, D>::WAVES * 64), (DqShape<T, D>::OCC)) bwd_dq_mfma_kernel(const BwdParams p) {
-  constexpr int kWavesDq = DqShape<T, D>::WAVES;
+__global__ void __launch_bounds__((DqShape<D>::WAVES * 64), (DqShape<D>::OCC)) bwd_dq_mfma_kernel(const BwdParams p) {
+  constexpr int kWavesDq = DqShape<D>::WAVES;
   typedef typename Vec<T>::v8 v8;
   typedef typename Vec<T>::v4 v4;
   typedef QImg<T, D> QI;
@@ -1239,7 +1112,7 @@ __global__ void __launch_bounds__((DqShape<T, D>::WAVES * 64), (DqShape<T, D>::O
   // Operand reads in flight per product phase with one wave per SIMD (cfg3
   // shape: 2.51 -> 1.99 ms); two waves per SIMD hide each other's latency and
   // keep the scheduler's order (fenced prefetch there: +1-2%).
-  constexpr int QL = DqShape<T, D>::WIDE ? 4 : 0;
+  constexpr int QL = DqShape<D>::WIDE ? 4 : 0;
   constexpr int LOADS = (KI::CHUNKS + kWavesDq * 64 - 1) / (kWavesDq * 64);
   extern __shared__ __align__(16) unsigned char smem[];
 
@@ -1314,22 +1187,21 @@ __global__ void __launch_bounds__((DqShape<T, D>::WAVES * 64), (DqShape<T, D>::O
 #pragma unroll
   for (int md = 0; md < MD; ++md) dq[md] = f32x16{};
 
-  // 16-bit tiles move by direct global->LDS loads (dma_span): wave w copies
+  // Tiles move by direct global->LDS loads (dma_span): wave w copies
   // chunks [w LOADS 64, (w + 1) LOADS 64) of the image to the same offsets
-  // of the stage. fp32 images (32-byte chunks) are staged through registers.
-  constexpr bool DMA = sizeof(T) == 2;
-  static_assert(!DMA || KI::CHUNKS % (kWavesDq * 64) == 0, "16-bit tile splits over the waves");
+  // of the stage.
+  static_assert(KI::CHUNKS % (kWavesDq * 64) == 0, "tile splits over the waves");
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   const unsigned lane_off = (unsigned)((wave_u * LOADS * 64 + lane) * 16);
   auto tile_dma = [&](int it) {
     const unsigned long long base =
         (unsigned long long)(uintptr_t)(p.kvimg + kv_tile_index(b, j_lo + it, hk, p.ntk, a.heads_kv) * KI::BYTES);
     const unsigned lds = (unsigned)(uintptr_t)(smem + (it % 2) * KI::BYTES) + (unsigned)(wave_u * LOADS * 64 * 16);
-    dma_span<DMA ? LOADS : 1>(lds, lane_off, base);
+    dma_span<LOADS>(lds, lane_off, base);
   };
   // Block k of this wave's share of tile `it` (the one-wave kernel spreads a
   // tile's copies over the score products; cfg3-shape backward -3..-9%).
-  constexpr bool kSpreadCopies = DMA && DqShape<T, D>::WIDE;
+  constexpr bool kSpreadCopies = DqShape<D>::WIDE;
   static_assert(!kSpreadCopies || 2 * LOADS <= 2 * KS, "every copy block issues between score products");
   auto tile_dma_block = [&](int it, int k) {
     const unsigned long long base =
@@ -1337,20 +1209,6 @@ __global__ void __launch_bounds__((DqShape<T, D>::WAVES * 64), (DqShape<T, D>::O
     const unsigned lds = (unsigned)(uintptr_t)(smem + (it % 2) * KI::BYTES) + (unsigned)((wave_u * LOADS + k) * 1024);
     dma_blocks<1>(lds, lane_off, base + k * 1024);
   };
-  v8 stg[DMA ? 1 : LOADS];
-  auto tile_load = [&](int it) {
-    const v8* src = reinterpret_cast<const v8*>(p.kvimg + kv_tile_index(b, j_lo + it, hk, p.ntk, a.heads_kv) * KI::BYTES);
-#pragma unroll
-    for (int x = 0; x < LOADS; ++x)
-      if (KI::CHUNKS % (kWavesDq * 64) == 0 || tid + x * kWavesDq * 64 < KI::CHUNKS) stg[x] = src[tid + x * kWavesDq * 64];
-  };
-  auto tile_store = [&](int it) {
-    v8* dst = reinterpret_cast<v8*>(smem + (it % 2) * KI::BYTES);
-#pragma unroll
-    for (int x = 0; x < LOADS; ++x)
-      if (KI::CHUNKS % (kWavesDq * 64) == 0 || tid + x * kWavesDq * 64 < KI::CHUNKS) dst[tid + x * kWavesDq * 64] = stg[x];
-  };
-
   static_assert(kBKV == 32, "one mask word per key tile");
   auto compute = [&](int it) {
     const int kvb = (j_lo + it) * kBKV;
@@ -1371,24 +1229,16 @@ __global__ void __launch_bounds__((DqShape<T, D>::WAVES * 64), (DqShape<T, D>::O
         dp[mt][r] = -dl;
       }
     if constexpr (QL > 0) {
-      // One wave per SIMD (head_dim 256, 16-bit): S and dP stay in VGPRs
+      // One wave per SIMD (head_dim 256): S and dP stay in VGPRs
       // (mfma32_vgpr), where the VALU fills and reads them.
-      constexpr bool SV = sizeof(T) == 2 && DqShape<T, D>::WIDE;
-      if constexpr (SV) mfma_vgpr_fill(s[0], dp[0]);
+      mfma_vgpr_fill(s[0], dp[0]);
       prefetched_products<2 * KS, QL, v8>(
           [&](int j) { return st[((j & 1) ? KI::VA : KI::KA) + (2 * (j >> 1) + hi) * kBKV + (l32 ^ (KI::SWZ * hi))]; },
           [&](int j, const v8& o) {
-            if constexpr (SV) {
-              if (j & 1)
-                mfma32_vgpr(o, gf[j >> 1], dp[0]);
-              else
-                mfma32_vgpr(o, qf[j >> 1], s[0]);
-            } else {
-              if (j & 1)
-                dp[0] = mfma32(o, gf[j >> 1], dp[0]);
-              else
-                s[0] = mfma32(o, qf[j >> 1], s[0]);
-            }
+            if (j & 1)
+              mfma32_vgpr(o, gf[j >> 1], dp[0]);
+            else
+              mfma32_vgpr(o, qf[j >> 1], s[0]);
           },
           [&](int j) {
             // One wave per SIMD: the next tile's copies go out one block
@@ -1397,7 +1247,7 @@ __global__ void __launch_bounds__((DqShape<T, D>::WAVES * 64), (DqShape<T, D>::O
             if constexpr (kSpreadCopies)
               if ((j & 1) && (j >> 1) < LOADS) tile_dma_block(min(it + 1, n - 1), j >> 1);
           });
-      if constexpr (SV) mfma_vgpr_drain(s[0], dp[0]);
+      mfma_vgpr_drain(s[0], dp[0]);
     } else {
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks)
@@ -1433,10 +1283,7 @@ __global__ void __launch_bounds__((DqShape<T, D>::WAVES * 64), (DqShape<T, D>::O
     if constexpr (QL > 0) {
       prefetched_products<KS2 * MD, QL, v8>(
           [&](int j) {
-            if constexpr (KI::HAS_T)
-              return st[KI::KT + (2 * (j / MD) + hi) * D + 32 * (j % MD) + l32];
-            else
-              return tr_operand<v8>(reinterpret_cast<const unsigned char*>(st + KI::KA), lane, j / MD, j % MD);
+            return tr_operand<v8>(reinterpret_cast<const unsigned char*>(st + KI::KA), lane, j / MD, j % MD);
           },
           [&](int j, const v8& o) { dq[j % MD] = mfma32(o, dsf[j / MD], dq[j % MD]); });
     } else {
@@ -1444,38 +1291,21 @@ __global__ void __launch_bounds__((DqShape<T, D>::WAVES * 64), (DqShape<T, D>::O
       for (int ks2 = 0; ks2 < KS2; ++ks2)
 #pragma unroll
         for (int md = 0; md < MD; ++md)
-          dq[md] = mfma32(KI::HAS_T ? st[KI::KT + (2 * ks2 + hi) * D + 32 * md + l32]
-                                    : tr_operand<v8>(reinterpret_cast<const unsigned char*>(st + KI::KA), lane, ks2, md),
-                          dsf[ks2], dq[md]);
+          dq[md] = mfma32(tr_operand<v8>(reinterpret_cast<const unsigned char*>(st + KI::KA), lane, ks2, md), dsf[ks2], dq[md]);
       lead_schedule<T, KS2 * MD, 4>();
     }
   };
 
-  if constexpr (DMA) {
-    // Tile it + 1 lands in stage (it + 1) % 2 during interval it: the
-    // barrier opening the interval ends every read of tile it - 1 there, and
-    // the one opening interval it + 1 waits for the copies (vmcnt(0)).
-    if (n > 0) tile_dma(0);
-    load_qg();
-    for (int it = 0; it < n; ++it) {
-      dma_ring_barrier<0>();
-      if constexpr (!kSpreadCopies)
-        if (it + 1 < n) tile_dma(it + 1);
-      compute(it);
-    }
-  } else {
-    load_qg();
-    if (n > 0) {
-      tile_load(0);
-      tile_store(0);
-    }
-    ring_barrier();
-    for (int it = 0; it < n; ++it) {
-      if (it + 1 < n) tile_load(it + 1);
-      compute(it);
-      if (it + 1 < n) tile_store(it + 1);
-      ring_barrier();
-    }
+  // Tile it + 1 lands in stage (it + 1) % 2 during interval it: the
+  // barrier opening the interval ends every read of tile it - 1 there, and
+  // the one opening interval it + 1 waits for the copies (vmcnt(0)).
+  if (n > 0) tile_dma(0);
+  load_qg();
+  for (int it = 0; it < n; ++it) {
+    dma_ring_barrier<0>();
+    if constexpr (!kSpreadCopies)
+      if (it + 1 < n) tile_dma(it + 1);
+    compute(it);
   }
 
   // ---- epilogue: lane l32 owns query row i; register (md, r) is head-dim
@@ -1523,7 +1353,7 @@ constexpr int kWavesDqS = 4;
 // none), and the largest dS store they may use (beyond it dq recomputes S and
 // dP).
 template <typename T, int D>
-constexpr int kDsHeadsPerWave = (sizeof(T) == 2 && D == 256) ? 2 : 0;
+constexpr int kDsHeadsPerWave = D == 256 ? 2 : 0;
 constexpr int64_t kDsMaxBytes = 8ll << 30;
 template <typename T, int D, int HW>
 struct DqSShape {
@@ -1701,7 +1531,7 @@ hipError_t launch_main(const BwdParams& p, hipStream_t s) {
   hipError_t e;
   if ((e = record_timing(p.g.timing_begin, s)) != hipSuccess) return e;
   if (a.seqlen_k > 0) {
-    if constexpr (DqShape<T, D>::WIDE) {
+    if constexpr (DqShape<D>::WIDE) {
       auto kern = bwd_dkv_wide_kernel<T, D, ALIBI, MASK, false>;
       if constexpr (kDsHeadsPerWave<T, D> > 0)
         if (p.ds) kern = bwd_dkv_wide_kernel<T, D, ALIBI, MASK, true>;
@@ -1751,7 +1581,7 @@ hipError_t launch_main(const BwdParams& p, hipStream_t s) {
     const size_t lds = 2 * (size_t)KVImg<T, D>::BYTES;
     if ((e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)) != hipSuccess)
       return e;
-    constexpr int kWavesDq = DqShape<T, D>::WAVES;
+    constexpr int kWavesDq = DqShape<D>::WAVES;
     const int qb_rows = (kWavesDq / p.heads_per_wg) * 32;
     const int nqt = (a.seqlen_q + qb_rows - 1) / qb_rows;
     const int64_t nblk = (int64_t)nqt * a.batch * a.heads_kv * (p.group / p.heads_per_wg);
@@ -1767,7 +1597,7 @@ hipError_t launch_main(const BwdParams& p, hipStream_t s) {
 // causal key blocks differ in work by up to the sequence length), at most 8
 // and at most the (query head, query tile) pairs a key block can see.
 int dkv_splits(const goda_prefill_args& a) {
-  if ((a.head_dim < 256 && a.dtype != GODA_DTYPE_F32) || a.heads_kv <= 0) return 1;
+  if (a.head_dim < 256 || a.heads_kv <= 0) return 1;
   const int64_t wgs = (int64_t)((a.seqlen_k + 32 * kWavesWide - 1) / (32 * kWavesWide)) * a.heads_kv * a.batch;
   if (wgs <= 0) return 1;
   int64_t ns = (1024 + wgs - 1) / wgs;
@@ -1776,13 +1606,6 @@ int dkv_splits(const goda_prefill_args& a) {
   return (int)std::min<int64_t>(ns, 8);
 }
 
-// Key-major mask words: (batches, heads) of the mask (1 where it broadcasts)
-// x keys x query tiles.
-int64_t mask_t_words(const goda_prefill_args& a) {
-  if (!a.mask_bits) return 0;
-  const int64_t bm = a.mask_stride_b ? a.batch : 1, hm = a.mask_stride_h ? a.heads_q : 1;
-  return bm * hm * a.seqlen_k * ((a.seqlen_q + kQRows - 1) / kQRows);
-}
 int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
 
 // Workspace: query-tile images, key-tile images, the dk/dv partials, the
@@ -1805,7 +1628,7 @@ BwdLayout bwd_layout(const goda_prefill_args& a) {
   l.ds = l.total = l.mask;
   if (a.mask_bits) {
     l.mask = align256(l.mask);
-    l.ds = l.total = l.mask + 4 * mask_t_words(a);
+    l.ds = l.total = l.mask + 4 * bwd_mask_t_words(a);
   }
   constexpr int HW = kDsHeadsPerWave<T, D>;
   const int group = a.heads_kv > 0 ? a.heads_q / a.heads_kv : 0;
@@ -1841,7 +1664,7 @@ hipError_t launch_d(BwdParams p, hipStream_t s) {
   const BwdLayout l = bwd_layout<T, D>(a);
   p.ntq = (a.seqlen_q + kQRows - 1) / kQRows;
   p.ntk = (a.seqlen_k + kBKV - 1) / kBKV;
-  p.heads_per_wg = gcd_int(p.group, DqShape<T, D>::WAVES);
+  p.heads_per_wg = gcd_int(p.group, DqShape<D>::WAVES);
   p.qimg = reinterpret_cast<unsigned char*>(p.g.workspace);
   p.kvimg = p.qimg + l.kvimg;
   p.nsplit = dkv_splits(a);
@@ -1857,15 +1680,7 @@ hipError_t launch_d(BwdParams p, hipStream_t s) {
   hipError_t e;
   if (a.mask_bits) {
     p.mask_t = reinterpret_cast<uint32_t*>(p.qimg + l.mask);
-    const int64_t hm = a.mask_stride_h ? a.heads_q : 1;
-    p.mt_stride_h = a.mask_stride_h ? (int64_t)a.seqlen_k * p.ntq : 0;
-    p.mt_stride_b = a.mask_stride_b ? hm * a.seqlen_k * p.ntq : 0;
-    const int64_t threads = (int64_t)p.ntq * ((a.seqlen_k + 31) / 32);
-    if (threads > 0) {
-      const dim3 grid((unsigned)((threads + 255) / 256), (unsigned)hm, a.mask_stride_b ? a.batch : 1);
-      bwd_mask_t_kernel<<<grid, 256, 0, s>>>(p);
-      if ((e = hipGetLastError()) != hipSuccess) return e;
-    }
+    if ((e = launch_bwd_mask_t(p, s)) != hipSuccess) return e;
   }
   if (p.ntq > 0) {
     pack_q_bwd_kernel<T, D><<<dim3(p.ntq, a.heads_q, a.batch), 256, 0, s>>>(p);
@@ -1884,22 +1699,31 @@ template <typename T>
 hipError_t launch_t(const BwdParams& p, hipStream_t s) {
   if (p.a.head_dim == 64) return launch_d<T, 64>(p, s);
   if (p.a.head_dim == 128) return launch_d<T, 128>(p, s);
-  if constexpr (sizeof(T) == 2) {
-    if (p.a.head_dim == 256) return launch_d<T, 256>(p, s);
-  }
+  if (p.a.head_dim == 256) return launch_d<T, 256>(p, s);
   return hipErrorNotSupported;
 }
 
 }  // namespace
 
-bool prefill_bwd_mfma_supported(const goda_prefill_args& a) {
-  if (a.dtype == GODA_DTYPE_F32) return a.head_dim == 64 || a.head_dim == 128;
-  if (a.dtype != GODA_DTYPE_BF16 && a.dtype != GODA_DTYPE_F16) return false;
-  return a.head_dim == 64 || a.head_dim == 128 || a.head_dim == 256;
+int64_t bwd_mask_t_words(const goda_prefill_args& a) {
+  if (!a.mask_bits) return 0;
+  const int64_t bm = a.mask_stride_b ? a.batch : 1, hm = a.mask_stride_h ? a.heads_q : 1;
+  return bm * hm * a.seqlen_k * ((a.seqlen_q + kQRows - 1) / kQRows);
+}
+
+hipError_t launch_bwd_mask_t(BwdParams& p, hipStream_t s) {
+  const goda_prefill_args& a = p.a;
+  const int64_t hm = a.mask_stride_h ? a.heads_q : 1;
+  p.mt_stride_h = a.mask_stride_h ? (int64_t)a.seqlen_k * p.ntq : 0;
+  p.mt_stride_b = a.mask_stride_b ? hm * a.seqlen_k * p.ntq : 0;
+  const int64_t threads = (int64_t)p.ntq * ((a.seqlen_k + 31) / 32);
+  if (threads <= 0) return hipSuccess;
+  const dim3 grid((unsigned)((threads + 255) / 256), (unsigned)hm, a.mask_stride_b ? a.batch : 1);
+  bwd_mask_t_kernel<<<grid, 256, 0, s>>>(p);
+  return hipGetLastError();
 }
 
 int64_t prefill_bwd_mfma_workspace_bytes(const goda_prefill_args& a) {
-  if (a.dtype == GODA_DTYPE_F32) return a.head_dim == 64 ? workspace_bytes_d<float, 64>(a) : workspace_bytes_d<float, 128>(a);
   if (a.head_dim == 64) return workspace_bytes_d<bf16, 64>(a);
   if (a.head_dim == 128) return workspace_bytes_d<bf16, 128>(a);
   return workspace_bytes_d<bf16, 256>(a);
@@ -1908,7 +1732,6 @@ int64_t prefill_bwd_mfma_workspace_bytes(const goda_prefill_args& a) {
 hipError_t launch_prefill_bwd_mfma(BwdParams p, hipStream_t s) {
   if (p.a.dtype == GODA_DTYPE_BF16) return launch_t<bf16>(p, s);
   if (p.a.dtype == GODA_DTYPE_F16) return launch_t<f16>(p, s);
-  if (p.a.dtype == GODA_DTYPE_F32) return launch_t<float>(p, s);
   return hipErrorNotSupported;
 }
 

@@ -43,20 +43,23 @@ __device__ __forceinline__ f32x4 img_chunk(const unsigned char* img, int c, unsi
   return *reinterpret_cast<const f32x4*>(img + c * 1024 + lane16);
 }
 
-// Writes the images of one staged 32-row tile from LDS, 256 threads.
-template <int D>
-__device__ __forceinline__ void write_row_image(float (*rows)[D + 4], unsigned char* img, int tid) {
+// Writes the images of one staged 32-row tile from LDS, 256 threads: chunk c
+// goes to chunk position c * STEP of img.
+template <int D, int STEP = 1>
+__device__ __forceinline__ void write_row_image(const float (*rows)[D + 4], unsigned char* img, int tid, float scale = 1.f) {
 #pragma unroll 4
-  for (int i = tid; i < D / 8 * 64; i += 256)  // chunk i / 64, lane i % 64: row i % 32, elements 4 (i / 32) ..
-    *reinterpret_cast<f32x4*>(img + i * 16) = ld_vec<f32x4>(&rows[i % kF32Rows][4 * (i / kF32Rows)]);
+  for (int i = tid; i < D / 8 * 64; i += 256) {
+    const int c = i / 64, l = i % 64;  // row l % 32, elements 8 c + 4 (l / 32) ..
+    *reinterpret_cast<f32x4*>(img + c * STEP * 1024 + l * 16) = ld_vec<f32x4>(&rows[l % 32][8 * c + 4 * (l / 32)]) * scale;
+  }
 }
-template <int D>
-__device__ __forceinline__ void write_tr_image(float (*rows)[D + 4], unsigned char* img, int tid) {
+template <int D, int STEP = 1>
+__device__ __forceinline__ void write_tr_image(const float (*rows)[D + 4], unsigned char* img, int tid) {
 #pragma unroll 4
   for (int i = tid; i < D / 8 * 64; i += 256) {
     const int c = i / 64, l = i % 64;
     const int k = 8 * (c / (D / 32)) + 4 * (l / 32), d = 32 * (c % (D / 32)) + l % 32;
-    *reinterpret_cast<f32x4*>(img + i * 16) = f32x4{rows[k][d], rows[k + 1][d], rows[k + 2][d], rows[k + 3][d]};
+    *reinterpret_cast<f32x4*>(img + c * STEP * 1024 + l * 16) = f32x4{rows[k][d], rows[k + 1][d], rows[k + 2][d], rows[k + 3][d]};
   }
 }
 

@@ -39,14 +39,13 @@ struct BwdParams {
   goda_prefill_grads g;
   int group;
   float scale_log2;
-  int64_t delta_rows;    // row stride of the delta buffer: batch * seqlen_q
-  float* delta;          // fp32 [heads_q, delta_rows]: rowsum(dO * O)
-  // MFMA path: operand images in the workspace (set by its launcher).
+  // Operand images in the workspace (set by the launcher).
   int ntq, ntk;          // 32-row query tiles / key tiles per sequence
   int heads_per_wg;      // query heads per dq workgroup
+  int key_split;         // fp32 dq: waves of a workgroup sharing an item's key tiles
   unsigned char* qimg;   // [batch][ntq][heads_q] query-tile images
   unsigned char* kvimg;  // [batch][ntk][heads_kv] key-tile images
-  // head_dim 256: the dk/dv walk over (query head, query tile) pairs is split
+  // head_dim 256 or fp32: the dk/dv walk over (query head, query tile) pairs is split
   // over nsplit workgroups per key block; with nsplit > 1 they write fp32
   // partials [nsplit][dk, dv][batch * seqlen_k][heads_kv][head_dim] here.
   int nsplit;
@@ -69,20 +68,32 @@ struct BwdParams {
   int ds_hpw;            // query heads per workgroup of the dq-from-dS kernel
 };
 
-// Backward: workspace bytes and the launch (generic VALU kernels for every
-// dtype; MFMA kernels for bf16/fp16 where an instance exists).
+// Stored dS tiles: key tiles held before query tile qt of a sequence. With
+// `tri`, query tile q holds min(ntk, q + c + 1) key tiles (a causal sequence
+// whose keys run c tiles past its queries), else ntk.
+__host__ __device__ __forceinline__ int64_t ds_row_off(int qt, int ntk, int c, bool tri) {
+  if (!tri) return (int64_t)qt * ntk;
+  const int m = ntk - c > 0 ? ntk - c : 0;  // tiles below m are not yet full
+  const int q1 = qt < m ? qt : m;
+  return (int64_t)q1 * (q1 - 1) / 2 + (int64_t)q1 * (c + 1) + (int64_t)(qt - q1) * ntk;
+}
+// Backward: workspace bytes and the launch.
 int64_t prefill_bwd_workspace_bytes(const goda_prefill_args& a);
 hipError_t launch_prefill_bwd(const BwdParams& p, hipStream_t s);
-bool prefill_bwd_mfma_supported(const goda_prefill_args& a);
-// Fused QK-RMSNorm backward (norm_bwd.hip): fp32 dw partials' bytes, the
-// normalized rows of q or k (contiguous [batch, seqlen, heads, head_dim],
-// packed rows at their packed index) for the generic kernels, and dx / dw
-// from the attention backward's dq / dk (gradients of the normalized rows).
+// Fused QK-RMSNorm backward (norm_bwd.hip): fp32 dw partials' bytes, and dx /
+// dw from the attention backward's dq / dk (gradients of the normalized rows).
 int64_t norm_bwd_part_bytes(const goda_prefill_args& a);
-hipError_t launch_norm_rows(const goda_prefill_args& a, bool q_side, void* dst, hipStream_t s);
 // dL/dw of the fused norms as zeros (an empty backward: no rows, no keys).
 hipError_t zero_norm_dw(const goda_prefill_args& a, const goda_prefill_grads& g, hipStream_t s);
 hipError_t launch_norm_bwd(const goda_prefill_args& a, const goda_prefill_grads& g, float* part, hipStream_t s);
+// Key-major mask words of the backward: (batches, heads) of the mask (1 where it
+// broadcasts) x keys x 32-row query tiles; the launch that writes them to
+// p.mask_t and sets their strides.
+int64_t bwd_mask_t_words(const goda_prefill_args& a);
+hipError_t launch_bwd_mask_t(BwdParams& p, hipStream_t s);
+// fp32 backward with operands streamed from L2.
+int64_t prefill_bwd_f32_workspace_bytes(const goda_prefill_args& a);
+hipError_t launch_prefill_bwd_f32(const BwdParams& p, hipStream_t s);
 int64_t prefill_bwd_mfma_workspace_bytes(const goda_prefill_args& a);
 hipError_t launch_prefill_bwd_mfma(BwdParams p, hipStream_t s);
 

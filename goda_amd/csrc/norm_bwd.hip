@@ -7,9 +7,6 @@
 // it); norm_bwd_kernel turns it into dx in place and writes one fp32 partial
 // of dw per workgroup; norm_dw_reduce_kernel sums the partials of both sides
 // in a fixed order (no atomics: the result does not depend on scheduling).
-// norm_rows_kernel writes the normalized rows themselves, for the backward
-// kernels that read q / k rows directly instead of through the MFMA path's
-// operand images.
 //
 // Row layout: a group of D/8 lanes holds one row, 8 elements per lane
 // (16-byte loads at 16-bit dtypes); a wave covers 512/D rows at a time and a
@@ -36,13 +33,13 @@ struct NormGeom {
 };
 
 struct NormRows {
-  const void* x;  // rows to normalize (the caller's q or k)
+  const void* x;  // rows before the norm (the caller's q or k)
   int64_t x_sb, x_st, x_sh;
-  void* y;        // norm_rows: normalized rows; norm_bwd: dy in, dx out
+  void* y;        // dy in, dx out
   int64_t y_sb, y_st, y_sh;
   const float* w;
   float eps;
-  float* part;    // norm_bwd: fp32 [gridDim.z][gridDim.y][gridDim.x][D]
+  float* part;    // fp32 [gridDim.z][gridDim.y][gridDim.x][D]
   int heads;
   bool q_side;    // rows of q (lengths lq) or of k (lengths lk)
 };
@@ -55,8 +52,8 @@ __device__ __forceinline__ int norm_len(const goda_prefill_args& a, int b, bool 
   return g.lk;
 }
 
-template <typename T, int D, bool BWD>
-__global__ void __launch_bounds__(256) norm_rows_kernel(const goda_prefill_args a, const NormRows n) {
+template <typename T, int D>
+__global__ void __launch_bounds__(256) norm_bwd_kernel(const goda_prefill_args a, const NormRows n) {
   typedef typename Vec<T>::v8 v8;
   typedef NormGeom<T, D> NG;
   const int b = blockIdx.z, h = blockIdx.y;
@@ -85,7 +82,7 @@ __global__ void __launch_bounds__(256) norm_rows_kernel(const goda_prefill_args 
     xv[k] = dv[k] = v8{};
     if (r < len) {
       xv[k] = ld_stream<v8>(xb + (row0 + r) * n.x_st);
-      if (BWD) dv[k] = ld_stream<v8>(yb + (row0 + r) * n.y_st);
+      dv[k] = ld_stream<v8>(yb + (row0 + r) * n.y_st);
     }
   }
 #pragma unroll
@@ -101,12 +98,6 @@ __global__ void __launch_bounds__(256) norm_rows_kernel(const goda_prefill_args 
     }
     const float rs = rms_scale(lane_group_sum<NG::LPR>(ss), D, n.eps);
     v8 out;
-    if (!BWD) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) out[e] = (T)(x[e] * rs * g[e]);
-      if (r < len) st_vec<v8>(yp, out);
-      continue;
-    }
     float dy[8], t = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -120,7 +111,6 @@ __global__ void __launch_bounds__(256) norm_rows_kernel(const goda_prefill_args 
     for (int e = 0; e < 8; ++e) out[e] = (T)(rs * (g[e] * dy[e] - x[e] * m));
     if (r < len) st_vec<v8>(yp, out);
   }
-  if (!BWD) return;
   // dw partial of this workgroup: row groups in slots, summed in slot order.
   __shared__ float sdw[NG::SLOTS][D];
 #pragma unroll
@@ -176,34 +166,31 @@ hipError_t launch_dw_reduce(const DwSum& q, const DwSum& k, int head_dim, hipStr
 }
 
 template <typename T, int D>
-hipError_t launch_rows(const goda_prefill_args& a, const NormRows& n, bool bwd, int64_t seqlen, hipStream_t s) {
+hipError_t launch_rows(const goda_prefill_args& a, const NormRows& n, int64_t seqlen, hipStream_t s) {
   const dim3 grid((unsigned)((seqlen + kNormRows - 1) / kNormRows), (unsigned)n.heads, (unsigned)a.batch);
   if (grid.x == 0 || grid.y == 0 || grid.z == 0) return hipSuccess;
-  if (bwd)
-    norm_rows_kernel<T, D, true><<<grid, 256, 0, s>>>(a, n);
-  else
-    norm_rows_kernel<T, D, false><<<grid, 256, 0, s>>>(a, n);
+  norm_bwd_kernel<T, D><<<grid, 256, 0, s>>>(a, n);
   return hipGetLastError();
 }
 
 template <typename T>
-hipError_t launch_rows_t(const goda_prefill_args& a, const NormRows& n, bool bwd, int64_t seqlen, hipStream_t s) {
+hipError_t launch_rows_t(const goda_prefill_args& a, const NormRows& n, int64_t seqlen, hipStream_t s) {
   switch (a.head_dim) {
     case 64:
-      return launch_rows<T, 64>(a, n, bwd, seqlen, s);
+      return launch_rows<T, 64>(a, n, seqlen, s);
     case 128:
-      return launch_rows<T, 128>(a, n, bwd, seqlen, s);
+      return launch_rows<T, 128>(a, n, seqlen, s);
     case 256:
-      return launch_rows<T, 256>(a, n, bwd, seqlen, s);
+      return launch_rows<T, 256>(a, n, seqlen, s);
     default:
       return hipErrorNotSupported;
   }
 }
 
-hipError_t launch_rows_any(const goda_prefill_args& a, const NormRows& n, bool bwd, int64_t seqlen, hipStream_t s) {
-  if (a.dtype == GODA_DTYPE_BF16) return launch_rows_t<bf16>(a, n, bwd, seqlen, s);
-  if (a.dtype == GODA_DTYPE_F16) return launch_rows_t<f16>(a, n, bwd, seqlen, s);
-  if (a.dtype == GODA_DTYPE_F32) return launch_rows_t<float>(a, n, bwd, seqlen, s);
+hipError_t launch_rows_any(const goda_prefill_args& a, const NormRows& n, int64_t seqlen, hipStream_t s) {
+  if (a.dtype == GODA_DTYPE_BF16) return launch_rows_t<bf16>(a, n, seqlen, s);
+  if (a.dtype == GODA_DTYPE_F16) return launch_rows_t<f16>(a, n, seqlen, s);
+  if (a.dtype == GODA_DTYPE_F32) return launch_rows_t<float>(a, n, seqlen, s);
   return hipErrorNotSupported;
 }
 
@@ -218,25 +205,6 @@ int64_t norm_bwd_part_bytes(const goda_prefill_args& a) {
   if (a.q_norm_weight) n += parts(a.seqlen_q, a.heads_q, a.batch);
   if (a.k_norm_weight) n += parts(a.seqlen_k, a.heads_kv, a.batch);
   return n * a.head_dim * (int64_t)sizeof(float);
-}
-
-hipError_t launch_norm_rows(const goda_prefill_args& a, bool q_side, void* dst, hipStream_t s) {
-  NormRows n{};
-  const int heads = q_side ? a.heads_q : a.heads_kv;
-  const int64_t seqlen = q_side ? a.seqlen_q : a.seqlen_k;
-  n.x = q_side ? a.q : a.k;
-  n.x_sb = q_side ? a.q_stride_b : a.k_stride_b;
-  n.x_st = q_side ? a.q_stride_t : a.k_stride_t;
-  n.x_sh = q_side ? a.q_stride_h : a.k_stride_h;
-  n.y = dst;  // contiguous [batch, seqlen, heads, D] (rows of packed sequences at their packed index)
-  n.y_sh = a.head_dim;
-  n.y_st = (int64_t)heads * a.head_dim;
-  n.y_sb = seqlen * n.y_st;
-  n.w = q_side ? a.q_norm_weight : a.k_norm_weight;
-  n.eps = a.norm_eps;
-  n.heads = heads;
-  n.q_side = q_side;
-  return launch_rows_any(a, n, false, seqlen, s);
 }
 
 hipError_t zero_norm_dw(const goda_prefill_args& a, const goda_prefill_grads& g, hipStream_t s) {
@@ -269,7 +237,7 @@ hipError_t launch_norm_bwd(const goda_prefill_args& a, const goda_prefill_grads&
     n.part = part;
     n.heads = heads;
     n.q_side = q_side;
-    if ((e = launch_rows_any(a, n, true, seqlen, s)) != hipSuccess) return e;
+    if ((e = launch_rows_any(a, n, seqlen, s)) != hipSuccess) return e;
     const int64_t np = parts(seqlen, heads, a.batch);
     sum[side] = DwSum{part, np, q_side ? g.dq_norm_weight : g.dk_norm_weight};
     part += np * a.head_dim;

@@ -454,3 +454,45 @@ def test_backward_fused_qk_norm_partial_sums(b, t, hq, hkv, d):
     """The rows of a norm workgroup (64) and the partials of a reduction round
     (64), one less, one more and several rounds, on both sides."""
     _norm_case(b, t, t, hq, hkv, d, torch.bfloat16, rope=False, seed=53)
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("b,tq,tk,hq,hkv,causal,window", [
+    (1, 1, 1, 1, 1, True, -1),  # one row, one key
+    (1, 33, 97, 3, 1, True, -1),  # partial tiles on both sides, more keys than rows
+    (2, 65, 65, 6, 2, True, -1),  # a third tile of one row, idle waves
+    (1, 160, 160, 5, 5, True, 32),  # windowed
+    (1, 40, 130, 4, 1, False, -1),
+])
+def test_backward_fp32_streamed(d, b, tq, tk, hq, hkv, causal, window):
+    """fp32 at the edges of its 32-row tiles, with the walks of dk/dv and dq
+    split over several waves and workgroups."""
+    _case(b, tq, tk, hq, hkv, d, torch.float32, causal=causal, seed=d + tq, window=window)
+
+
+def test_backward_fp32_without_stored_ds():
+    """Past 8 GB of dS tiles the dq kernel forms S and dP again: the gradients
+    of the whole batch are those of its halves, which store them. The two forms
+    differ in the order of dq's fp32 sums and in the rounding of the exponents'
+    bias terms: slopes of at most 0.707 / 64 over 4608 keys keep those under 74
+    log2 units, so two roundings change a probability by 2 * 74 * 2^-24 * ln 2
+    = 6.1e-6 of itself (at the slopes themselves it would be 3.9e-4), and
+    gradients of at most 1 stay within 1e-4."""
+    b, t, hq, d = 8, 4608, 16, 64
+    g = torch.Generator(device=DEV).manual_seed(5)
+    q, k, v, d_o = (torch.randn(b, t, h, d, device=DEV, generator=g) * 0.5 for h in (hq, 4, 4, hq))
+    slopes = torch.tensor(wl.alibi_slopes(hq), dtype=torch.float32, device=DEV) / 64
+    mask = torch.rand(b, 1, 1, t, device=DEV, generator=g) < 0.9
+
+    def grads(rows):
+        x = [y[rows].contiguous() for y in (q, k, v)]
+        kw = dict(causal=False, alibi_slopes=slopes, attn_mask=mask[rows])
+        o, lse = ops.attention_prefill(*x, return_lse=True, **kw)
+        plan = ops.plan_prefill_bwd(*x, o, lse, d_o[rows].contiguous(), **kw)
+        return plan(), plan.grads.workspace_bytes
+
+    whole, ws = grads(slice(0, b))
+    half, ws_half = grads(slice(0, 4))
+    assert ws < 8 << 30 and ws_half > 4 << 30  # recomputed / stored
+    for w, h in zip(whole, half):
+        assert (w[:4] - h).abs().max().item() <= 1e-4 * max(1.0, h.abs().max().item())
