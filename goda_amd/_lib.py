@@ -220,6 +220,8 @@ SYMBOLS = {
     "goda_attn_decode": (_i32, [ctypes.POINTER(DecodeArgs), _vp]),
     "goda_attn_decode_noalloc": (_i32, [ctypes.POINTER(DecodeArgs), _vp]),
     "goda_attn_kv_append": (_i32, [ctypes.POINTER(KvAppendArgs), _vp]),
+    "goda_attn_doc_segments_scratch_bytes": (_i64, [_i32, _i32]),
+    "goda_attn_doc_segments": (_i32, [_vp, _i32, _i64, _i32, _i32, _vp, _vp, _vp, _i64, _vp]),
 }
 
 _lock = threading.Lock()

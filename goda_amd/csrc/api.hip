@@ -75,10 +75,13 @@ int32_t check_prefill(const goda_prefill_args* a, bool need_ptrs) {
     // rope_q_offset + i); k rows at rope_k_offset + j.
     const int64_t qmax = (int64_t)a->rope_q_offset + (a->rope_pos_abs ? a->seqlen_q : a->seqlen_k) - 1;
     const int64_t kmax = (int64_t)a->rope_k_offset + a->seqlen_k - 1;
-    if (a->rope_q && (a->rope_q_offset < 0 || qmax >= a->rope_len))
+    if (a->rope_pos_abs == 2) {  // packed row index modulo rope_len: always inside the table
+      if (!a->cu_seqlens_q)
+        return fail(GODA_ERR_INVALID_ARG, "prefill: rope_pos_abs 2 needs packed rows (cu_seqlens)");
+    } else if (a->rope_q && (a->rope_q_offset < 0 || qmax >= a->rope_len))
       return fail(GODA_ERR_INVALID_ARG, "prefill: q positions up to %lld exceed rope_len %d",
                   (long long)qmax, a->rope_len);
-    if (a->rope_k && (a->rope_k_offset < 0 || kmax >= a->rope_len))
+    if (a->rope_pos_abs != 2 && a->rope_k && (a->rope_k_offset < 0 || kmax >= a->rope_len))
       return fail(GODA_ERR_INVALID_ARG, "prefill: k positions up to %lld exceed rope_len %d",
                   (long long)kmax, a->rope_len);
     if (a->rope_q && !a->rope_pos_abs && !a->cu_seqlens_q && a->seqlen_q > a->seqlen_k && !a->seqused_k)
@@ -281,6 +284,25 @@ int32_t goda_attn_kv_append(const goda_kv_append_args* a, void* stream) {
                   a->rope_len);
   }
   return hip_status(goda::launch_kv_append(*a, reinterpret_cast<hipStream_t>(stream)), "kv_append");
+}
+
+int64_t goda_attn_doc_segments_scratch_bytes(int32_t rows, int32_t cols) {
+  if (rows < 0 || cols < 0) return fail(GODA_ERR_INVALID_ARG, "doc_segments: negative size");
+  return ((int64_t)rows * cols + 3 * (int64_t)rows) * 4;
+}
+
+int32_t goda_attn_doc_segments(const void* ids, int32_t id_bytes, int64_t stride_row, int32_t rows, int32_t cols,
+                               int32_t* cu, int32_t* result, void* scratch, int64_t scratch_bytes, void* stream) {
+  if (rows <= 0 || cols <= 0 || (int64_t)rows * cols > 0x7fffffff)
+    return fail(GODA_ERR_INVALID_ARG, "doc_segments: bad sizes (rows %d, cols %d)", rows, cols);
+  if (id_bytes != 4 && id_bytes != 8) return fail(GODA_ERR_INVALID_ARG, "doc_segments: ids of %d bytes", id_bytes);
+  if (!ids || !cu || !result || !scratch) return fail(GODA_ERR_INVALID_ARG, "doc_segments: NULL pointer");
+  if (scratch_bytes < goda_attn_doc_segments_scratch_bytes(rows, cols))
+    return fail(GODA_ERR_WORKSPACE, "doc_segments: scratch of %lld bytes needed, %lld given",
+                (long long)goda_attn_doc_segments_scratch_bytes(rows, cols), (long long)scratch_bytes);
+  return hip_status(goda::launch_doc_segments(ids, id_bytes, stride_row, rows, cols, reinterpret_cast<int32_t*>(scratch), cu,
+                                              result, reinterpret_cast<hipStream_t>(stream)),
+                    "doc_segments");
 }
 
 }  // extern "C"

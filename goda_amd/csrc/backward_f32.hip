@@ -110,7 +110,7 @@ __global__ void __launch_bounds__(256) pack_q_f32_kernel(const BwdParams p) {
       o1 = ld_stream<f32x4>(orow);
       o2 = ld_stream<f32x4>(orow + D / 2);
     }
-    norm_rope_f32<D>(q1, q2, c, a.q_norm_weight, a.norm_eps, i < g.lq && a.rope_q, i < g.lq ? rope_qpos(a, diag, i) : 0,
+    norm_rope_f32<D>(q1, q2, c, a.q_norm_weight, a.norm_eps, i < g.lq && a.rope_q, i < g.lq ? rope_qpos(a, g, i) : 0,
                      a.rope_cos, a.rope_sin);
     st_vec<f32x4>(&qrows[r][c], q1);
     st_vec<f32x4>(&qrows[r][c + D / 2], q2);
@@ -164,7 +164,7 @@ __global__ void __launch_bounds__(256) pack_kv_bwd_f32_kernel(const BwdParams p)
       v1 = ld_stream<f32x4>(vr);
       v2 = ld_stream<f32x4>(vr + D / 2);
     }
-    norm_rope_f32<D>(k1, k2, c, a.k_norm_weight, a.norm_eps, row < g.lk && a.rope_k, a.rope_k_offset + row, a.rope_cos,
+    norm_rope_f32<D>(k1, k2, c, a.k_norm_weight, a.norm_eps, row < g.lk && a.rope_k, rope_kpos(a, g, row), a.rope_cos,
                      a.rope_sin);
     st_vec<f32x4>(&krows[r][c], k1);
     st_vec<f32x4>(&krows[r][c + D / 2], k2);
@@ -379,7 +379,7 @@ __global__ void __launch_bounds__(kWaves * 64, kWavesPerSimd<D>) bwd_dkv_f32_ker
       if (is_k) {
         x1 *= a.softmax_scale;
         x2 *= a.softmax_scale;
-        const int64_t at = (int64_t)(a.rope_k_offset + kr) * (D / 2) + d0;
+        const int64_t at = (int64_t)(rope_kpos(a, g, kr)) * (D / 2) + d0;
         if (a.rope_k && kr < g.lk) rotate_back(x1, x2, a.rope_cos + at, a.rope_sin + at);
         out = row_of(p.g.dk, p.g.dk_stride_b, p.g.dk_stride_t, p.g.dk_stride_h, varlen, b, g.k_row0 + kr, hk);
       } else {
@@ -424,7 +424,7 @@ __global__ void __launch_bounds__(256) bwd_dkv_reduce_f32_kernel(const BwdParams
   }
   k1 *= a.softmax_scale;
   k2 *= a.softmax_scale;
-  const int64_t at = (int64_t)(a.rope_k_offset + key) * (D / 2) + d0;
+  const int64_t at = (int64_t)(rope_kpos(a, g, key)) * (D / 2) + d0;
   if (a.rope_k && key < g.lk) rotate_back(k1, k2, a.rope_cos + at, a.rope_sin + at);
   float* krow = row_of(p.g.dk, p.g.dk_stride_b, p.g.dk_stride_t, p.g.dk_stride_h, varlen, b, g.k_row0 + key, hk) + d0;
   float* vrow = row_of(p.g.dv, p.g.dv_stride_b, p.g.dv_stride_t, p.g.dv_stride_h, varlen, b, g.k_row0 + key, hk) + d0;
@@ -593,7 +593,7 @@ __global__ void __launch_bounds__(kWaves * 64, (RECOMPUTE && D == 128 ? 1 : kWav
     x1 *= a.softmax_scale;
     x2 *= a.softmax_scale;
     if (a.rope_q) {
-      const int64_t at = (int64_t)rope_qpos(a, diag, qr0 + r) * (D / 2) + d0;
+      const int64_t at = (int64_t)rope_qpos(a, g, qr0 + r) * (D / 2) + d0;
       rotate_back(x1, x2, a.rope_cos + at, a.rope_sin + at);
     }
     float* out = row_of(p.g.dq, p.g.dq_stride_b, p.g.dq_stride_t, p.g.dq_stride_h, varlen, b, g.q_row0 + qr0 + r, hq) + d0;

@@ -259,7 +259,7 @@ __global__ void __launch_bounds__(256) pack_q_bwd_kernel(const BwdParams p) {
     }
     v8 qs1, qs2;
     norm_rope_row<T, D, HALF8>(q1, q2, c, a.q_norm_weight, a.norm_eps, i < g.lq && a.rope_q,
-                               i < g.lq ? rope_qpos(a, diag, i) : 0, a, p.scale_log2, &qs1, &qs2);
+                               i < g.lq ? rope_qpos(a, g, i) : 0, a, p.scale_log2, &qs1, &qs2);
     st_vec<v8>(&qsrows[r][c], qs1);
     st_vec<v8>(&qsrows[r][c + D / 2], qs2);
     st_vec<v8>(&grows[r][c], g1);
@@ -339,7 +339,7 @@ __global__ void __launch_bounds__(256) pack_kv_bwd_kernel(const BwdParams p) {
       v1 = ld_stream<v8>(vr + c);
       v2 = ld_stream<v8>(vr + c + D / 2);
     }
-    norm_rope_row<T, D, HALF8>(k1, k2, c, a.k_norm_weight, a.norm_eps, row < g.lk && a.rope_k, a.rope_k_offset + row,
+    norm_rope_row<T, D, HALF8>(k1, k2, c, a.k_norm_weight, a.norm_eps, row < g.lk && a.rope_k, rope_kpos(a, g, row),
                                a);
     st_vec<v8>(&krows[r][c], k1);
     st_vec<v8>(&krows[r][c + D / 2], k2);
@@ -730,7 +730,7 @@ __global__ void __launch_bounds__(kWavesKv * 64, 1) bwd_dkv_mfma_kernel(const Bw
       st_vec<v4>(row + 32 * md + 8 * gq + 4 * hi, v4{(T)x[4 * gq], (T)x[4 * gq + 1], (T)x[4 * gq + 2], (T)x[4 * gq + 3]});
   };
   const bool rot = a.rope_k && key < g.lk;
-  const int pos = a.rope_k_offset + key;
+  const int pos = rope_kpos(a, g, key);
   // dk: pairs of head-dim blocks (md, md + MD/2: the rotation's partners),
   // scaled and rotated back. dK^T accumulated against the row-major q image,
   // which holds q * scale * log2(e): dk = scale * (dS^T q) = ln(2) * dK^T.
@@ -1024,7 +1024,7 @@ __global__ void __launch_bounds__(kWavesWide * 64, 1) bwd_dkv_wide_kernel(const 
       st_vec<v4>(row + 32 * md + 8 * gq + 4 * hi, v4{(T)x[4 * gq], (T)x[4 * gq + 1], (T)x[4 * gq + 2], (T)x[4 * gq + 3]});
   };
   const bool rot = a.rope_k && key < g.lk;
-  const int pos = a.rope_k_offset + key;
+  const int pos = rope_kpos(a, g, key);
   // dk: one pair of head-dim blocks (md, md + MD/2: the rotation's partners)
   // at a time, scaled and rotated back.
   const float dks = kLn2;
@@ -1077,7 +1077,7 @@ __global__ void __launch_bounds__(256) bwd_dkv_reduce_kernel(const BwdParams p) 
   k1 *= kLn2;
   k2 *= kLn2;
   if (a.rope_k && key < g.lk) {
-    const int pos = a.rope_k_offset + key;
+    const int pos = rope_kpos(a, g, key);
     const f32x4 cs = ld_vec<f32x4>(a.rope_cos + (int64_t)pos * (D / 2) + d0);
     const f32x4 sn = ld_vec<f32x4>(a.rope_sin + (int64_t)pos * (D / 2) + d0);
     const f32x4 y1 = k1 * cs + k2 * sn;
@@ -1314,7 +1314,7 @@ __global__ void __launch_bounds__((DqShape<D>::WAVES * 64), (DqShape<D>::OCC)) b
 #pragma unroll
   for (int md = 0; md < MD; ++md) dq[md] *= a.softmax_scale;
   if (a.rope_q) {
-    const int pos = rope_qpos(a, diag, i);
+    const int pos = rope_qpos(a, g, i);
 #pragma unroll
     for (int md = 0; md < MD / 2; ++md)
 #pragma unroll
@@ -1486,7 +1486,7 @@ __global__ void __launch_bounds__(kWavesDqS * 64, 1) bwd_dq_ds_kernel(const BwdP
   // 32 md + 8 (r/4) + 4 hi + r%4.
   const int i = wrow0 + l32;
   if (i >= g.lq) return;
-  const int pos = a.rope_q ? rope_qpos(a, diag, i) : 0;
+  const int pos = a.rope_q ? rope_qpos(a, g, i) : 0;
 #pragma unroll
   for (int h = 0; h < HW; ++h) {
 #pragma unroll

@@ -181,10 +181,17 @@ __device__ __forceinline__ SeqGeom seq_geom(int b, int seqlen_q, int seqlen_k,
 }
 
 // RoPE position of query row i (0-based within its sequence; diag = Lk - Lq):
-// rope_q_offset + diag + i, or rope_q_offset + i with rope_pos_abs (a
-// caller-given start position), clamped into the table the host validated.
-__device__ __forceinline__ int rope_qpos(const goda_prefill_args& a, int diag, int i) {
-  return min(max(a.rope_q_offset + (a.rope_pos_abs ? 0 : diag) + i, 0), a.rope_len - 1);
+// rope_q_offset + diag + i, or rope_q_offset + i with rope_pos_abs 1 (a
+// caller-given start position), clamped into the table the host validated; with
+// rope_pos_abs 2 the packed row index modulo rope_len (its position in the
+// row of documents it was packed from). Key row j likewise.
+__device__ __forceinline__ int rope_qpos(const goda_prefill_args& a, const SeqGeom& g, int i) {
+  if (a.rope_pos_abs == 2) return (int)((uint32_t)(g.q_row0 + i) % (uint32_t)a.rope_len);
+  return min(max(a.rope_q_offset + (a.rope_pos_abs ? 0 : g.lk - g.lq) + i, 0), a.rope_len - 1);
+}
+__device__ __forceinline__ int rope_kpos(const goda_prefill_args& a, const SeqGeom& g, int j) {
+  if (a.rope_pos_abs == 2) return (int)((uint32_t)(g.k_row0 + j) % (uint32_t)a.rope_len);
+  return a.rope_k_offset + j;
 }
 
 // Row (b, query head h, query row i) of the bit-packed mask: bit j % 32 of

@@ -132,6 +132,10 @@ constexpr int64_t kDecodeScratchBytes = GODA_DECODE_NOALLOC_SCRATCH_BYTES;
 // device with hipGetSymbolAddress).
 hipError_t decode_scratch(void** ptr);
 
+// Document segments of packed rows (segments.hip).
+hipError_t launch_doc_segments(const void* ids, int elem_bytes, int64_t stride, int rows, int cols, int32_t* scratch,
+                               int32_t* cu, int32_t* out, hipStream_t s);
+
 hipError_t launch_kv_append(const goda_kv_append_args& a, hipStream_t s);
 
 // Records the caller's optional timing event (a hipEvent_t or NULL) on s.

@@ -191,7 +191,7 @@ __global__ void __launch_bounds__(256) pack_kv_kernel(const PrefillParams p) {
         x2[e] = (float)k2[e] * inv * (1.f + a.k_norm_weight[c + D / 2 + e]);
       }
       if (a.rope_k && row < g.lk) {
-        const int pos = a.rope_k_offset + row;
+        const int pos = rope_kpos(a, g, row);
         const float* cs = a.rope_cos + (int64_t)pos * (D / 2) + c;
         const float* sn = a.rope_sin + (int64_t)pos * (D / 2) + c;
 #pragma unroll
@@ -222,7 +222,7 @@ __global__ void __launch_bounds__(256) pack_kv_kernel(const PrefillParams p) {
       k1 = ld_stream<v8>(kr + c);
       k2 = ld_stream<v8>(kr + c + D / 2);
       if (a.rope_k) {
-        const int pos = a.rope_k_offset + row;
+        const int pos = rope_kpos(a, g, row);
         const float* cs = a.rope_cos + (int64_t)pos * (D / 2) + c;
         const float* sn = a.rope_sin + (int64_t)pos * (D / 2) + c;
         const f32x4 c0 = ld_vec<f32x4>(cs), c1 = ld_vec<f32x4>(cs + 4);
@@ -509,7 +509,7 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
             }
           }
           if (a.rope_q) {
-            const int pos = rope_qpos(a, diag, qi);
+            const int pos = rope_qpos(a, g, qi);
 #pragma unroll
             for (int ks = 0; ks < KS / 2; ++ks) {
               const int f0 = 16 * ks + 8 * hi;

@@ -35,8 +35,8 @@ Extra keyword arguments fuse the positional encoding into the kernels:
 UNROTATED), or `alibi_slopes` [Hq]; `qk_norm=(q_scale, k_scale, eps)` fuses
 goda's QK-RMSNorm (mint/nn/norm.py:17-27, weight 1 + scale, before RoPE) into
 the kernels' q/k loads, forward and backward (the backward also returns the
-two scales' gradients); with doc_ids packing, or a differentiable call over a
-KV cache, it runs as ordinary torch ops instead. There is no SDPA or CPU
+two scales' gradients); over a KV cache with doc_ids, or in a differentiable
+call, it runs as ordinary torch ops instead. There is no SDPA or CPU
 fallback.
 """
 
@@ -57,7 +57,12 @@ def _segments(doc_ids: torch.Tensor) -> tuple[torch.Tensor, int, bool]:
     every id occupies one run per row. Only then do the runs equal goda's
     mask doc_ids[i] == doc_ids[j] over the whole row
     (mint/nn/flashattn.py:238-240); goda's packing loader writes ids that way
-    (mint/data/dist/pretrain.py:243-273). One device-to-host read."""
+    (mint/data/dist/pretrain.py:243-273). On the GPU by `ops.doc_segments`; the
+    torch form below serves CPU tensors and what that one leaves open."""
+    if doc_ids.is_cuda:
+        found = ops.doc_segments(doc_ids)
+        if found is not None:
+            return found
     b, t = doc_ids.shape
     starts = torch.ones(b, t, dtype=torch.bool, device=doc_ids.device)
     starts[:, 1:] = doc_ids[:, 1:] != doc_ids[:, :-1]
@@ -117,9 +122,8 @@ class FlashAttention(nn.Module):
         # Only the left window is used: the reference's SDPA path reads
         # window_size[0] alone (mint/nn/flashattn.py:251-253, 258-264).
         window_left = window_size[0] if window_size[0] >= 0 else -1
-        if qk_norm is not None and (doc_ids is not None or (kv_cache is not None and _needs_grad(q, k, *qk_norm[:2]))):
-            # doc_ids packing rotates rows before the kernel (and the norm comes
-            # before RoPE); a differentiable call over a KV cache: plain torch.
+        if qk_norm is not None and kv_cache is not None and (doc_ids is not None or _needs_grad(q, k, *qk_norm[:2])):
+            # documents or a differentiable call over a KV cache: plain torch.
             q, k = headdim.rms_norm(q, qk_norm[0], qk_norm[2]), headdim.rms_norm(k, qk_norm[1], qk_norm[2])
             qk_norm = None
         base_attn_mask = _bool_base_mask(base_attn_mask, causal=causal, doc_ids=doc_ids)
@@ -166,11 +170,23 @@ class FlashAttention(nn.Module):
             if not segments[2]:
                 segments = None  # an id recurs in separate runs of a row: the dense mask below
         if segments is not None:
-            if rope is not None:
-                # Positions are row positions, not document positions: rotate
-                # in place on the GPU before packing (RoPE is applied before
-                # attention in goda too, mint/nn/attn.py:60).
-                q, k = _rotate(q, rope, start_pos), _rotate(k, rope, start_pos)
+            kw = _norm_kwargs(qk_norm, q=True, k=True)
+            if not headdim.is_native(d):
+                # norm and RoPE as torch ops, before the zero-padding
+                if qk_norm is not None:
+                    q, k = headdim.rms_norm(q, qk_norm[0], qk_norm[2]), headdim.rms_norm(k, qk_norm[1], qk_norm[2])
+                    kw = {}
+                if rope is not None:
+                    q, k = _rotate(q, rope, start_pos), _rotate(k, rope, start_pos)
+            elif rope is not None:
+                # Positions are row positions, not document positions: the
+                # kernels take a packed row's index modulo the row length
+                # (RoPE comes before attention in goda too, mint/nn/attn.py:60).
+                tables = [x[start_pos : start_pos + t] for x in rope]
+                if any(x.shape[0] != t for x in tables):
+                    raise ValueError(f"goda_amd FlashAttention: RoPE tables of {rope[0].shape[0]} positions; rows "
+                                     f"{start_pos} .. {start_pos + t - 1} are needed")
+                kw.update(rope_cos=tables[0], rope_sin=tables[1], rope_q=True, rope_k=True, rope_packed_rows=True)
             cu, max_len, _ = segments
             o = autograd.attention_prefill(
                 q.reshape(b * t, hq, d),
@@ -183,6 +199,7 @@ class FlashAttention(nn.Module):
                 cu_seqlens_k=cu,
                 max_seqlen_q=max_len,
                 max_seqlen_k=max_len,
+                **kw,
             )
             return o.reshape(b, t, hq, d)
         kw = _norm_kwargs(qk_norm, q=True, k=True)
@@ -270,6 +287,7 @@ def _norm_kwargs(qk_norm, *, q: bool, k: bool) -> dict:
 
 
 def _rotate(x: torch.Tensor, rope: tuple[torch.Tensor, torch.Tensor], start_pos: int) -> torch.Tensor:
+    # (documents of a head dim without kernels)
     t = x.shape[1]
     cos = rope[0][start_pos : start_pos + t][None, :, None, :].to(x.dtype)
     sin = rope[1][start_pos : start_pos + t][None, :, None, :].to(x.dtype)

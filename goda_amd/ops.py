@@ -217,6 +217,7 @@ def _prefill_args(
     rope_q_offset: int = 0,
     rope_k_offset: int = 0,
     rope_pos_abs: bool = False,
+    rope_packed_rows: bool = False,
     q_norm_weight: torch.Tensor | None = None,
     k_norm_weight: torch.Tensor | None = None,
     norm_eps: float = 1e-6,
@@ -236,7 +237,8 @@ def _prefill_args(
     `attn_mask` is a boolean mask broadcastable to [B, Hq, Lq, Lk] (or a
     `PackedMask`), composed with causal / window like goda's base_attn_mask;
     `rope_pos_abs` rotates query row i at rope_q_offset + i instead of
-    rope_q_offset + (Lk - Lq) + i."""
+    rope_q_offset + (Lk - Lq) + i; `rope_packed_rows` (varlen) rotates packed
+    query and key rows at their index modulo the length of the tables."""
     for name, t in (("q", q), ("k", k), ("v", v)):
         _require_gpu(name, t)
         _require_last_contig(name, t)
@@ -328,7 +330,7 @@ def _prefill_args(
     a.rope_cos, a.rope_sin, a.rope_len = _ptr(cos), _ptr(sin), rope_len
     a.rope_q, a.rope_k = int(bool(rope_q)), int(bool(rope_k))
     a.rope_q_offset, a.rope_k_offset = int(rope_q_offset), int(rope_k_offset)
-    a.rope_pos_abs = int(bool(rope_pos_abs))
+    a.rope_pos_abs = 2 if rope_packed_rows else int(bool(rope_pos_abs))
     qn = _f32_vec("q_norm_weight", q_norm_weight, d, dev)
     kn = _f32_vec("k_norm_weight", k_norm_weight, d, dev)
     a.q_norm_weight, a.k_norm_weight, a.norm_eps = _ptr(qn), _ptr(kn), float(norm_eps)
@@ -342,6 +344,31 @@ def _prefill_args(
 
     keep = (q, k, v, o, lse, slopes, cos, sin, cu_q, cu_k, used, qn, kn, pm)
     return a, keep, o, lse
+
+
+def doc_segments(doc_ids: torch.Tensor) -> tuple[torch.Tensor, int, bool] | None:
+    """cu_seqlens (int32, on the GPU) of the maximal runs of equal ids inside
+    each row of doc_ids [B, T], the longest run, and whether every id occupies
+    one run of its row, through `goda_attn_doc_segments`: two launches and one
+    read of three words. None where the kernel leaves the last question open
+    (over 1024 runs of ids in no order) or does not take the ids."""
+    _require_gpu("doc_ids", doc_ids)
+    if doc_ids.dim() != 2 or doc_ids.dtype not in (torch.int32, torch.int64) or not 0 < doc_ids.numel() < 1 << 31:
+        return None
+    if doc_ids.stride(1) != 1:
+        doc_ids = doc_ids.contiguous()
+    b, t = doc_ids.shape
+    lib = _lib.load()
+    need = int(lib.goda_attn_doc_segments_scratch_bytes(b, t))
+    scratch = torch.empty(need, dtype=torch.uint8, device=doc_ids.device)
+    out = torch.empty(3 + b * t + 1, dtype=torch.int32, device=doc_ids.device)
+    result, cu = out[:3], out[3:]
+    _lib.check(lib.goda_attn_doc_segments(doc_ids.data_ptr(), doc_ids.element_size(), doc_ids.stride(0), b, t, cu.data_ptr(),
+                                          result.data_ptr(), scratch.data_ptr(), need, _stream()))
+    count, longest, recurring = result.tolist()  # launch sizes (the reference synchronizes here too)
+    if recurring == 2:
+        return None
+    return cu[: count + 1], longest, recurring == 0
 
 
 def attention_prefill_bwd(q, k, v, o, lse, d_o, **kwargs):

@@ -112,7 +112,12 @@ typedef struct goda_prefill_args {
   int32_t rope_pos_abs;        /* 1: query row i rotates at rope_q_offset + i
                                   (a caller-given start position, as goda's
                                   RoPE(q, k, start_pos), mint/nn/pos.py:100-112);
-                                  0: at rope_q_offset + (Lk - Lq) + i */
+                                  0: at rope_q_offset + (Lk - Lq) + i;
+                                  2 (packed rows, cu_seqlens): query and key
+                                  rows rotate at their packed row index modulo
+                                  rope_len, the offsets unused: documents packed
+                                  from rows of rope_len tokens keep their
+                                  positions in the row */
 
   /* Fused QK-RMSNorm weights, fp32 [head_dim] each, or NULL (no norm on
    * that side; goda's q_norm / k_norm, mint/nn/norm.py:17-27, weight
@@ -321,6 +326,17 @@ int32_t goda_attn_decode_noalloc(const goda_decode_args* args, void* stream);
  * Replaces KVCache.update (mint/kvcache/base.py:35-50) without the
  * device-to-host read of mint/nn/flashattn.py:202. */
 int32_t goda_attn_kv_append(const goda_kv_append_args* args, void* stream);
+
+/* Document segments of goda's doc_ids [rows, cols] (row stride in elements,
+ * 4- or 8-byte integers): cu receives the rows * cols + 1 or fewer cumulative
+ * starts of the maximal runs of equal ids inside each row (a run never crosses a
+ * row), then rows * cols; result (3 words, device) = {number of runs, longest
+ * run, 1 if an id occupies more than one run of its row, 2 if that was not
+ * determined (over 1024 runs of ids in no order), else 0}. Replaces the
+ * doc_ids -> cu_seqlens conversion of mint/nn/flashattn.py:98-137. */
+int64_t goda_attn_doc_segments_scratch_bytes(int32_t rows, int32_t cols);
+int32_t goda_attn_doc_segments(const void* ids, int32_t id_bytes, int64_t stride_row, int32_t rows, int32_t cols,
+                               int32_t* cu, int32_t* result, void* scratch, int64_t scratch_bytes, void* stream);
 
 #ifdef __cplusplus
 }

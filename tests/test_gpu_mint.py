@@ -13,6 +13,7 @@ from goda_amd import workloads as wl
 from goda_amd.kernels_ import FlashAttentionGQAKernel, FlashAttentionMQAKernel
 from goda_amd.mint.kvcache import KVCache
 from goda_amd.mint.nn import ALiBiPositionalBias, FlashAttention, GroupedQueryAttention, LinearScaledRoPE, RoPE
+from goda_amd.mint.nn.flashattn import _segments
 from oracle import attention as ref
 from tests.helpers import TOL, max_err, rope_oracle
 
@@ -266,3 +267,60 @@ def test_kvcache_head_major_storage_decodes_like_contiguous():
     o1 = ops.attention_decode(q, kc, vc, seqlens)
     o2 = ops.attention_decode(q, kc.contiguous(), vc.contiguous(), seqlens)
     assert torch.equal(o1, o2)
+
+
+@pytest.mark.parametrize("dtype,d,tol", [(torch.float32, 64, 1e-4), (torch.bfloat16, 128, 2e-2), (torch.float32, 256, 1e-4)])
+@pytest.mark.parametrize("start_pos", [0, 5])
+def test_flashattention_doc_ids_fused_rope_and_norm(dtype, d, tol, start_pos):
+    """Documents packed from rows: RoPE at the row position (not the document's)
+    and the QK-norm before it, inside the kernels, forward and backward, equal
+    the same documents attended one row at a time by the dense kernels under
+    the document mask. The gradients' bound adds the storage rounding of the
+    largest reference gradient."""
+    t, hq, hkv = 70, 4, 2
+    doc = torch.tensor([[0] * 33 + [1] * 5 + [2] * 32, [7] * 1 + [3] * 69]).to(DEV)
+    g = torch.Generator().manual_seed(d)
+    q, k, v, d_o = ((torch.randn(2, t, h, d, generator=g) * 0.5).to(dtype).to(DEV) for h in (hq, hkv, hkv, hq))
+    wq, wk = ((torch.randn(d, generator=g) * 0.2).to(DEV) for _ in range(2))
+    rope = tuple(x.to(DEV) for x in wl.rope_tables(t + 9, d, 10000.0))
+    leaves = [x.requires_grad_(True) for x in (q, k, v, wq, wk)]
+    fa = FlashAttention()
+    kw = dict(causal=True, rope=rope, start_pos=start_pos, qk_norm=(wq, wk, 1e-6))
+    o = fa(q, k, v, doc_ids=doc, **kw)
+    got = torch.autograd.grad(o, leaves, d_o)
+    o_ref = fa(q, k, v, base_attn_mask=doc[:, None, :, None] == doc[:, None, None, :], **kw)
+    want = torch.autograd.grad(o_ref, leaves, d_o)
+    ulp = {torch.float32: 2.0**-24, torch.bfloat16: 2.0**-8}[dtype]
+    for x, y in zip((o, *got), (o_ref, *want)):
+        assert (x.float() - y.float()).abs().max().item() <= tol + ulp * y.float().abs().max().item()
+    with torch.no_grad():
+        assert torch.equal(fa(q, k, v, doc_ids=doc, **kw), o)
+
+
+def test_flashattention_doc_ids_refuses_short_tables():
+    q = torch.zeros(1, 8, 2, 64, device=DEV)
+    rope = tuple(x.to(DEV) for x in wl.rope_tables(10, 64, 10000.0))
+    with pytest.raises(ValueError):
+        FlashAttention()(q, q, q, causal=True, doc_ids=torch.zeros(1, 8, dtype=torch.long, device=DEV), rope=rope, start_pos=5)
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("b,t,kind", [(1, 1, "up"), (3, 255, "up"), (2, 256, "down"), (5, 257, "mixed"), (300, 17, "up"),
+                                      (2, 700, "recurring"), (1, 3000, "many"), (4, 1000, "one")])
+def test_doc_segments_match_the_torch_form(dtype, b, t, kind):
+    """The kernel's cu_seqlens, longest run and one-run-per-id flag against the
+    torch form on the CPU, at the edges of its 256-column steps, for ids in and
+    out of order, recurring ids, and more unordered runs than it compares."""
+    g = torch.Generator().manual_seed(b * t)
+    runs = torch.cumsum((torch.rand(b, t, generator=g) < (0.9 if kind == "many" else 0.05)).long(), 1)
+    ids = {"up": runs, "down": -runs, "mixed": (runs * 7919) % 10007, "recurring": runs % 5, "many": (runs * 7919) % 10007,
+           "one": torch.zeros_like(runs)}[kind].to(dtype)
+    cu, longest, one_run = _segments(ids)
+    found = ops.doc_segments(ids.to(DEV))
+    if kind == "many":
+        assert found is None
+        found = _segments(ids.to(DEV))
+    assert found[0].cpu().tolist() == cu.tolist() and found[1] == longest and found[2] == one_run
+    pad = torch.zeros(b, t + 3, dtype=dtype)
+    pad[:, :t] = ids
+    assert _segments(pad.to(DEV)[:, :t])[0].cpu().tolist() == cu.tolist()  # a row stride
