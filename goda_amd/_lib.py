@@ -204,6 +204,23 @@ class PrefillGrads(ctypes.Structure):
     ]
 
 
+class PackMaskArgs(ctypes.Structure):
+    _fields_ = [
+        ("mask", _vp),
+        ("stride_b", _i64),
+        ("stride_h", _i64),
+        ("stride_q", _i64),
+        ("stride_k", _i64),
+        ("batch", _i32),
+        ("heads", _i32),
+        ("rows", _i32),
+        ("keys", _i32),
+        ("mask_keys", _i32),
+        ("reserved0", _i32),
+        ("bits", _vp),
+    ]
+
+
 # Every symbol the header declares, with its ctypes signature.
 SYMBOLS = {
     "goda_attn_abi_version": (_i32, []),
@@ -220,6 +237,8 @@ SYMBOLS = {
     "goda_attn_decode": (_i32, [ctypes.POINTER(DecodeArgs), _vp]),
     "goda_attn_decode_noalloc": (_i32, [ctypes.POINTER(DecodeArgs), _vp]),
     "goda_attn_kv_append": (_i32, [ctypes.POINTER(KvAppendArgs), _vp]),
+    "goda_attn_sizeof_pack_mask_args": (_i64, []),
+    "goda_attn_pack_mask": (_i32, [ctypes.POINTER(PackMaskArgs), _vp]),
     "goda_attn_doc_segments_scratch_bytes": (_i64, [_i32, _i32]),
     "goda_attn_doc_segments": (_i32, [_vp, _i32, _i64, _i32, _i32, _vp, _vp, _vp, _i64, _vp]),
 }
@@ -268,6 +287,7 @@ def load() -> ctypes.CDLL:
             (DecodeArgs, lib.goda_attn_sizeof_decode_args),
             (KvAppendArgs, lib.goda_attn_sizeof_kv_append_args),
             (PrefillGrads, lib.goda_attn_sizeof_prefill_grads),
+            (PackMaskArgs, lib.goda_attn_sizeof_pack_mask_args),
         ):
             if ctypes.sizeof(struct) != fn():
                 raise RuntimeError(

@@ -286,6 +286,19 @@ int32_t goda_attn_kv_append(const goda_kv_append_args* a, void* stream) {
   return hip_status(goda::launch_kv_append(*a, reinterpret_cast<hipStream_t>(stream)), "kv_append");
 }
 
+int64_t goda_attn_sizeof_pack_mask_args(void) { return sizeof(goda_pack_mask_args); }
+
+int32_t goda_attn_pack_mask(const goda_pack_mask_args* a, void* stream) {
+  if (!a) return fail(GODA_ERR_INVALID_ARG, "pack_mask: args is NULL");
+  if (a->batch < 0 || a->heads < 0 || a->rows < 0 || a->keys < 0 || a->mask_keys < 0 || a->mask_keys > a->keys)
+    return fail(GODA_ERR_INVALID_ARG, "pack_mask: bad sizes (batch %d, heads %d, rows %d, keys %d, mask_keys %d)", a->batch,
+                a->heads, a->rows, a->keys, a->mask_keys);
+  if ((int64_t)a->batch * a->heads * a->rows * a->keys == 0) return ok();
+  if (!a->mask || !a->bits || (reinterpret_cast<uintptr_t>(a->bits) & 7) != 0)
+    return fail(GODA_ERR_INVALID_ARG, "pack_mask: mask is NULL or bits not an 8-byte aligned pointer");
+  return hip_status(goda::launch_pack_mask(*a, reinterpret_cast<hipStream_t>(stream)), "pack_mask");
+}
+
 int64_t goda_attn_doc_segments_scratch_bytes(int32_t rows, int32_t cols) {
   if (rows < 0 || cols < 0) return fail(GODA_ERR_INVALID_ARG, "doc_segments: negative size");
   return ((int64_t)rows * cols + 3 * (int64_t)rows) * 4;

@@ -132,6 +132,9 @@ constexpr int64_t kDecodeScratchBytes = GODA_DECODE_NOALLOC_SCRATCH_BYTES;
 // device with hipGetSymbolAddress).
 hipError_t decode_scratch(void** ptr);
 
+// Bit-packed boolean mask (mask.hip).
+hipError_t launch_pack_mask(const goda_pack_mask_args& a, hipStream_t s);
+
 // Document segments of packed rows (segments.hip).
 hipError_t launch_doc_segments(const void* ids, int elem_bytes, int64_t stride, int rows, int cols, int32_t* scratch,
                                int32_t* cu, int32_t* out, hipStream_t s);

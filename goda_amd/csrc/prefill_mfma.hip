@@ -113,6 +113,12 @@ constexpr bool kSplitStaging = D >= 128;
 template <int D>
 constexpr bool kPersistent = D <= 128;
 
+// With a caller's mask: key tiles that no row of the workgroup sees are not
+// walked. The tiles that are stand in a list behind the LDS ring, for up to
+// this many tiles (more: all are walked).
+constexpr int kListTiles = 4096;
+constexpr int kListBytes = kListTiles * 2 + kListTiles / 8;
+
 // Index of workspace tile j of sequence b, KV head hk.
 __device__ __forceinline__ int64_t ws_tile(int b, int j, int hk, int ntiles, int hkv) {
   return ((int64_t)b * ntiles + j) * hkv + hk;
@@ -552,15 +558,22 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
   if (causal) kv_hi = min(kv_hi, diag + q_last + 1);
   int kv_lo = 0;
   if (use_window) kv_lo = max(0, diag + qr0 - window_left);
-  const int j_lo = kv_lo / BKV;
-  const int j_hi = kv_hi > 0 ? (kv_hi + BKV - 1) / BKV : 0;
+  int j_lo = kv_lo / BKV;
+  int j_hi = kv_hi > 0 ? (kv_hi + BKV - 1) / BKV : 0;
   // Key tile of step j. With ALiBi the steps walk the tiles from the last
   // down: the bias slope*(key - row) grows along the keys, so the first tile
   // holds (nearly) every row's max and the lazy rescale seldom fires again;
   // in key order the max moved by the slope per key and rescaled often.
   // Stages and loop bounds stay in step order.
-  const int j_rev = j_lo + j_hi - 1;
-  auto tile_of = [&](int j) { return ALIBI ? j_rev - j : j; };
+  // With a caller's mask (and a tile list, below) step j is entry j of the list.
+  const uint16_t* tile_list = nullptr;
+  int j_rev = j_lo + j_hi - 1;
+  auto tile_of = [&](int j) {
+    const int i = ALIBI ? j_rev - j : j;
+    if constexpr (MASK)
+      if (tile_list) return __builtin_amdgcn_readfirstlane((int)tile_list[i]);
+    return i;
+  };
 
   f32x16 oacc[MD][NT];
 #pragma unroll
@@ -604,6 +617,48 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
     for (int nt = 0; nt < NT; ++nt) {
       mrow[nt] = reinterpret_cast<const mword_t*>(mask_row(a, b, hq, min(wrow0 + 32 * nt + l32, g.lq - 1)));
       mw[nt] = MaskWord<BKV>::kAll;
+    }
+    // The list of the tiles that hold a visible key: each wave marks those of
+    // its rows in a bit set, lanes l and l ^ 32 two tiles of a row at a time;
+    // then a tile's place is the number of marked tiles before it. (Masks of
+    // documents, prefixes or padding hide whole tiles, which otherwise cost
+    // as much as visible ones: B=4, T=2048, 16/4 heads, a prefix mask over
+    // half the tiles, 142 -> 121 us.)
+    const int ntl = j_hi - j_lo;
+    if (ntl > 0 && ntl <= kListTiles) {
+      uint16_t* list = reinterpret_cast<uint16_t*>(smem + kStages * TG::BYTES);
+      uint32_t* seen = reinterpret_cast<uint32_t*>(list + kListTiles);
+      const int nw = (ntl + 31) / 32;
+      for (int i = tid; i < nw; i += WAVES * 64) seen[i] = 0;
+      __syncthreads();
+#pragma unroll 4
+      for (int t = 0; t < ntl; t += 2) {
+        const int u = t + hi;
+        bool any = false;
+        if (u < ntl) {
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) any = any || mrow[nt][j_lo + u] != 0;
+        }
+        const uint64_t m = __builtin_amdgcn_ballot_w64(any);
+        const uint32_t pair = ((uint32_t)m != 0 ? 1u : 0u) | ((uint32_t)(m >> 32) != 0 ? 2u : 0u);
+        if (pair && lane == 0) atomicOr(&seen[t >> 5], pair << (t & 31));
+      }
+      __syncthreads();
+      int total = 0;
+      for (int t = tid; t < nw * 32; t += WAVES * 64) {
+        const uint32_t w = seen[t >> 5];
+        if ((w >> (t & 31)) & 1u) {
+          int at = __popc(w & ((1u << (t & 31)) - 1u));
+          for (int i = 0; i < (t >> 5); ++i) at += __popc(seen[i]);
+          list[at] = (uint16_t)(j_lo + t);
+        }
+      }
+      for (int i = 0; i < nw; ++i) total += __popc(seen[i]);
+      __syncthreads();
+      tile_list = list;
+      j_lo = 0;
+      j_hi = __builtin_amdgcn_readfirstlane(total);
+      j_rev = j_hi - 1;
     }
   }
 
@@ -1221,7 +1276,7 @@ hipError_t launch_attn(PrefillParams p, hipStream_t s) {
   const int64_t nblk = (int64_t)nqt * a.batch * a.heads_kv * (p.group / hg);
   if (nblk <= 0) return hipSuccess;
   if (nblk > 0x7fffffff) return hipErrorInvalidValue;
-  const size_t lds = (size_t)kStages * TileGeom<T, D, C::BKV, C::WAVES>::BYTES;
+  const size_t lds = (size_t)kStages * TileGeom<T, D, C::BKV, C::WAVES>::BYTES + (MASK ? kListBytes : 0);
   auto kern = prefill_fa_kernel<T, D, C::BKV, C::NT, C::WAVES, ALIBI, MASK, false>;
   hipError_t e;
   // Persistent grid (see prefill_fa_kernel): head_dim <= 128, dense batches

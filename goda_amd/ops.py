@@ -105,23 +105,32 @@ def pack_mask(
     if m.shape[3] not in (1, seqlen_k) and not allow_short_keys:
         raise ValueError(f"goda_amd: base_attn_mask has {m.shape[3]} keys; the attention has {seqlen_k}")
     m = m.to(device)
+    # a dimension expanded to its size (stride 0) is one mask for all of it
+    for dim in range(3):
+        if m.shape[dim] > 1 and m.stride(dim) == 0:
+            m = m.narrow(dim, 0, 1)
     bm, hm, qm, lk = m.shape
-    if lk == 1:
-        m = m.expand(bm, hm, qm, seqlen_k)
-        lk = seqlen_k
+    if not m.is_cuda:
+        bits = _pack_bits_cpu(m, seqlen_k)
+        return PackedMask(bits, *(bits.stride(i) if m.shape[i] > 1 else 0 for i in range(3)), seqlen_k)
+    bits = torch.empty(bm, hm, qm, 2 * ((seqlen_k + 63) // 64), dtype=torch.int32, device=m.device)
+    a = _lib.PackMaskArgs()
+    a.mask, a.bits = m.data_ptr(), bits.data_ptr()
+    a.stride_b, a.stride_h, a.stride_q = m.stride(0), m.stride(1), m.stride(2)
+    a.stride_k = 0 if lk == 1 else m.stride(3)  # one byte for every key
+    a.batch, a.heads, a.rows, a.keys, a.mask_keys = bm, hm, qm, seqlen_k, seqlen_k if lk == 1 else lk
+    _lib.check(_lib.load().goda_attn_pack_mask(ctypes.byref(a), _stream()))
+    return PackedMask(bits, *(bits.stride(i) if m.shape[i] > 1 else 0 for i in range(3)), seqlen_k)
+
+
+def _pack_bits_cpu(m: torch.Tensor, seqlen_k: int) -> torch.Tensor:
+    bm, hm, qm, lk = m.shape
     words = 2 * ((seqlen_k + 63) // 64)
-    u8 = torch.zeros(bm, hm, qm, words * 32, dtype=torch.uint8, device=device)
-    u8[..., :lk] = m
-    weights = torch.tensor([1, 2, 4, 8, 16, 32, 64, 128], dtype=torch.uint8, device=device)
+    u8 = torch.zeros(bm, hm, qm, words * 32, dtype=torch.uint8)
+    u8[..., : seqlen_k if lk == 1 else lk] = m
+    weights = torch.tensor([1, 2, 4, 8, 16, 32, 64, 128], dtype=torch.uint8)
     by = (u8.view(bm, hm, qm, words * 4, 8) * weights).sum(-1, dtype=torch.uint8)
-    bits = by.contiguous().view(torch.int32)  # little-endian: byte k holds keys 8k .. 8k+7
-    return PackedMask(
-        bits,
-        bits.stride(0) if bm > 1 else 0,
-        bits.stride(1) if hm > 1 else 0,
-        bits.stride(2) if qm > 1 else 0,
-        seqlen_k,
-    )
+    return by.contiguous().view(torch.int32)  # little-endian: byte k holds keys 8k .. 8k+7
 
 
 def _rope_tables(cos: torch.Tensor | None, sin: torch.Tensor | None, head_dim: int, device):

@@ -327,6 +327,20 @@ int32_t goda_attn_decode_noalloc(const goda_decode_args* args, void* stream);
  * device-to-host read of mint/nn/flashattn.py:202. */
 int32_t goda_attn_kv_append(const goda_kv_append_args* args, void* stream);
 
+/* Bit-packs a boolean mask (one byte a key, any nonzero byte visible) of any
+ * byte strides into the words of goda_prefill_args.mask_bits: bits receives
+ * [batch][heads][rows][2 * ceil(keys / 64)] contiguous words; key j >= mask_keys
+ * is hidden. stride_k 0 with mask_keys = keys broadcasts one byte to every key. */
+typedef struct goda_pack_mask_args {
+  const void* mask;
+  int64_t stride_b, stride_h, stride_q, stride_k; /* bytes */
+  int32_t batch, heads, rows, keys, mask_keys;
+  int32_t reserved0;
+  void* bits;
+} goda_pack_mask_args;
+int64_t goda_attn_sizeof_pack_mask_args(void);
+int32_t goda_attn_pack_mask(const goda_pack_mask_args* args, void* stream);
+
 /* Document segments of goda's doc_ids [rows, cols] (row stride in elements,
  * 4- or 8-byte integers): cu receives the rows * cols + 1 or fewer cumulative
  * starts of the maximal runs of equal ids inside each row (a run never crosses a

@@ -176,3 +176,64 @@ def test_flashattention_right_window_is_ignored_like_the_reference():
     assert torch.equal(o_lr, o_l)
     o_ref = ref.attention(q.cpu().float(), k.cpu().float(), v.cpu().float(), causal=True, window_size=(17, 5))
     assert max_err(o_lr, o_ref) <= TOL[torch.bfloat16]
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (2, 1, 3, 31), (1, 3, 5, 64), (2, 2, 7, 257), (1, 1, 1, 4100)])
+@pytest.mark.parametrize("form", ["plain", "offset", "strided", "expanded", "one key"])
+def test_pack_mask_kernel_matches_the_cpu_form(shape, form):
+    """The packing kernel's words against the CPU form: ragged and unaligned
+    rows, key strides other than 1, expanded dimensions, one byte for all keys,
+    and bytes other than 0 and 1."""
+    b, h, tq, tk = shape
+    g = torch.Generator().manual_seed(tk)
+    m = torch.randint(0, 3, shape, generator=g, dtype=torch.uint8)
+    if form == "offset":
+        m = torch.cat([torch.zeros(b, h, tq, 3, dtype=torch.uint8), m], -1)[..., 3:]
+    elif form == "strided":
+        m = torch.stack([m, 1 - m.clamp(max=1)], -1)[..., 0]
+    elif form == "expanded":
+        m = m[:1, :1, :1].expand(b, h, tq, tk)
+    elif form == "one key":
+        m = m[..., :1]
+    dev = torch.as_strided(m.contiguous().to(DEV), m.shape, m.contiguous().stride()) if form in ("plain", "one key") else None
+    if dev is None:  # the same strides on the GPU
+        base = torch.empty(0, dtype=torch.uint8).set_(m.untyped_storage()).to(DEV)
+        dev = torch.as_strided(base, m.shape, m.stride(), m.storage_offset())
+    want = ops.pack_mask((m != 0), b, h, tq, tk, "cpu")
+    got = ops.pack_mask(dev.view(torch.bool), b, h, tq, tk, DEV)
+    full = lambda p: torch.as_strided(p.bits.cpu(), (b, h, tq, p.bits.shape[-1]), (p.stride_b, p.stride_h, p.stride_q, 1))  # noqa: E731
+    assert torch.equal(full(got), full(want))
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.bfloat16, 128), (torch.float16, 256), (torch.float32, 128)])
+@pytest.mark.parametrize("causal,alibi", [(True, False), (False, False), (False, True)])
+@pytest.mark.parametrize("tk", [64, 65, 330, 2100])
+def test_mask_of_hidden_tiles(dtype, d, causal, alibi, tk):
+    """Masks that hide whole key tiles: none, all or some of a workgroup's, the
+    first and the last among them, other tiles in other row blocks and heads."""
+    b, hq, hkv, tq = 2, 4, 2, min(tk, 330)
+    q, k, v = _rand((b, tq, hq, d), dtype, 1), _rand((b, tk, hkv, d), dtype, 2), _rand((b, tk, hkv, d), dtype, 3)
+    g = torch.Generator().manual_seed(tk)
+    blocks = torch.rand((b, hq, (tq + 31) // 32, (tk + 31) // 32), generator=g) < 0.3
+    blocks[0, :, 2:6] = False  # rows without a key
+    if blocks.shape[2] > 8:
+        blocks[1, :, 4:6, :3] = False
+    m = blocks.repeat_interleave(32, 2)[:, :, :tq].repeat_interleave(32, 3)[..., :tk]
+    slopes = torch.tensor(wl.alibi_slopes(hq), dtype=torch.float32) if alibi else None
+    o, lse = ops.attention_prefill(q.to(DEV), k.to(DEV), v.to(DEV), causal=causal, attn_mask=m.to(DEV), return_lse=True,
+                                   alibi_slopes=None if slopes is None else slopes.to(DEV))
+    o_ref, lse_ref = ref.attention_rows(q.float(), k.float(), v.float(), torch.arange(tq), causal=causal, base_attn_mask=m,
+                                        alibi_slopes=slopes)
+    assert max_err(o, torch.nan_to_num(o_ref)) <= TOL[dtype]
+    assert lse_err(lse, lse_ref) <= (5e-3 if dtype != torch.float32 else 1e-4) * max(1.0, tk / 300 if alibi else 1.0)
+
+
+def test_mask_over_more_tiles_than_the_list_holds():
+    """Over 4096 key tiles every tile is walked; one key tile in 50 is visible."""
+    tk, d = 64 * 4096 + 40, 64
+    q, k, v = (_rand((1, t, 1, d), torch.bfloat16, s).to(DEV) for t, s in ((2, 1), (tk, 2), (tk, 3)))
+    m = (torch.arange(tk, device=DEV) // 64 % 50 == 49)[None, None, None]
+    o = ops.attention_prefill(q, k, v, causal=False, attn_mask=m)
+    keep = m[0, 0, 0]
+    o_ref = ops.attention_prefill(q, k[:, keep].contiguous(), v[:, keep].contiguous(), causal=False)
+    assert max_err(o, o_ref) <= TOL[torch.bfloat16]
