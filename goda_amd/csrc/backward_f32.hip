@@ -668,7 +668,7 @@ hipError_t launch_main(BwdParams p, hipStream_t s) {
     }
   }
   if (p.ntq > 0) {
-    p.key_split = f32_key_split((int64_t)p.ntq * a.heads_q * a.batch, p.ntk);
+    p.key_split = f32_key_split(a, (int64_t)p.ntq * a.heads_q * a.batch);
     const int per_wg = kWaves / p.key_split;
     const int64_t nblk = ((int64_t)p.ntq * p.group + per_wg - 1) / per_wg * a.heads_kv * a.batch;
     if (nblk > 0x7fffffff) return hipErrorInvalidValue;

@@ -111,11 +111,23 @@ hipError_t launch_prefill_mfma(const PrefillParams& p, hipStream_t s);
 bool prefill_f32_streams(const goda_prefill_args& a);
 int64_t prefill_f32_workspace_bytes(const goda_prefill_args& a);
 hipError_t launch_prefill_f32(const PrefillParams& p, hipStream_t s);
-// Waves that share the key tiles of an fp32 item (32 query rows of one head):
-// enough that `items` fill the GPU, at most one per key tile.
-inline int f32_key_split(int64_t items, int ntiles_k) {
-  const int split = items <= 2048 ? 4 : items <= 4096 ? 2 : 1;
-  return ntiles_k < split ? (ntiles_k >= 2 ? 2 : 1) : split;
+// Waves of a workgroup that share the key tiles of an fp32 item (32 query rows
+// of one head; `items` of them). Few items: four waves each, so that they fill
+// the GPU. More: the longest items of a long walk still end the kernel, so they
+// are shared (four ways, two at head_dim 256 with its one wave per SIMD); a
+// short walk only pays the sums. Forward us at 1 / 2 / 4 waves, causal:
+//   B=2 T=512 6/2 D=128      192 items   75 /  46 /  32
+//   B=2 T=1000 8/2 D=256     512 items  280 / 161 / 119
+//   B=16 T=512 4/4 D=128    1024 items   89 /  92 /  95 (window 128: 48 / 50 / 64)
+//   B=1 T=2048 16/1 D=256   1024 items  542 / 324 / 348
+//   B=1 T=2048 32/8 D=128   2048 items  430 / 308 / 320
+//   B=4 T=2048 16/16 D=64   4096 items  443 / 413 / 375
+//   B=8 T=4096 16/1 D=256  16384 items 8660 / 8941 / 9371
+inline int f32_key_split(const goda_prefill_args& a, int64_t items) {
+  int tiles = (a.seqlen_k + 31) / 32;
+  if (a.window_left >= 0 && a.causal && a.window_left / 32 + 2 < tiles) tiles = a.window_left / 32 + 2;
+  const int split = items <= 512 ? 4 : items > 4096 || tiles < 32 ? 1 : a.head_dim == 256 ? 2 : 4;
+  return tiles >= split ? split : tiles >= 2 ? 2 : 1;
 }
 
 // Split-K decode (bf16 / fp16 / fp32).

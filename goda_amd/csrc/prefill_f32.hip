@@ -356,7 +356,7 @@ hipError_t launch_attn(PrefillParams p, hipStream_t s) {
   const goda_prefill_args& a = p.a;
   p.qtiles = (a.seqlen_q + kF32Rows - 1) / kF32Rows;
   const int64_t items = (int64_t)p.qtiles * a.heads_q * a.batch;
-  p.key_split = f32_key_split(items, (a.seqlen_k + kF32Rows - 1) / kF32Rows);
+  p.key_split = f32_key_split(a, items);
   const int per_wg = kWaves / p.key_split;
   const int64_t nblk = ((int64_t)p.qtiles * p.group + per_wg - 1) / per_wg * a.heads_kv * a.batch;
   if (nblk > 0x7fffffff) return hipErrorInvalidValue;
