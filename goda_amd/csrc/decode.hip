@@ -24,6 +24,7 @@
 //           broadcast through LDS (16-bit types: packed dot products over
 //           key pairs, p rounded to T); the lane mapping is described at VRows.
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -162,17 +163,51 @@ __device__ __forceinline__ int visible(const goda_decode_args& a, int b, int* kb
   return L - k0;
 }
 
+// x / y for wave-uniform x >= 0, y > 0: in 32 bits where both fit (a 64-bit
+// division is some 150 instructions).
+__device__ __forceinline__ int64_t udiv(int64_t x, int64_t y) {
+  if (((x | y) >> 32) == 0) return (int64_t)((uint32_t)x / (uint32_t)y);
+  return x / y;
+}
+
 // Keys per range: the caller's split, else total / grid rounded up.
 __device__ __forceinline__ int64_t range_keys(int64_t total, int grid, int split) {
   if (split > 0) return split;
-  const int64_t q = (total + grid - 1) / grid;
-  return max((int64_t)kMinRange, (q + kMinRange - 1) / kMinRange * kMinRange);
+  const int64_t q = udiv(total + grid - 1, grid);
+  static_assert((kMinRange & (kMinRange - 1)) == 0, "ranges rounded up by a mask");
+  return max((int64_t)kMinRange, (q + kMinRange - 1) & ~(int64_t)(kMinRange - 1));
 }
+
+// The visible key counts of up to 64 sequences in one register of the wave
+// (lane = sequence) with their running sums: read and summed once for the
+// total, the position of a range and the keys before a sequence. `ok` where
+// 32 bits hold the sums; other batches go through the loops below.
+struct Lens {
+  bool ok;
+  int n, k0, incl;
+  __device__ __forceinline__ explicit Lens(const goda_decode_args& a) : ok(a.batch <= 64 && a.max_seqlen < (1 << 25)), n(0), k0(0), incl(0) {
+    if (!ok) return;
+    const int lane = threadIdx.x & 63;
+    if (lane < a.batch) n = visible(a, lane, &k0);
+    incl = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int t = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += t;
+    }
+  }
+  __device__ __forceinline__ int at(int v, int l) const { return __builtin_amdgcn_readlane(v, l); }
+};
 
 // Wave-wide sums of the visible key counts: over all sequences, and over the
 // sequences before `b` (every lane returns both).
-__device__ __forceinline__ void visible_sums(const goda_decode_args& a, int b, long long* all,
+__device__ __forceinline__ void visible_sums(const goda_decode_args& a, const Lens& s64, int b, long long* all,
                                              long long* before) {
+  if (s64.ok) {
+    *all = s64.at(s64.incl, 63);
+    *before = s64.at(s64.incl, b) - s64.at(s64.n, b);
+    return;
+  }
   const int lane = threadIdx.x & 63;
   long long s = 0, sb = 0;
   for (int i = lane; i < a.batch; i += 64) {
@@ -199,8 +234,14 @@ struct Cursor {
 
 // The sequence holding flattened position R (R < total), by a wave-wide
 // inclusive scan of U * n over 64 sequences at a time.
-__device__ Cursor locate(const goda_decode_args& a, int U, int64_t R) {
+__device__ Cursor locate(const goda_decode_args& a, const Lens& s64, int U, int64_t R) {
   const int lane = threadIdx.x & 63;
+  if (s64.ok) {
+    const uint64_t hit = __builtin_amdgcn_ballot_w64((int64_t)U * s64.incl > R);
+    const int l = __builtin_ctzll(hit);  // (R < total: some lane's sum exceeds it)
+    const int n = s64.at(s64.n, l);
+    return Cursor{l, s64.at(s64.k0, l), n, (int64_t)U * (s64.at(s64.incl, l) - n)};
+  }
   long long base = 0;
   Cursor c{0, 0, 0, 0};
   for (int b0 = 0; b0 < a.batch; b0 += 64) {
@@ -654,22 +695,23 @@ decode_splitk_kernel(const DecodeParams p) {
   const goda_decode_args& a = p.a;
   const int nhs = (p.group + HMAX - 1) / HMAX;
   const int U = a.heads_kv * nhs;
+  const Lens lens(a);
   long long all, unused;
-  visible_sums(a, 0, &all, &unused);
+  visible_sums(a, lens, 0, &all, &unused);
   const int64_t total = (int64_t)U * all;
   const int64_t per = range_keys(total, gridDim.x, p.split);
-  const int64_t nranges = (total + per - 1) / per;
+  const int64_t nranges = udiv(total + per - 1, per);
 
   for (int64_t r = blockIdx.x; r < nranges; r += gridDim.x) {
     const int64_t R0 = r * per;
     const int64_t R1 = min(total, R0 + per);
-    Cursor cur = locate(a, U, R0);
+    Cursor cur = locate(a, lens, U, R0);
     int64_t pos = R0;
     bool first = true;
     while (pos < R1) {
       if (pos >= cur.base + (int64_t)U * cur.n && !advance(a, U, cur)) return;
       const int64_t in_b = pos - cur.base;
-      const int j = uniform((int)(in_b / cur.n));
+      const int j = uniform((int)udiv(in_b, cur.n));
       const int off = uniform((int)(in_b - (int64_t)j * cur.n));
       const int len = (int)min((int64_t)(cur.n - off), R1 - pos);
       Segment sg;
@@ -691,9 +733,9 @@ decode_splitk_kernel(const DecodeParams p) {
 // Combines the partials of a unit that spans several ranges, and writes
 // o = 0, lse = -inf for a sequence with no visible key; units held whole by
 // one range were written by the main kernel. Grid (head-dim blocks, unit,
-// sequence): each thread owns one (head, d) output element, and the partial
-// loads of a thread are issued four at a time.
+// sequence): each thread owns one (head, d) output element.
 constexpr int kMergeThreads = 256;
+constexpr int kMergeBatch = 8;
 
 template <typename T, int D, int HMAX>
 __global__ void __launch_bounds__(kMergeThreads) merge_kernel(const DecodeParams p) {
@@ -707,8 +749,9 @@ __global__ void __launch_bounds__(kMergeThreads) merge_kernel(const DecodeParams
   const int nh = min(HMAX, p.group - hs * HMAX);
   const int idx = blockIdx.x * kMergeThreads + threadIdx.x;
   const int h = idx / D, d = idx % D;
+  const Lens lens(a);
   long long all, before;
-  visible_sums(a, b, &all, &before);
+  visible_sums(a, lens, b, &all, &before);
   if (h >= nh) return;
   int kbeg;
   const int n = visible(a, b, &kbeg);
@@ -722,28 +765,50 @@ __global__ void __launch_bounds__(kMergeThreads) merge_kernel(const DecodeParams
   const int64_t total = (int64_t)U * all;
   const int64_t per = range_keys(total, p.grid, p.split);
   const int64_t S = (int64_t)U * before + (int64_t)j * n;
-  const int64_t r0 = S / per, r1 = (S + n - 1) / per;
+  const int64_t r0 = udiv(S, per), r1 = udiv(S + n - 1, per);
   if (r0 == r1) return;  // written whole by the range that holds it
   const float* part_o = reinterpret_cast<const float*>(a.workspace);
   const float* part_lse = part_o + p.nslots * HMAX * D;
   // The unit is the last segment of range r0 (slot 1) unless it starts that
   // range (slot 0), and the first segment (slot 0) of every later range.
   const int64_t slot0 = 2 * r0 + (S == r0 * per ? 0 : 1);
-  auto slot = [&](int64_t r) { return r == r0 ? slot0 : 2 * r; };
-  float M = kNegInf;
-#pragma unroll 4
-  for (int64_t r = r0; r <= r1; ++r) M = fmaxf(M, part_lse[slot(r) * HMAX + h]);
-  const float Mu = (M == kNegInf) ? 0.f : M;
-  float wsum = 0.f, o = 0.f;
-#pragma unroll 4
-  for (int64_t r = r0; r <= r1; ++r) {
-    const int64_t sl = slot(r);
-    const float w = __expf(part_lse[sl * HMAX + h] - Mu);
-    wsum += w;
-    o = fmaf(w, part_o[(sl * HMAX + h) * D + d], o);
+  // One pass, kMergeBatch partials' loads in flight: each batch moves the
+  // reference max and brings the sums so far to it. (A pass over the lse values
+  // and then one over both, four at a time, took 8.6 us for units of some 16
+  // partials: a chain of round trips to memory.)
+  float M = kNegInf, wsum = 0.f, o = 0.f;
+  for (int64_t rb = r0; rb <= r1; rb += kMergeBatch) {
+    float ls[kMergeBatch], ov[kMergeBatch];
+#pragma unroll
+    for (int i = 0; i < kMergeBatch; ++i) {
+      const int64_t r = min(rb + i, r1);
+      const int64_t sl = r == r0 ? slot0 : 2 * r;
+      ls[i] = part_lse[sl * HMAX + h];
+      ov[i] = part_o[(sl * HMAX + h) * D + d];
+    }
+    float m = M;
+#pragma unroll
+    for (int i = 0; i < kMergeBatch; ++i) {
+      if (rb + i > r1) {
+        ls[i] = kNegInf;
+        ov[i] = 0.f;
+      }
+      m = fmaxf(m, ls[i]);
+    }
+    const float mu = (m == kNegInf) ? 0.f : m;
+    const float f = __expf(M - mu);
+    wsum *= f;
+    o *= f;
+#pragma unroll
+    for (int i = 0; i < kMergeBatch; ++i) {
+      const float w = __expf(ls[i] - mu);
+      wsum += w;
+      o = fmaf(w, ov[i], o);
+    }
+    M = m;
   }
   orow[d] = (T)(wsum > 0.f ? o / wsum : 0.f);
-  if (lse_out && d == 0) *lse_out = wsum > 0.f ? Mu + logf(wsum) : kNegInf;
+  if (lse_out && d == 0) *lse_out = wsum > 0.f ? M + logf(wsum) : kNegInf;
 }
 
 // Workgroups of `kernel` the device holds at once (cached per device).
@@ -819,75 +884,118 @@ hipError_t launch_t(const DecodeParams& p, hipStream_t s) {
 // elements l + 64 m, so a row's norm is one wave reduction and each RoPE pair
 // (i, i + D/2) sits in one lane (D >= 128) or in lanes l, l ^ 32 (D = 64).
 // The lengths are advanced by a second launch on the same stream, so every
-// workgroup of the first one has read the old positions before they change.
+// workgroup of the first one has read the old positions before they change;
+// kv_append_few_kernel does both where one workgroup holds a sequence's rows.
 // ---------------------------------------------------------------------------
 template <typename T, int D>
-__global__ void __launch_bounds__(256) kv_append_kernel(const goda_kv_append_args a) {
+__device__ __forceinline__ void append_row(const goda_kv_append_args& a, int b, int t, int h, int pos, int lane) {
   constexpr int M = D / 64;  // elements per lane
+  const T* kn = reinterpret_cast<const T*>(a.k_new) + (int64_t)b * a.kn_stride_b + (int64_t)t * a.kn_stride_t + (int64_t)h * a.kn_stride_h;
+  const T* vn = reinterpret_cast<const T*>(a.v_new) + (int64_t)b * a.vn_stride_b + (int64_t)t * a.vn_stride_t + (int64_t)h * a.vn_stride_h;
+  T* kc = reinterpret_cast<T*>(a.k_cache) + (int64_t)b * a.k_stride_b + (int64_t)pos * a.k_stride_t + (int64_t)h * a.k_stride_h;
+  T* vc = reinterpret_cast<T*>(a.v_cache) + (int64_t)b * a.v_stride_b + (int64_t)pos * a.v_stride_t + (int64_t)h * a.v_stride_h;
+  const int rp = (a.rope_pos_abs ? t : pos) + a.rope_k_offset;
+  float x[M];
+  T v[M];
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    x[m] = Elem<T>::to_f32(kn[lane + 64 * m]);
+    v[m] = vn[lane + 64 * m];
+  }
+  if (a.k_norm_weight) {
+    float ss = 0.f;
+#pragma unroll
+    for (int m = 0; m < M; ++m) ss = fmaf(x[m], x[m], ss);
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) ss += shfl_xor_f(ss, o);
+    const float inv = rms_scale(ss, D, a.norm_eps);
+#pragma unroll
+    for (int m = 0; m < M; ++m) x[m] *= inv * (1.f + a.k_norm_weight[lane + 64 * m]);
+  }
+  if (a.rope_k) {
+    if constexpr (M == 1) {
+      // pair (l, l + 32): lanes l < 32 hold x1, lanes l >= 32 hold x2
+      const float other = shfl_xor_f(x[0], 32);
+      const int f = lane & 31;
+      const float c = a.rope_cos[(int64_t)rp * (D / 2) + f], sn = a.rope_sin[(int64_t)rp * (D / 2) + f];
+      x[0] = lane < 32 ? x[0] * c - other * sn : other * sn + x[0] * c;
+    } else {
+#pragma unroll
+      for (int m = 0; m < M / 2; ++m) {
+        const int f = lane + 64 * m;
+        const float c = a.rope_cos[(int64_t)rp * (D / 2) + f], sn = a.rope_sin[(int64_t)rp * (D / 2) + f];
+        const float x1 = x[m], x2 = x[m + M / 2];
+        x[m] = x1 * c - x2 * sn;
+        x[m + M / 2] = x1 * sn + x2 * c;
+      }
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    kc[lane + 64 * m] = Elem<T>::from_f32(x[m]);
+    vc[lane + 64 * m] = v[m];
+  }
+}
+
+template <typename T, int D>
+__global__ void __launch_bounds__(256) kv_append_kernel(const goda_kv_append_args a) {
   const int t = blockIdx.x;
   const int b = blockIdx.y;
   const int pos = a.cache_seqlens[b] + t;
   if (pos < 0 || pos >= a.max_seqlen) return;
-  const int lane = threadIdx.x & 63;
-  const T* kn = reinterpret_cast<const T*>(a.k_new) + (int64_t)b * a.kn_stride_b + (int64_t)t * a.kn_stride_t;
-  const T* vn = reinterpret_cast<const T*>(a.v_new) + (int64_t)b * a.vn_stride_b + (int64_t)t * a.vn_stride_t;
-  T* kc = reinterpret_cast<T*>(a.k_cache) + (int64_t)b * a.k_stride_b + (int64_t)pos * a.k_stride_t;
-  T* vc = reinterpret_cast<T*>(a.v_cache) + (int64_t)b * a.v_stride_b + (int64_t)pos * a.v_stride_t;
-  const int rp = (a.rope_pos_abs ? t : pos) + a.rope_k_offset;
-  for (int h = threadIdx.x >> 6; h < a.heads_kv; h += 4) {
-    float x[M];
-#pragma unroll
-    for (int m = 0; m < M; ++m) x[m] = Elem<T>::to_f32(kn[(int64_t)h * a.kn_stride_h + lane + 64 * m]);
-    if (a.k_norm_weight) {
-      float ss = 0.f;
-#pragma unroll
-      for (int m = 0; m < M; ++m) ss = fmaf(x[m], x[m], ss);
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) ss += shfl_xor_f(ss, o);
-      const float inv = rms_scale(ss, D, a.norm_eps);
-#pragma unroll
-      for (int m = 0; m < M; ++m) x[m] *= inv * (1.f + a.k_norm_weight[lane + 64 * m]);
-    }
-    if (a.rope_k) {
-      if constexpr (M == 1) {
-        // pair (l, l + 32): lanes l < 32 hold x1, lanes l >= 32 hold x2
-        const float other = shfl_xor_f(x[0], 32);
-        const int f = lane & 31;
-        const float c = a.rope_cos[(int64_t)rp * (D / 2) + f], sn = a.rope_sin[(int64_t)rp * (D / 2) + f];
-        x[0] = lane < 32 ? x[0] * c - other * sn : other * sn + x[0] * c;
-      } else {
-#pragma unroll
-        for (int m = 0; m < M / 2; ++m) {
-          const int f = lane + 64 * m;
-          const float c = a.rope_cos[(int64_t)rp * (D / 2) + f], sn = a.rope_sin[(int64_t)rp * (D / 2) + f];
-          const float x1 = x[m], x2 = x[m + M / 2];
-          x[m] = x1 * c - x2 * sn;
-          x[m + M / 2] = x1 * sn + x2 * c;
-        }
-      }
-    }
-#pragma unroll
-    for (int m = 0; m < M; ++m) {
-      kc[(int64_t)h * a.k_stride_h + lane + 64 * m] = Elem<T>::from_f32(x[m]);
-      vc[(int64_t)h * a.v_stride_h + lane + 64 * m] = vn[(int64_t)h * a.vn_stride_h + lane + 64 * m];
-    }
-  }
+  for (int h = threadIdx.x >> 6; h < a.heads_kv; h += 4) append_row<T, D>(a, b, t, h, pos, threadIdx.x & 63);
 }
 
-// Advances the lengths by `add`, clamped to [0, lmax]: a sequence that would
-// pass the end keeps the rows that fit (kv_append_kernel drops the others),
-// and the overflow is reported through `status` instead of being silent.
+// Length `len` plus `add`, clamped to [0, lmax] (a sequence that would pass the
+// end keeps the rows that fit); the overflow is reported through `status`.
+__device__ __forceinline__ void bump(int32_t* len, int add, int lmax, int32_t* status) {
+  const int64_t to = (int64_t)*len + add;
+  *len = (int32_t)(to > lmax ? lmax : to < 0 ? 0 : to);
+  if ((to > lmax || to < 0) && status) *status = 1;
+}
+
+// A few rows (a generation step's token): one workgroup writes all rows of a
+// sequence, a wave per (row, head), and then advances its length, in one launch.
+constexpr int kFewRows = 64;  // (row, head) pairs of a sequence: four rounds of the 16 waves
+template <typename T, int D>
+__global__ void __launch_bounds__(1024) kv_append_few_kernel(const goda_kv_append_args a) {
+  const int b = blockIdx.x;
+  const int pos = a.cache_seqlens[b];
+  for (int i = threadIdx.x >> 6; i < a.seqlen_new * a.heads_kv; i += blockDim.x >> 6) {
+    const int t = i / a.heads_kv;
+    if (pos + t >= 0 && pos + t < a.max_seqlen) append_row<T, D>(a, b, t, i % a.heads_kv, pos + t, threadIdx.x & 63);
+  }
+  __syncthreads();  // every wave has read the old length
+  if (threadIdx.x == 0) bump(a.cache_seqlens + b, a.seqlen_new, a.max_seqlen, a.status);
+}
+
 __global__ void kv_bump_kernel(int32_t* seqlens, int n, int add, int lmax, int32_t* status) {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= n) return;
-  const int64_t len = (int64_t)seqlens[b] + add;
-  const bool bad = len > lmax || len < 0;
-  seqlens[b] = (int32_t)(len > lmax ? lmax : len < 0 ? 0 : len);
-  if (bad && status) *status = 1;
+  if (b < n) bump(seqlens + b, add, lmax, status);
+}
+
+template <typename T>
+hipError_t launch_append_few(const goda_kv_append_args& a, hipStream_t s) {
+  const int waves = std::min(16, a.seqlen_new * a.heads_kv);
+  switch (a.head_dim) {
+    case 64:
+      kv_append_few_kernel<T, 64><<<a.batch, 64 * waves, 0, s>>>(a);
+      break;
+    case 128:
+      kv_append_few_kernel<T, 128><<<a.batch, 64 * waves, 0, s>>>(a);
+      break;
+    case 256:
+      kv_append_few_kernel<T, 256><<<a.batch, 64 * waves, 0, s>>>(a);
+      break;
+    default:
+      return hipErrorNotSupported;
+  }
+  return hipGetLastError();
 }
 
 template <typename T>
 hipError_t launch_append_t(const goda_kv_append_args& a, hipStream_t s) {
+  if (a.seqlen_new > 0 && (int64_t)a.seqlen_new * a.heads_kv <= kFewRows) return launch_append_few<T>(a, s);
   if (a.seqlen_new > 0) {
     const dim3 grid(a.seqlen_new, a.batch);
     switch (a.head_dim) {

@@ -241,3 +241,28 @@ def test_cfg5_two_stream_step_matches_each_part_alone():
     assert torch.equal(pl.result, o_p)
     assert torch.equal(dl.result, o_d)
     report(mix.name, "two-stream step vs parts alone (bit-identical)", 0.0, 0.0)
+
+
+@pytest.mark.parametrize("b,lmax", [(1, 700), (64, 100), (65, 100)])
+@pytest.mark.parametrize("pieces", [1, 7, 8, 9, 17])
+def test_decode_merge_batches(b, lmax, pieces):
+    """Units cut into one partial less, as many and one more than a batch of the
+    merge, with the lengths of up to 64 sequences held in one register or of
+    more in a loop, and a value that one partial makes infinite."""
+    d, hq, hkv = 64, 4, 2
+    n = 64 * pieces - 5
+    rows = max(n, min(lmax, 1200))
+    lens = torch.full((b,), n, dtype=torch.int32)
+    lens[-1] = max(1, n // 3)
+    g = torch.Generator().manual_seed(b + pieces)
+    q = (torch.randn(b, hq, d, generator=g) * 0.5)
+    kc, vc = ((torch.randn(b, rows, hkv, d, generator=g) * 0.5) for _ in range(2))
+    o, lse = ops.attention_decode(q.to(DEV), kc.to(DEV), vc.to(DEV), lens.to(DEV), split_size=64, return_lse=True)
+    o_ref, lse_ref = ref.decode_attention(q, kc, vc, lens)
+    assert (o.cpu() - o_ref).abs().max().item() <= 1e-4 and (lse.cpu() - lse_ref).abs().max().item() <= 1e-4
+    vc[0, n // 2, 0, 3] = float("inf")
+    o2 = ops.attention_decode(q.to(DEV), kc.to(DEV), vc.to(DEV), lens.to(DEV), split_size=64).cpu()
+    hit = torch.zeros_like(o, dtype=torch.bool).cpu()
+    if n // 2 < int(lens[0]):
+        hit[0, : hq // hkv, 3] = True
+    assert torch.equal(torch.isinf(o2), hit) and not torch.isnan(o2).any()

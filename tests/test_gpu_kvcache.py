@@ -227,3 +227,27 @@ def test_chunked_prefill_on_a_cfg4_sized_cache_is_bounded_by_the_visible_prefix(
         qr = ref.apply_rope(q[bi : bi + 1].float(), cos, sin, torch.arange(l0, l0 + tq))
         o_ref, _ = ref.attention_rows(qr, kk, vv, rows, causal=True)
         assert max_err(o[bi : bi + 1, rows], o_ref) <= TOL[torch.bfloat16]
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.float16, 128), (torch.float32, 256)])
+@pytest.mark.parametrize("tn,hkv", [(1, 1), (1, 17), (4, 16), (5, 13), (64, 1), (65, 1)])
+def test_append_of_few_rows_equals_the_general_launch(dtype, d, tn, hkv):
+    """Up to 64 (row, head) pairs a sequence take one launch that also advances
+    the lengths: rows, lengths and overflow report bit for bit those of the same
+    rows appended as the tail of a longer append."""
+    b, lmax = 3, 100
+    g = torch.Generator().manual_seed(tn * hkv)
+    k, v = ((torch.randn(b, 70 + tn, hkv, d, generator=g) * 0.5).to(dtype).to("cuda") for _ in range(2))
+    w = (torch.randn(d, generator=g) * 0.2).to("cuda")
+    cos, sin = (x.to("cuda") for x in wl.rope_tables(lmax + 80, d, 10000.0))
+    start = torch.tensor([0, 17, lmax - 70 - max(1, tn // 2)], dtype=torch.int32, device="cuda").clamp(min=0)
+    outs = []
+    for cuts in ([0, 70, 70 + tn], [0, 70 + tn]):
+        kc, vc = (torch.zeros(b, lmax, hkv, d, dtype=dtype, device="cuda") for _ in range(2))
+        lens, status = start.clone(), torch.zeros(1, dtype=torch.int32, device="cuda")
+        for i, j in zip(cuts, cuts[1:]):
+            ops.kv_append(k[:, i:j], v[:, i:j], kc, vc, lens, rope_cos=cos, rope_sin=sin, rope_k=True, k_norm_weight=w,
+                          status=status)
+        outs.append((kc, vc, lens, status))
+    for x, y in zip(*outs):
+        assert torch.equal(x, y)
