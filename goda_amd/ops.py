@@ -32,8 +32,15 @@ def _ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+# The current stream's handle without the Stream object that
+# torch.cuda.current_stream() builds (about 4 us of a call's host time).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 def _require_gpu(name: str, t: torch.Tensor) -> None:
@@ -59,6 +66,8 @@ def _i32_vec(name: str, t: torch.Tensor | None, n: int, device: torch.device) ->
 def _f32_vec(name: str, t: torch.Tensor | None, n: int, device: torch.device) -> torch.Tensor | None:
     if t is None:
         return None
+    if t.dtype == torch.float32 and t.dim() == 1 and t.shape[0] == n and t.is_contiguous() and t.device == device:
+        return t  # (the usual weight, as it is)
     t = t.detach().reshape(-1)
     if t.numel() != n:
         raise ValueError(f"goda_amd: {name} must have {n} elements")
@@ -138,6 +147,17 @@ def _rope_tables(cos: torch.Tensor | None, sin: torch.Tensor | None, head_dim: i
         return None, None, 0
     if cos is None or sin is None:
         raise ValueError("goda_amd: rope_cos and rope_sin go together")
+    if (
+        cos.dtype == sin.dtype == torch.float32
+        and cos.dim() == 2
+        and cos.shape == sin.shape
+        and cos.shape[1] == head_dim // 2
+        and cos.is_contiguous()
+        and sin.is_contiguous()
+        and cos.device == device
+        and sin.device == device
+    ):
+        return cos, sin, cos.shape[0]  # (the usual tables, as they are)
     cos = cos.reshape(-1, head_dim // 2).to(device=device, dtype=torch.float32).contiguous()
     sin = sin.reshape(-1, head_dim // 2).to(device=device, dtype=torch.float32).contiguous()
     if cos.shape != sin.shape:
@@ -283,9 +303,7 @@ def _prefill_args(
         if k.shape[0] != batch or v.shape != k.shape or k.shape[3] != d:
             raise ValueError(f"goda_amd: k {tuple(k.shape)} / v {tuple(v.shape)} do not match q {tuple(q.shape)}")
         cu_q = cu_k = None
-        qs = (q.stride(0), q.stride(1), q.stride(2))
-        ks = (k.stride(0), k.stride(1), k.stride(2))
-        vs = (v.stride(0), v.stride(1), v.stride(2))
+        qs, ks, vs = q.stride()[:3], k.stride()[:3], v.stride()[:3]
     if hq % hkv != 0:
         raise ValueError(f"goda_amd: heads_q {hq} is not a multiple of heads_kv {hkv}")
     used = _i32_vec("seqused_k", seqused_k, batch, dev)
@@ -509,8 +527,8 @@ def plan_decode(
     b, hq, d = q.shape
     if cache_layout == "bthd":
         _, lmax, hkv, dk = k_cache.shape
-        ks = (k_cache.stride(0), k_cache.stride(1), k_cache.stride(2))
-        vs = (v_cache.stride(0), v_cache.stride(1), v_cache.stride(2))
+        ks = k_cache.stride()[:3]
+        vs = v_cache.stride()[:3]
     elif cache_layout == "bhtd":
         _, hkv, lmax, dk = k_cache.shape
         ks = (k_cache.stride(0), k_cache.stride(2), k_cache.stride(1))
@@ -621,11 +639,11 @@ def kv_append(
     a.batch, a.heads_kv, a.head_dim = b, hkv, d
     a.max_seqlen, a.seqlen_new = k_cache.shape[1], tn
     a.k_new, a.v_new = k_new.data_ptr(), v_new.data_ptr()
-    a.kn_stride_b, a.kn_stride_t, a.kn_stride_h = k_new.stride(0), k_new.stride(1), k_new.stride(2)
-    a.vn_stride_b, a.vn_stride_t, a.vn_stride_h = v_new.stride(0), v_new.stride(1), v_new.stride(2)
+    a.kn_stride_b, a.kn_stride_t, a.kn_stride_h, _ = k_new.stride()
+    a.vn_stride_b, a.vn_stride_t, a.vn_stride_h, _ = v_new.stride()
     a.k_cache, a.v_cache = k_cache.data_ptr(), v_cache.data_ptr()
-    a.k_stride_b, a.k_stride_t, a.k_stride_h = k_cache.stride(0), k_cache.stride(1), k_cache.stride(2)
-    a.v_stride_b, a.v_stride_t, a.v_stride_h = v_cache.stride(0), v_cache.stride(1), v_cache.stride(2)
+    a.k_stride_b, a.k_stride_t, a.k_stride_h, _ = k_cache.stride()
+    a.v_stride_b, a.v_stride_t, a.v_stride_h, _ = v_cache.stride()
     a.cache_seqlens = cache_seqlens.data_ptr()
     a.rope_cos, a.rope_sin, a.rope_len = _ptr(cos), _ptr(sin), rope_len
     a.rope_k, a.rope_k_offset = int(bool(rope_k)), int(rope_k_offset)
