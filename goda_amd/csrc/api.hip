@@ -78,6 +78,8 @@ int32_t check_prefill(const goda_prefill_args* a, bool need_ptrs) {
     if (a->rope_pos_abs == 2) {  // packed row index modulo rope_len: always inside the table
       if (!a->cu_seqlens_q)
         return fail(GODA_ERR_INVALID_ARG, "prefill: rope_pos_abs 2 needs packed rows (cu_seqlens)");
+      if (a->rope_len < 64)
+        return fail(GODA_ERR_INVALID_ARG, "prefill: rope_pos_abs 2 needs tables of at least 64 positions (got %d)", a->rope_len);
     } else if (a->rope_q && (a->rope_q_offset < 0 || qmax >= a->rope_len))
       return fail(GODA_ERR_INVALID_ARG, "prefill: q positions up to %lld exceed rope_len %d",
                   (long long)qmax, a->rope_len);

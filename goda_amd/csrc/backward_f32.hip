@@ -89,12 +89,12 @@ __global__ void __launch_bounds__(256) pack_q_f32_kernel(const BwdParams p) {
   const int i0 = qt * kF32Rows;
   if (i0 >= g.lq) return;
   const bool varlen = a.cu_seqlens_q != nullptr;
-  const int diag = g.lk - g.lq;
   __shared__ __align__(16) float qrows[kF32Rows][D + 4], grows[kF32Rows][D + 4];
   __shared__ float delta[kF32Rows];
   const int tid = threadIdx.x;
   constexpr int TPR = D / 8;
   const int c = (tid % TPR) * 4;
+  const RopePos rope = rope_qrows(a, g, i0);
 #pragma unroll
   for (int r = tid / TPR; r < kF32Rows; r += 256 / TPR) {
     const int i = i0 + r;
@@ -110,7 +110,7 @@ __global__ void __launch_bounds__(256) pack_q_f32_kernel(const BwdParams p) {
       o1 = ld_stream<f32x4>(orow);
       o2 = ld_stream<f32x4>(orow + D / 2);
     }
-    norm_rope_f32<D>(q1, q2, c, a.q_norm_weight, a.norm_eps, i < g.lq && a.rope_q, i < g.lq ? rope_qpos(a, g, i) : 0,
+    norm_rope_f32<D>(q1, q2, c, a.q_norm_weight, a.norm_eps, i < g.lq && a.rope_q, rope.at(r),
                      a.rope_cos, a.rope_sin);
     st_vec<f32x4>(&qrows[r][c], q1);
     st_vec<f32x4>(&qrows[r][c + D / 2], q2);
@@ -152,6 +152,7 @@ __global__ void __launch_bounds__(256) pack_kv_bwd_f32_kernel(const BwdParams p)
   const int tid = threadIdx.x;
   constexpr int TPR = D / 8;
   const int c = (tid % TPR) * 4;
+  const RopePos rope = rope_krows(a, g, kv0);
 #pragma unroll
   for (int r = tid / TPR; r < kF32Rows; r += 256 / TPR) {
     const int row = kv0 + r;
@@ -164,7 +165,7 @@ __global__ void __launch_bounds__(256) pack_kv_bwd_f32_kernel(const BwdParams p)
       v1 = ld_stream<f32x4>(vr);
       v2 = ld_stream<f32x4>(vr + D / 2);
     }
-    norm_rope_f32<D>(k1, k2, c, a.k_norm_weight, a.norm_eps, row < g.lk && a.rope_k, rope_kpos(a, g, row), a.rope_cos,
+    norm_rope_f32<D>(k1, k2, c, a.k_norm_weight, a.norm_eps, row < g.lk && a.rope_k, rope.at(r), a.rope_cos,
                      a.rope_sin);
     st_vec<f32x4>(&krows[r][c], k1);
     st_vec<f32x4>(&krows[r][c + D / 2], k2);
@@ -357,6 +358,7 @@ __global__ void __launch_bounds__(kWaves * 64, kWavesPerSimd<D>) bwd_dkv_f32_ker
   SumSmem<D>& sm = *reinterpret_cast<SumSmem<D>*>(smem);
   const int64_t prow = ((int64_t)b * a.seqlen_k + kv0);
   const int64_t rows = (int64_t)a.batch * a.seqlen_k;
+  const RopePos rope = rope_krows(a, g, kv0);
   auto write = [&](bool is_k) {
     constexpr int PAIRS = D / 8;  // 16-byte pieces of half a row
     for (int i = tid; i < kF32Rows * PAIRS; i += kWaves * 64) {
@@ -379,7 +381,7 @@ __global__ void __launch_bounds__(kWaves * 64, kWavesPerSimd<D>) bwd_dkv_f32_ker
       if (is_k) {
         x1 *= a.softmax_scale;
         x2 *= a.softmax_scale;
-        const int64_t at = (int64_t)(rope_kpos(a, g, kr)) * (D / 2) + d0;
+        const int64_t at = (int64_t)rope.at(r) * (D / 2) + d0;
         if (a.rope_k && kr < g.lk) rotate_back(x1, x2, a.rope_cos + at, a.rope_sin + at);
         out = row_of(p.g.dk, p.g.dk_stride_b, p.g.dk_stride_t, p.g.dk_stride_h, varlen, b, g.k_row0 + kr, hk);
       } else {
@@ -424,7 +426,8 @@ __global__ void __launch_bounds__(256) bwd_dkv_reduce_f32_kernel(const BwdParams
   }
   k1 *= a.softmax_scale;
   k2 *= a.softmax_scale;
-  const int64_t at = (int64_t)(rope_kpos(a, g, key)) * (D / 2) + d0;
+  const int key0 = (int)((int64_t)blockIdx.x * 256 / PAIRS);  // of the workgroup
+  const int64_t at = (int64_t)rope_krows(a, g, key0).at(key - key0) * (D / 2) + d0;
   if (a.rope_k && key < g.lk) rotate_back(k1, k2, a.rope_cos + at, a.rope_sin + at);
   float* krow = row_of(p.g.dk, p.g.dk_stride_b, p.g.dk_stride_t, p.g.dk_stride_h, varlen, b, g.k_row0 + key, hk) + d0;
   float* vrow = row_of(p.g.dv, p.g.dv_stride_b, p.g.dv_stride_t, p.g.dv_stride_h, varlen, b, g.k_row0 + key, hk) + d0;
@@ -583,6 +586,7 @@ __global__ void __launch_bounds__(kWaves * 64, (RECOMPUTE && D == 128 ? 1 : kWav
   constexpr int RPS = 64 / PAIRS;  // rows a wave writes at once
   const int rows = kF32Rows / split, w0 = wave - part;
   const int d0 = 4 * (lane % PAIRS);
+  const RopePos rope = rope_qrows(a, g, qr0);
   for (int r = part * rows + lane / PAIRS; r < (part + 1) * rows; r += RPS) {
     if (qr0 + r >= g.lq) break;
     f32x4 x1 = {}, x2 = {};
@@ -593,7 +597,7 @@ __global__ void __launch_bounds__(kWaves * 64, (RECOMPUTE && D == 128 ? 1 : kWav
     x1 *= a.softmax_scale;
     x2 *= a.softmax_scale;
     if (a.rope_q) {
-      const int64_t at = (int64_t)rope_qpos(a, g, qr0 + r) * (D / 2) + d0;
+      const int64_t at = (int64_t)rope.at(r) * (D / 2) + d0;
       rotate_back(x1, x2, a.rope_cos + at, a.rope_sin + at);
     }
     float* out = row_of(p.g.dq, p.g.dq_stride_b, p.g.dq_stride_t, p.g.dq_stride_h, varlen, b, g.q_row0 + qr0 + r, hq) + d0;

@@ -236,11 +236,11 @@ __global__ void __launch_bounds__(256) pack_q_bwd_kernel(const BwdParams p) {
   const int i0 = qt * kQRows;
   if (i0 >= g.lq) return;
   const bool varlen = a.cu_seqlens_q != nullptr;
-  const int diag = g.lk - g.lq;
   __shared__ __align__(16) T qsrows[kQRows][D + 8];  // q * scale * log2(e)
   __shared__ __align__(16) T grows[kQRows][D + 8];
   const int tid = threadIdx.x;
   constexpr int HALF8 = D / 16;
+  const RopePos rope = rope_qrows(a, g, i0);
 
   // normalized, rotated q and dO rows (zero past the sequence); a row's
   // HALF8 threads are consecutive lanes (and the loop is uniform per wave)
@@ -259,7 +259,7 @@ __global__ void __launch_bounds__(256) pack_q_bwd_kernel(const BwdParams p) {
     }
     v8 qs1, qs2;
     norm_rope_row<T, D, HALF8>(q1, q2, c, a.q_norm_weight, a.norm_eps, i < g.lq && a.rope_q,
-                               i < g.lq ? rope_qpos(a, g, i) : 0, a, p.scale_log2, &qs1, &qs2);
+                               rope.at(r), a, p.scale_log2, &qs1, &qs2);
     st_vec<v8>(&qsrows[r][c], qs1);
     st_vec<v8>(&qsrows[r][c + D / 2], qs2);
     st_vec<v8>(&grows[r][c], g1);
@@ -326,6 +326,7 @@ __global__ void __launch_bounds__(256) pack_kv_bwd_kernel(const BwdParams p) {
   __shared__ __align__(16) T vrows[kBKV][D + 8];
   const int tid = threadIdx.x;
   constexpr int HALF8 = D / 16;
+  const RopePos rope = rope_krows(a, g, kv0);
   for (int idx = tid; idx < kBKV * HALF8; idx += 256) {
     const int r = idx / HALF8;
     const int c = (idx % HALF8) * 8;
@@ -339,7 +340,7 @@ __global__ void __launch_bounds__(256) pack_kv_bwd_kernel(const BwdParams p) {
       v1 = ld_stream<v8>(vr + c);
       v2 = ld_stream<v8>(vr + c + D / 2);
     }
-    norm_rope_row<T, D, HALF8>(k1, k2, c, a.k_norm_weight, a.norm_eps, row < g.lk && a.rope_k, rope_kpos(a, g, row),
+    norm_rope_row<T, D, HALF8>(k1, k2, c, a.k_norm_weight, a.norm_eps, row < g.lk && a.rope_k, rope.at(r),
                                a);
     st_vec<v8>(&krows[r][c], k1);
     st_vec<v8>(&krows[r][c + D / 2], k2);
@@ -730,7 +731,7 @@ __global__ void __launch_bounds__(kWavesKv * 64, 1) bwd_dkv_mfma_kernel(const Bw
       st_vec<v4>(row + 32 * md + 8 * gq + 4 * hi, v4{(T)x[4 * gq], (T)x[4 * gq + 1], (T)x[4 * gq + 2], (T)x[4 * gq + 3]});
   };
   const bool rot = a.rope_k && key < g.lk;
-  const int pos = rope_kpos(a, g, key);
+  const int pos = rope_krows(a, g, kw0).at(l32);
   // dk: pairs of head-dim blocks (md, md + MD/2: the rotation's partners),
   // scaled and rotated back. dK^T accumulated against the row-major q image,
   // which holds q * scale * log2(e): dk = scale * (dS^T q) = ln(2) * dK^T.
@@ -1024,7 +1025,7 @@ __global__ void __launch_bounds__(kWavesWide * 64, 1) bwd_dkv_wide_kernel(const 
       st_vec<v4>(row + 32 * md + 8 * gq + 4 * hi, v4{(T)x[4 * gq], (T)x[4 * gq + 1], (T)x[4 * gq + 2], (T)x[4 * gq + 3]});
   };
   const bool rot = a.rope_k && key < g.lk;
-  const int pos = rope_kpos(a, g, key);
+  const int pos = rope_krows(a, g, kw0).at(l32);
   // dk: one pair of head-dim blocks (md, md + MD/2: the rotation's partners)
   // at a time, scaled and rotated back.
   const float dks = kLn2;
@@ -1077,7 +1078,8 @@ __global__ void __launch_bounds__(256) bwd_dkv_reduce_kernel(const BwdParams p) 
   k1 *= kLn2;
   k2 *= kLn2;
   if (a.rope_k && key < g.lk) {
-    const int pos = rope_kpos(a, g, key);
+    const int key0 = (int)((int64_t)blockIdx.x * 256 / G);  // of the workgroup
+    const int pos = rope_krows(a, g, key0).at(key - key0);
     const f32x4 cs = ld_vec<f32x4>(a.rope_cos + (int64_t)pos * (D / 2) + d0);
     const f32x4 sn = ld_vec<f32x4>(a.rope_sin + (int64_t)pos * (D / 2) + d0);
     const f32x4 y1 = k1 * cs + k2 * sn;
@@ -1314,7 +1316,7 @@ __global__ void __launch_bounds__((DqShape<D>::WAVES * 64), (DqShape<D>::OCC)) b
 #pragma unroll
   for (int md = 0; md < MD; ++md) dq[md] *= a.softmax_scale;
   if (a.rope_q) {
-    const int pos = rope_qpos(a, g, i);
+    const int pos = rope_qrows(a, g, wrow0).at(l32);
 #pragma unroll
     for (int md = 0; md < MD / 2; ++md)
 #pragma unroll
@@ -1486,7 +1488,7 @@ __global__ void __launch_bounds__(kWavesDqS * 64, 1) bwd_dq_ds_kernel(const BwdP
   // 32 md + 8 (r/4) + 4 hi + r%4.
   const int i = wrow0 + l32;
   if (i >= g.lq) return;
-  const int pos = a.rope_q ? rope_qpos(a, g, i) : 0;
+  const int pos = rope_qrows(a, g, wrow0).at(l32);
 #pragma unroll
   for (int h = 0; h < HW; ++h) {
 #pragma unroll

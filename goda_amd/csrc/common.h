@@ -180,18 +180,33 @@ __device__ __forceinline__ SeqGeom seq_geom(int b, int seqlen_q, int seqlen_k,
   return g;
 }
 
-// RoPE position of query row i (0-based within its sequence; diag = Lk - Lq):
-// rope_q_offset + diag + i, or rope_q_offset + i with rope_pos_abs 1 (a
-// caller-given start position), clamped into the table the host validated; with
-// rope_pos_abs 2 the packed row index modulo rope_len (its position in the
-// row of documents it was packed from). Key row j likewise.
-__device__ __forceinline__ int rope_qpos(const goda_prefill_args& a, const SeqGeom& g, int i) {
-  if (a.rope_pos_abs == 2) return (int)((uint32_t)(g.q_row0 + i) % (uint32_t)a.rope_len);
-  return min(max(a.rope_q_offset + (a.rope_pos_abs ? 0 : g.lk - g.lq) + i, 0), a.rope_len - 1);
+// RoPE positions of the query or key rows r0 + l, l < 64 (r0 wave-uniform,
+// 0-based within the sequence; diag = Lk - Lq): rope_q_offset + diag + row, or
+// rope_q_offset + row with rope_pos_abs 1 (a caller-given start position), and
+// rope_k_offset + row for keys, clamped into the table the host validated; with
+// rope_pos_abs 2 the packed row index modulo rope_len (its position in the row
+// of documents it was packed from). One division per tile and rope_len >= 64
+// there: a division per row cost the smallest calls 2%.
+struct RopePos {
+  int base, len;
+  bool packed;
+  __device__ __forceinline__ int at(int l) const {
+    const int p = base + l;
+    if (packed) return p >= len ? p - len : p;
+    return min(max(p, 0), len - 1);
+  }
+};
+__device__ __forceinline__ RopePos rope_rows(const goda_prefill_args& a, int64_t seq_row0, int offset, int r0) {
+  // (out of the way of the usual case: smallest calls wait for every line of code)
+  if (__builtin_expect(a.rope_pos_abs != 2 || a.rope_len <= 0, 1)) return RopePos{offset + r0, a.rope_len, false};
+  const uint32_t row = (uint32_t)__builtin_amdgcn_readfirstlane((int)(seq_row0 + r0));
+  return RopePos{(int)(row % (uint32_t)a.rope_len), a.rope_len, true};
 }
-__device__ __forceinline__ int rope_kpos(const goda_prefill_args& a, const SeqGeom& g, int j) {
-  if (a.rope_pos_abs == 2) return (int)((uint32_t)(g.k_row0 + j) % (uint32_t)a.rope_len);
-  return a.rope_k_offset + j;
+__device__ __forceinline__ RopePos rope_qrows(const goda_prefill_args& a, const SeqGeom& g, int r0) {
+  return rope_rows(a, g.q_row0, a.rope_q_offset + (a.rope_pos_abs ? 0 : g.lk - g.lq), r0);
+}
+__device__ __forceinline__ RopePos rope_krows(const goda_prefill_args& a, const SeqGeom& g, int r0) {
+  return rope_rows(a, g.k_row0, a.rope_k_offset, r0);
 }
 
 // Row (b, query head h, query row i) of the bit-packed mask: bit j % 32 of

@@ -60,6 +60,7 @@ __global__ void __launch_bounds__(256) pack_kv_f32_kernel(const PrefillParams p)
   const int tid = threadIdx.x;
   constexpr int TPR = D / 8;  // threads per row: consecutive lanes
   const int c = (tid % TPR) * 4;
+  const RopePos rope = rope_krows(a, g, kv0);
 #pragma unroll
   for (int r = tid / TPR; r < kF32Rows; r += 256 / TPR) {
     const int row = kv0 + r;
@@ -72,7 +73,7 @@ __global__ void __launch_bounds__(256) pack_kv_f32_kernel(const PrefillParams p)
       v1 = ld_stream<f32x4>(vr);
       v2 = ld_stream<f32x4>(vr + D / 2);
     }
-    norm_rope_f32<D>(k1, k2, c, a.k_norm_weight, a.norm_eps, row < g.lk && a.rope_k, rope_kpos(a, g, row), a.rope_cos,
+    norm_rope_f32<D>(k1, k2, c, a.k_norm_weight, a.norm_eps, row < g.lk && a.rope_k, rope.at(r), a.rope_cos,
                      a.rope_sin);
     st_vec<f32x4>(&krows[r][c], k1);
     st_vec<f32x4>(&krows[r][c + D / 2], k2);
@@ -186,7 +187,7 @@ __global__ void __launch_bounds__(kWaves * 64, kWavesPerSimd<D>) prefill_f32_ker
       }
     }
     if (a.rope_q) {
-      const int pos = rope_qpos(a, g, qi);
+      const int pos = rope_qrows(a, g, qr0).at(l32);
 #pragma unroll
       for (int s = 0; s < KS / 2; ++s) {
         const f32x4 cs = ld_vec<f32x4>(a.rope_cos + (int64_t)pos * (D / 2) + 8 * s + 4 * hi);

@@ -90,7 +90,7 @@ prefill_generic_kernel(const PrefillParams p) {
         for (int j = 0; j < 4; ++j) q[4 * gi + j] *= inv * (1.f + a.q_norm_weight[16 * gi + 4 * part + j]);
     }
     if (a.rope_q) {
-      const int pos = rope_qpos(a, g, i);
+      const int pos = rope_qrows(a, g, q0).at(row);
       const float* cs = a.rope_cos + (int64_t)pos * (D / 2);
       const float* sn = a.rope_sin + (int64_t)pos * (D / 2);
 #pragma unroll
@@ -127,6 +127,7 @@ prefill_generic_kernel(const PrefillParams p) {
   float m = kNegInf, l = 0.f;
 
   for (int kv0 = (kv_lo / kKeys) * kKeys; kv0 < kv_hi; kv0 += kKeys) {
+    const RopePos rope = rope_krows(a, g, kv0);
     __syncthreads();
     // Stage K (rotated) and V rows [kv0, kv0+kKeys) as fp32.
     constexpr int HALF4 = D / 8;  // 4-element groups in half a row
@@ -144,7 +145,7 @@ prefill_generic_kernel(const PrefillParams p) {
         load4<T>(vrow + c4, v1);
         load4<T>(vrow + c4 + D / 2, v2);
         if (a.rope_k && !a.k_norm_weight) {  // with the norm: rotated after it
-          const int pos = rope_kpos(a, g, j);
+          const int pos = rope.at(jr);
           const float* cs = a.rope_cos + (int64_t)pos * (D / 2) + c4;
           const float* sn = a.rope_sin + (int64_t)pos * (D / 2) + c4;
 #pragma unroll
@@ -175,7 +176,7 @@ prefill_generic_kernel(const PrefillParams p) {
       ss += shfl_xor_f(ss, 4);
       const float inv = rms_scale(ss, D, a.norm_eps);
       const int j = kv0 + jr;
-      const int pos = rope_kpos(a, g, j);
+      const int pos = rope.at(jr);
       for (int f = p8; f < D / 2; f += 8) {
         float x1 = Ks[jr][f] * inv * (1.f + a.k_norm_weight[f]);
         float x2 = Ks[jr][f + D / 2] * inv * (1.f + a.k_norm_weight[f + D / 2]);

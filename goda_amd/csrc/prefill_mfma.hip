@@ -190,6 +190,8 @@ __global__ void __launch_bounds__(256) pack_kv_kernel(const PrefillParams p) {
       const float inv = inv_rms[r];
       v8 k1 = ld_vec<v8>(&rows[r][c]);
       v8 k2 = ld_vec<v8>(&rows[r][c + D / 2]);
+  RopePos rope{};
+  if (a.rope_k) rope = rope_krows(a, g, kv0);
       float x1[8], x2[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
@@ -197,7 +199,7 @@ __global__ void __launch_bounds__(256) pack_kv_kernel(const PrefillParams p) {
         x2[e] = (float)k2[e] * inv * (1.f + a.k_norm_weight[c + D / 2 + e]);
       }
       if (a.rope_k && row < g.lk) {
-        const int pos = rope_kpos(a, g, row);
+        const int pos = rope.at(r);
         const float* cs = a.rope_cos + (int64_t)pos * (D / 2) + c;
         const float* sn = a.rope_sin + (int64_t)pos * (D / 2) + c;
 #pragma unroll
@@ -228,7 +230,7 @@ __global__ void __launch_bounds__(256) pack_kv_kernel(const PrefillParams p) {
       k1 = ld_stream<v8>(kr + c);
       k2 = ld_stream<v8>(kr + c + D / 2);
       if (a.rope_k) {
-        const int pos = rope_kpos(a, g, row);
+        const int pos = rope.at(r);
         const float* cs = a.rope_cos + (int64_t)pos * (D / 2) + c;
         const float* sn = a.rope_sin + (int64_t)pos * (D / 2) + c;
         const f32x4 c0 = ld_vec<f32x4>(cs), c1 = ld_vec<f32x4>(cs + 4);
@@ -515,7 +517,7 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
             }
           }
           if (a.rope_q) {
-            const int pos = rope_qpos(a, g, qi);
+            const int pos = rope_qrows(a, g, wrow0 + 32 * nt).at(l32);
 #pragma unroll
             for (int ks = 0; ks < KS / 2; ++ks) {
               const int f0 = 16 * ks + 8 * hi;

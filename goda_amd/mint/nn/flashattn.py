@@ -186,6 +186,8 @@ class FlashAttention(nn.Module):
                 if any(x.shape[0] != t for x in tables):
                     raise ValueError(f"goda_amd FlashAttention: RoPE tables of {rope[0].shape[0]} positions; rows "
                                      f"{start_pos} .. {start_pos + t - 1} are needed")
+                if t < 64:  # (the kernels' least table: the same positions over and over)
+                    tables = [x.repeat(-(-64 // t), 1) for x in tables]
                 kw.update(rope_cos=tables[0], rope_sin=tables[1], rope_q=True, rope_k=True, rope_packed_rows=True)
             cu, max_len, _ = segments
             o = autograd.attention_prefill(

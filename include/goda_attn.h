@@ -115,9 +115,10 @@ typedef struct goda_prefill_args {
                                   0: at rope_q_offset + (Lk - Lq) + i;
                                   2 (packed rows, cu_seqlens): query and key
                                   rows rotate at their packed row index modulo
-                                  rope_len, the offsets unused: documents packed
-                                  from rows of rope_len tokens keep their
-                                  positions in the row */
+                                  rope_len (at least 64), the offsets unused:
+                                  documents packed from rows of rope_len tokens
+                                  keep their positions in the row (shorter rows:
+                                  tables that repeat) */
 
   /* Fused QK-RMSNorm weights, fp32 [head_dim] each, or NULL (no norm on
    * that side; goda's q_norm / k_norm, mint/nn/norm.py:17-27, weight

@@ -270,15 +270,16 @@ def test_kvcache_head_major_storage_decodes_like_contiguous():
 
 
 @pytest.mark.parametrize("dtype,d,tol", [(torch.float32, 64, 1e-4), (torch.bfloat16, 128, 2e-2), (torch.float32, 256, 1e-4)])
-@pytest.mark.parametrize("start_pos", [0, 5])
-def test_flashattention_doc_ids_fused_rope_and_norm(dtype, d, tol, start_pos):
+@pytest.mark.parametrize("start_pos,t", [(0, 70), (5, 70), (3, 41), (0, 300)])
+def test_flashattention_doc_ids_fused_rope_and_norm(dtype, d, tol, start_pos, t):
     """Documents packed from rows: RoPE at the row position (not the document's)
     and the QK-norm before it, inside the kernels, forward and backward, equal
     the same documents attended one row at a time by the dense kernels under
-    the document mask. The gradients' bound adds the storage rounding of the
+    the document mask (rows shorter than the kernels' least table of 64 among
+    them). The gradients' bound adds the storage rounding of the
     largest reference gradient."""
-    t, hq, hkv = 70, 4, 2
-    doc = torch.tensor([[0] * 33 + [1] * 5 + [2] * 32, [7] * 1 + [3] * 69]).to(DEV)
+    hq, hkv = 4, 2
+    doc = torch.tensor([[0] * 33 + [1] * 5 + [2] * (t - 38), [7] * 1 + [3] * (t - 1)]).to(DEV)
     g = torch.Generator().manual_seed(d)
     q, k, v, d_o = ((torch.randn(2, t, h, d, generator=g) * 0.5).to(dtype).to(DEV) for h in (hq, hkv, hkv, hq))
     wq, wk = ((torch.randn(d, generator=g) * 0.2).to(DEV) for _ in range(2))
