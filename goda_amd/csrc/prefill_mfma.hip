@@ -633,17 +633,24 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
       const int nw = (ntl + 31) / 32;
       for (int i = tid; i < nw; i += WAVES * 64) seen[i] = 0;
       __syncthreads();
-#pragma unroll 4
-      for (int t = 0; t < ntl; t += 2) {
-        const int u = t + hi;
-        bool any = false;
-        if (u < ntl) {
+      for (int t0 = 0; t0 < ntl; t0 += 8) {
+        bool any[4];
 #pragma unroll
-          for (int nt = 0; nt < NT; ++nt) any = any || mrow[nt][j_lo + u] != 0;
+        for (int k = 0; k < 4; ++k) {  // (the loads of four pairs in flight)
+          const int u = t0 + 2 * k + hi;
+          any[k] = false;
+          if (u < ntl) {
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) any[k] = any[k] || mrow[nt][j_lo + u] != 0;
+          }
         }
-        const uint64_t m = __builtin_amdgcn_ballot_w64(any);
-        const uint32_t pair = ((uint32_t)m != 0 ? 1u : 0u) | ((uint32_t)(m >> 32) != 0 ? 2u : 0u);
-        if (pair && lane == 0) atomicOr(&seen[t >> 5], pair << (t & 31));
+        uint32_t bits = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const uint64_t m = __builtin_amdgcn_ballot_w64(any[k]);
+          bits |= (((uint32_t)m != 0 ? 1u : 0u) | ((uint32_t)(m >> 32) != 0 ? 2u : 0u)) << (2 * k);
+        }
+        if (bits && lane == 0) atomicOr(&seen[t0 >> 5], bits << (t0 & 31));
       }
       __syncthreads();
       int total = 0;
