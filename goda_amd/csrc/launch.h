@@ -22,6 +22,10 @@ struct PrefillParams {
   int persist_slots;  // persistent grid: resident workgroups per XCD (0: one workgroup per item)
   int persist_pairs;  // persistent grid: (sequence, head slice) pairs per XCD
   int key_split;      // fp32: waves of a workgroup sharing an item's key tiles
+  int ksplit;         // 16-bit, split keys: most pieces of an item, slots an item has
+  int piece_tiles;    // key tiles per piece; 0: from the lengths, on the device
+  int min_piece;
+  float* pieces;      // the pieces' sums, behind the tile images
 };
 
 struct DecodeParams {

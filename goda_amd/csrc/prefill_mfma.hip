@@ -47,6 +47,7 @@
 // operands uses the same (lane half, element) assignment, so the P^T operand
 // is the S^T accumulator re-packed in place.
 
+#include <algorithm>
 #include <mutex>
 
 #include "common.h"
@@ -119,6 +120,38 @@ constexpr bool kPersistent = D <= 128;
 constexpr int kListTiles = 4096;
 constexpr int kListBytes = kListTiles * 2 + kListTiles / 8;
 
+// Split keys (KSPLIT instances): an item's key tiles are cut into pieces that
+// workgroups of their own walk, for dense batches whose items are too few to
+// fill the GPU (see key_pieces). A piece of a cut item leaves its
+// sums in the workspace, and merge_pieces_kernel adds them: rows' O^T as
+// 16-byte quarters of 8 head-dims, [D/4][256 rows] per piece (a wave stores 1 KB
+// runs), then m and l of the 256 rows.
+constexpr int kPieceRows = 256;  // 8 waves of 32 rows
+template <int D>
+constexpr int64_t kPieceBytes = (int64_t)kPieceRows * (D + 2) * 4;
+constexpr int kCus = 256;
+
+// Key tiles per piece for this launch: p.piece_tiles, or (lengths on the
+// device) an equal share of all items' tiles, at least what keeps the longest
+// sequence to p.ksplit pieces.
+__device__ __forceinline__ int piece_tiles(const PrefillParams& p, int bkv) {
+  if (p.piece_tiles > 0) return p.piece_tiles;
+  const goda_prefill_args& a = p.a;
+  const int lane = threadIdx.x & 63;
+  long long tiles = 0;
+  for (int i = lane; i < a.batch; i += 64) tiles += (max(0, min(a.seqused_k[i], a.seqlen_k)) + bkv - 1) / bkv;
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) tiles += __shfl_xor(tiles, o, 64);
+  tiles *= (long long)p.qtiles * a.heads_kv * (p.group / p.heads_per_wg);
+  const int share = (int)min((long long)p.ntiles_k, (tiles + kCus - 1) / kCus);
+  return max(max(share, p.min_piece), (p.ntiles_k + p.ksplit - 1) / p.ksplit);
+}
+// Pieces of an item of n tiles, of equal length; a remainder of at most a
+// quarter piece makes them longer instead of one more.
+__device__ __forceinline__ int piece_count(int n, int per, int most) {
+  return max(1, min(most, (n + per - 1 - per / 4) / per));
+}
+
 // Index of workspace tile j of sequence b, KV head hk.
 __device__ __forceinline__ int64_t ws_tile(int b, int j, int hk, int ntiles, int hkv) {
   return ((int64_t)b * ntiles + j) * hkv + hk;
@@ -157,6 +190,8 @@ __global__ void __launch_bounds__(256) pack_kv_kernel(const PrefillParams p) {
   __shared__ float inv_rms[BKV];
   const int tid = threadIdx.x;
   constexpr int HALF8 = D / 16;  // 8-element chunks per half row
+  RopePos rope{};
+  if (a.rope_k) rope = rope_krows(a, g, kv0);
 
   if (a.k_norm_weight) {
     // Fused QK-RMSNorm: raw rows staged first, then each row's scale, then
@@ -190,8 +225,6 @@ __global__ void __launch_bounds__(256) pack_kv_kernel(const PrefillParams p) {
       const float inv = inv_rms[r];
       v8 k1 = ld_vec<v8>(&rows[r][c]);
       v8 k2 = ld_vec<v8>(&rows[r][c + D / 2]);
-  RopePos rope{};
-  if (a.rope_k) rope = rope_krows(a, g, kv0);
       float x1[8], x2[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
@@ -435,8 +468,9 @@ __device__ __forceinline__ void grid_item(const PrefillParams& p, const int lin,
 
 // One work item of the attention kernel: query tile qt of (sequence, head
 // slice) pair `pair`.
-template <typename T, int D, int BKV, int NT, int WAVES, bool ALIBI, bool MASK>
-__device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* smem, const int pair, const int qt) {
+template <typename T, int D, int BKV, int NT, int WAVES, bool ALIBI, bool MASK, bool KSPLIT = false>
+__device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* smem, const int pair, const int qt,
+                                        const int piece = 0) {
   typedef typename Vec<T>::v8 v8;
   typedef typename Vec<T>::v4 v4;
   typedef TileGeom<T, D, BKV, WAVES> TG;
@@ -562,6 +596,15 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
   if (use_window) kv_lo = max(0, diag + qr0 - window_left);
   int j_lo = kv_lo / BKV;
   int j_hi = kv_hi > 0 ? (kv_hi + BKV - 1) / BKV : 0;
+  int npieces = 1;
+  if constexpr (KSPLIT) {
+    const int all = max(0, j_hi - j_lo);
+    npieces = __builtin_amdgcn_readfirstlane(piece_count(all, piece_tiles(p, BKV), p.ksplit));
+    if (piece >= npieces) return;
+    const int len = (all + npieces - 1) / npieces;
+    j_lo += piece * len;
+    j_hi = min(j_hi, j_lo + len);
+  }
   // Key tile of step j. With ALiBi the steps walk the tiles from the last
   // down: the bias slope*(key - row) grows along the keys, so the first tile
   // holds (nearly) every row's max and the lazy rescale seldom fires again;
@@ -1050,6 +1093,26 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
   // Chunk c of row r sits at chunk c ^ (r mod CH) of the row, so neither the
   // writes (one row per lane) nor the reads (a row per CH lanes) meet on a
   // few banks.
+  if constexpr (KSPLIT) {
+    if (npieces > 1) {
+      static_assert(NT == 1 && WAVES * 32 == kPieceRows, "a piece is 256 rows");
+      const int64_t slot = ((int64_t)pair * p.qtiles + qt) * p.ksplit + piece;
+      float* po = p.pieces + slot * (kPieceBytes<D> / 4);
+      const int row = wave_u * 32 + l32;
+#pragma unroll
+      for (int md = 0; md < MD; ++md)
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr)
+          st_vec<f32x4>(po + ((8 * md + 2 * rr + hi) * kPieceRows + row) * 4,
+                        f32x4{oacc[md][0][4 * rr], oacc[md][0][4 * rr + 1], oacc[md][0][4 * rr + 2], oacc[md][0][4 * rr + 3]});
+      const float lsum = half_sum((l_run[0][0] + l_run[0][1]) + (l_run[0][2] + l_run[0][3]));
+      if (hi == 0) {
+        po[kPieceRows * D + row] = m_run[0];
+        po[kPieceRows * (D + 1) + row] = lsum;
+      }
+      return;
+    }
+  }
   constexpr bool kStageO = DMA && NT == 1;
   if constexpr (kStageO) {
     constexpr int DH = D < 128 ? D : 128;  // columns staged at a time
@@ -1195,6 +1258,72 @@ __global__ void __launch_bounds__(WAVES * 64, 1) prefill_fa_kernel(const Prefill
   }
 }
 
+// The pieces' grid: every item's first piece, then every item's second, ...
+// (grid_item's order within each), so that the full pieces come first.
+template <typename T, int D, int BKV, bool ALIBI>
+__global__ void __launch_bounds__(512, 1) prefill_fa_pieces_kernel(const PrefillParams p) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int nblk = gridDim.x / p.ksplit;
+  const int piece = blockIdx.x / nblk;
+  int pair, qt;
+  grid_item(p, blockIdx.x % nblk, nblk, (8 / p.heads_per_wg) * 32, pair, qt);
+  fa_item<T, D, BKV, 1, 8, ALIBI, false, true>(p, smem, pair, qt, piece);
+}
+
+// Adds the pieces of cut items. A workgroup takes 32 rows of an item, a thread
+// one row's D/32 quarters: 8 rows x 8 quarters a wave, so that it reads
+// 128-byte runs and writes 64-byte ones.
+template <typename T, int D, int BKV>
+__global__ void __launch_bounds__(256) merge_pieces_kernel(const PrefillParams p) {
+  typedef typename Vec<T>::v4 v4;
+  const goda_prefill_args& a = p.a;
+  const int qt = blockIdx.x / 8, wave32 = blockIdx.x % 8, pair = blockIdx.y;
+  const int hg = p.heads_per_wg, nslices = p.group / hg;
+  const int qb_rows = (8 / hg) * 32;
+  const int b = pair / (a.heads_kv * nslices), rem = pair % (a.heads_kv * nslices);
+  const int hq = rem / nslices * p.group + rem % nslices * hg + wave32 % hg;
+  const SeqGeom g = seq_geom(b, a.seqlen_q, a.seqlen_k, nullptr, nullptr, a.seqused_k);
+  // the item's pieces, as fa_item counts them
+  const int qr0 = qt * qb_rows;
+  if (qr0 >= g.lq) return;
+  const int diag = g.lk - g.lq;
+  const bool use_window = a.window_left >= 0 && (a.causal || g.lq == 1);
+  int kv_hi = g.lk;
+  if (a.causal) kv_hi = min(kv_hi, diag + min(qr0 + qb_rows, g.lq));
+  const int kv_lo = use_window ? max(0, diag + qr0 - a.window_left) : 0;
+  const int all = max(0, (kv_hi > 0 ? (kv_hi + BKV - 1) / BKV : 0) - kv_lo / BKV);
+  const int n = piece_count(all, piece_tiles(p, BKV), p.ksplit);
+  if (n == 1) return;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int rr = 8 * wave + (lane & 7);  // row of the 32
+  const int row = wave32 * 32 + rr;
+  const int qi = qr0 + wave32 / hg * 32 + rr;
+  const float* po = p.pieces + ((int64_t)pair * p.qtiles + qt) * p.ksplit * (kPieceBytes<D> / 4);
+  constexpr int64_t kStep = kPieceBytes<D> / 4;
+  float M = kNegInf;
+  for (int s = 0; s < n; ++s) M = fmaxf(M, po[s * kStep + kPieceRows * D + row]);
+  const float Mu = (M == kNegInf) ? 0.f : M;
+  float l = 0.f;
+  f32x4 o[D / 32];
+#pragma unroll
+  for (int c = 0; c < D / 32; ++c) o[c] = f32x4{};
+  for (int s = 0; s < n; ++s) {
+    const float* ps = po + s * kStep;
+    const float w = fast_exp2(ps[kPieceRows * D + row] - Mu);
+    l = fmaf(w, ps[kPieceRows * (D + 1) + row], l);
+#pragma unroll
+    for (int c = 0; c < D / 32; ++c) o[c] += w * ld_vec<f32x4>(ps + ((8 * c + (lane >> 3)) * kPieceRows + row) * 4);
+  }
+  if (qi >= g.lq) return;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  T* orow = reinterpret_cast<T*>(a.o) + (int64_t)b * a.o_stride_b + (int64_t)qi * a.o_stride_t + (int64_t)hq * a.o_stride_h;
+#pragma unroll
+  for (int c = 0; c < D / 32; ++c)
+    st_vec<v4>(orow + 4 * (8 * c + (lane >> 3)), v4{(T)(o[c][0] * inv), (T)(o[c][1] * inv), (T)(o[c][2] * inv), (T)(o[c][3] * inv)});
+  if (a.lse && lane < 8)
+    a.lse[(int64_t)b * a.lse_stride_b + (int64_t)hq * a.lse_stride_h + qi] = l > 0.f ? (M + log2f(l)) * kLn2 : kNegInf;
+}
+
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
@@ -1272,6 +1401,69 @@ int gcd_int(int x, int y) {
   return x;
 }
 
+// Whether the keys of a launch's items are cut, and how (PrefillParams fields).
+struct KeyPieces {
+  int ksplit = 1, tiles = 0, min_piece = 0;
+  int64_t items = 0;
+};
+// Cut where few items leave most CUs idle and the
+// longest is well past an equal share of the work: a piece costs a prologue
+// (about 5 tiles' time), and the cut items' sums a second launch and their way
+// through memory (130 KB a piece at head_dim 128). Whole call, us, uncut / cut,
+// bf16, causal (chunks: keys of 1/8 .. all of the cache):
+//   items  32  B=1, 256 rows on 8448 keys, 32/8 D=128     171 /  67
+//   items  16  B=2, 16 rows on 8000 keys, 32/8 D=128      137 /  54
+//   items  64  B=8, 64 rows on 8448 keys, 32/8 D=128      172 / 124
+//   items  96  B=1 T=4096 6/2 D=128                        92 /  66
+//   items 128  B=2 T=4096 4/4 D=128                        95 /  79
+//   items 128  B=1 T=4096 8/2 D=256                       169 / 156
+//   items 128  B=1 T=2048 16/1 D=256                       96 / 105
+//   items 128  B=4, 256 rows on 1024 keys, 32/8 D=128      41 /  44
+//   items 256  B=8, 256 rows on 8448 keys, 32/8 D=128     244 / 257
+//   items 256  B=2 T=2048 16/16 D=64                       48 /  62
+KeyPieces key_pieces(const goda_prefill_args& a) {
+  KeyPieces k;
+  if (a.dtype == GODA_DTYPE_F32 || a.mask_bits || a.cu_seqlens_q || a.seqlen_q <= 0 || a.seqlen_k <= 0 || a.heads_kv <= 0) return k;
+  const int bkv = kv_tile_for(a.head_dim, a.dtype);
+  const int group = a.heads_q / a.heads_kv;
+  const int hg = gcd_int(group, 8);
+  const int rows = 8 / hg * 32;
+  const int nqt = (a.seqlen_q + rows - 1) / rows;
+  const int64_t per_qt = (int64_t)a.batch * a.heads_kv * (group / hg);
+  k.items = per_qt * nqt;
+  // (lengths on the device may all be short: fewer items, so that little is lost)
+  const bool long_keys = a.seqlen_k >= 4096;
+  if (a.seqused_k ? k.items > (long_keys ? 64 : 48) || a.seqlen_k < 2048
+                  : k.items > (a.head_dim == 64 ? 64 : long_keys ? 128 : 96))
+    return k;
+  const int diag = a.seqlen_k - a.seqlen_q;
+  const bool window = a.window_left >= 0 && (a.causal || a.seqlen_q == 1);
+  int64_t total = 0;
+  int longest = 0;
+  for (int qt = 0; qt < nqt; ++qt) {
+    const int64_t q_last = std::min<int64_t>((int64_t)(qt + 1) * rows, a.seqlen_q);
+    const int64_t hi = a.causal ? std::min<int64_t>(a.seqlen_k, diag + q_last) : a.seqlen_k;
+    const int64_t lo = window ? std::max<int64_t>(0, diag + (int64_t)qt * rows - a.window_left) : 0;
+    const int n = (int)std::max<int64_t>(0, (hi + bkv - 1) / bkv - lo / bkv);
+    total += n * per_qt;
+    longest = std::max(longest, n);
+  }
+  k.min_piece = 8;
+  const int share = (int)std::max<int64_t>(k.min_piece, (total + kCus - 1) / kCus);
+  if (longest < (a.seqused_k ? 16 : share + 12)) return k;
+  constexpr int most = 8;  // (bounds the workspace)
+  if (a.seqused_k) {
+    k.ksplit = std::min(most, (longest + k.min_piece - 1) / k.min_piece);
+  } else {
+    k.tiles = std::max(share, (longest + most - 1) / most);
+    k.ksplit = (longest + k.tiles - 1) / k.tiles;
+  }
+  return k;
+}
+int64_t piece_bytes(int d) {
+  return d == 64 ? kPieceBytes<64> : d == 128 ? kPieceBytes<128> : kPieceBytes<256>;
+}
+
 template <typename T, int D, bool ALIBI, bool MASK>
 hipError_t launch_attn(PrefillParams p, hipStream_t s) {
   typedef Config<T, D> C;
@@ -1288,6 +1480,23 @@ hipError_t launch_attn(PrefillParams p, hipStream_t s) {
   const size_t lds = (size_t)kStages * TileGeom<T, D, C::BKV, C::WAVES>::BYTES + (MASK ? kListBytes : 0);
   auto kern = prefill_fa_kernel<T, D, C::BKV, C::NT, C::WAVES, ALIBI, MASK, false>;
   hipError_t e;
+  if constexpr (!MASK && sizeof(T) == 2) {
+    const KeyPieces k = key_pieces(a);
+    if (k.ksplit > 1) {
+      p.ksplit = k.ksplit;
+      p.piece_tiles = k.tiles;
+      p.min_piece = k.min_piece;
+      p.pieces = reinterpret_cast<float*>(reinterpret_cast<unsigned char*>(a.workspace) + image_bytes(a));
+      auto pk = prefill_fa_pieces_kernel<T, D, C::BKV, ALIBI>;
+      if ((e = hipFuncSetAttribute((const void*)pk, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)) != hipSuccess) return e;
+      if ((e = record_timing(a.timing_begin, s)) != hipSuccess) return e;
+      pk<<<dim3((unsigned)(nblk * k.ksplit)), 512, lds, s>>>(p);
+      if ((e = hipGetLastError()) != hipSuccess) return e;
+      merge_pieces_kernel<T, D, C::BKV><<<dim3(8 * nqt, (unsigned)(nblk / nqt)), 256, 0, s>>>(p);
+      if ((e = hipGetLastError()) != hipSuccess) return e;
+      return record_timing(a.timing_end, s);
+    }
+  }
   // Persistent grid (see prefill_fa_kernel): head_dim <= 128, dense batches
   // whose pairs split evenly over the 8 XCDs, more items than resident
   // workgroups.
@@ -1359,7 +1568,10 @@ bool prefill_mfma_supported(const goda_prefill_args& a) {
   return a.head_dim == 64 || a.head_dim == 128 || a.head_dim == 256;
 }
 
-int64_t prefill_mfma_workspace_bytes(const goda_prefill_args& a) { return image_bytes(a); }
+int64_t prefill_mfma_workspace_bytes(const goda_prefill_args& a) {
+  const KeyPieces k = key_pieces(a);
+  return image_bytes(a) + (k.ksplit > 1 ? k.items * k.ksplit * piece_bytes(a.head_dim) : 0);
+}
 
 hipError_t launch_prefill_mfma(const PrefillParams& p, hipStream_t s) {
   if (p.a.dtype == GODA_DTYPE_BF16) return launch_t<bf16>(p, s);

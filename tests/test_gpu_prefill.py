@@ -475,3 +475,37 @@ def test_prefill_fp32_wide_without_workspace(tk):
     torch.cuda.synchronize()
     assert (_lib.load().goda_attn_prefill_workspace_size(ctypes.byref(plan.args)) > 0) == (tk > 64)
     assert max_err(got, want) <= 1e-5
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.bfloat16, 128), (torch.float16, 256)])
+@pytest.mark.parametrize("b,tq,tk,hq,hkv,causal,window,alibi", [
+    (1, 1500, 1500, 4, 2, True, -1, False),  # few items of unequal length
+    (2, 70, 2100, 8, 2, True, -1, True),  # a chunk behind a prefix, ALiBi's downward walk
+    (1, 1, 3000, 2, 1, True, 1700, False),  # one row, a window over several pieces
+    (1, 40, 1337, 3, 1, False, -1, False),
+    (1, 300, 1100, 6, 6, True, 40, False),  # windowed: too short to cut
+])
+def test_prefill_split_keys(dtype, d, b, tq, tk, hq, hkv, causal, window, alibi):
+    """Batches of few items, whose keys are cut into pieces added up by a second
+    launch."""
+    _run_case(b, tq, tk, hq, hkv, d, dtype, causal, seed=tq, window=window, alibi=alibi, rope=not alibi)
+
+
+@pytest.mark.parametrize("dtype,d,hq,hkv", [(torch.bfloat16, 128, 8, 2), (torch.float16, 64, 4, 4), (torch.bfloat16, 256, 8, 1)])
+@pytest.mark.parametrize("lens", [[1500, 3, 700, 0, 1499], [2000], [40, 40, 40], [1025] + [17] * 69])
+def test_prefill_split_keys_lengths_on_the_device(dtype, d, hq, hkv, lens):
+    """Key counts read on the device: sequences cut into several pieces, one, or
+    none, an empty one, and more than 64 of them; rows with no key give 0."""
+    b, tq, tk = len(lens), 33, 2048
+    q, k, v = _rand((b, tq, hq, d), dtype, 1), _rand((b, tk, hkv, d), dtype, 2), _rand((b, tk, hkv, d), dtype, 3)
+    used = torch.tensor(lens, dtype=torch.int32)
+    o, lse = ops.attention_prefill(q.to(DEV), k.to(DEV), v.to(DEV), causal=True, seqused_k=used.to(DEV), return_lse=True)
+    for i, n in enumerate(lens):
+        first = max(0, tq - n)  # bottom-right: these rows see no key
+        assert torch.count_nonzero(o[i, :first]) == 0 and bool(torch.isneginf(lse[i, :, :first]).all())
+        if n == 0:
+            continue
+        rows = torch.arange(first, tq)
+        o_ref, lse_ref = ref.attention_rows(q[i : i + 1].float(), k[i : i + 1, :n].float(), v[i : i + 1, :n].float(), rows, causal=True)
+        assert max_err(o[i : i + 1, first:], o_ref) <= TOL[dtype]
+        assert lse_err(lse[i : i + 1, :, first:], lse_ref) <= 5e-3
