@@ -610,13 +610,15 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
   // holds (nearly) every row's max and the lazy rescale seldom fires again;
   // in key order the max moved by the slope per key and rescaled often.
   // Stages and loop bounds stay in step order.
-  // With a caller's mask (and a tile list, below) step j is entry j of the list.
+  // With a caller's mask (and a tile list, below) step j is entry j of the list,
+  // whose tiles count from list_base.
   const uint16_t* tile_list = nullptr;
+  int list_base = 0;
   int j_rev = j_lo + j_hi - 1;
   auto tile_of = [&](int j) {
     const int i = ALIBI ? j_rev - j : j;
     if constexpr (MASK)
-      if (tile_list) return __builtin_amdgcn_readfirstlane((int)tile_list[i]);
+      if (tile_list) return list_base + __builtin_amdgcn_readfirstlane((int)tile_list[i]);
     return i;
   };
 
@@ -702,12 +704,13 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
         if ((w >> (t & 31)) & 1u) {
           int at = __popc(w & ((1u << (t & 31)) - 1u));
           for (int i = 0; i < (t >> 5); ++i) at += __popc(seen[i]);
-          list[at] = (uint16_t)(j_lo + t);
+          list[at] = (uint16_t)t;
         }
       }
       for (int i = 0; i < nw; ++i) total += __popc(seen[i]);
       __syncthreads();
       tile_list = list;
+      list_base = j_lo;
       j_lo = 0;
       j_hi = __builtin_amdgcn_readfirstlane(total);
       j_rev = j_hi - 1;

@@ -237,3 +237,18 @@ def test_mask_over_more_tiles_than_the_list_holds():
     keep = m[0, 0, 0]
     o_ref = ops.attention_prefill(q, k[:, keep].contiguous(), v[:, keep].contiguous(), causal=False)
     assert max_err(o, o_ref) <= TOL[torch.bfloat16]
+
+
+def test_mask_and_window_at_the_end_of_a_long_cache():
+    """One row whose window lies past 65536 key tiles of 32 keys."""
+    tk, d, window = 32 * 65536 + 1000, 256, 300
+    k, v = (torch.zeros(1, tk, 1, d, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    q = _rand((1, 1, 2, d), torch.bfloat16, 1).to(DEV)
+    n = window + 1
+    k[:, -n:], v[:, -n:] = _rand((1, n, 1, d), torch.bfloat16, 2).to(DEV), _rand((1, n, 1, d), torch.bfloat16, 3).to(DEV)
+    m = torch.ones(1, 1, 1, tk, dtype=torch.bool, device=DEV)
+    m[..., -200:-100] = False
+    o = ops.attention_prefill(q, k, v, causal=True, window_left=window, attn_mask=m)
+    o_ref, _ = ref.attention_rows(q.cpu().float(), k[:, -n:].cpu().float(), v[:, -n:].cpu().float(), torch.arange(1), causal=True,
+                                  base_attn_mask=m[..., -n:].cpu())
+    assert max_err(o, o_ref) <= TOL[torch.bfloat16]
