@@ -183,15 +183,16 @@ int32_t goda_attn_prefill_fwd(const goda_prefill_args* a, void* stream) {
   if (a->batch == 0 || a->seqlen_q == 0) return ok();
   goda::PrefillParams p = make_prefill_params(a);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const int64_t need = prefill_workspace_bytes(*a);
+  const bool streams = goda::prefill_f32_streams(*a), mfma = goda::prefill_mfma_supported(*a);
+  const int64_t need = mfma && !streams ? goda::prefill_mfma_least_bytes(*a) : prefill_workspace_bytes(*a);
   if (need > 0 && (!a->workspace || a->workspace_bytes < need)) {
     // (fp32 at head_dim 256 also runs without a workspace, on the vector ALUs)
-    if (!goda::prefill_mfma_supported(*a)) return hip_status(goda::launch_prefill_generic(p, s), "prefill_fwd");
+    if (!mfma) return hip_status(goda::launch_prefill_generic(p, s), "prefill_fwd");
     return fail(GODA_ERR_WORKSPACE, "prefill: workspace of %lld bytes needed, %lld given",
                 (long long)need, (long long)a->workspace_bytes);
   }
-  if (goda::prefill_f32_streams(*a)) return hip_status(goda::launch_prefill_f32(p, s), "prefill_fwd");
-  if (goda::prefill_mfma_supported(*a)) return hip_status(goda::launch_prefill_mfma(p, s), "prefill_fwd");
+  if (streams) return hip_status(goda::launch_prefill_f32(p, s), "prefill_fwd");
+  if (mfma) return hip_status(goda::launch_prefill_mfma(p, s), "prefill_fwd");
   return hip_status(goda::launch_prefill_generic(p, s), "prefill_fwd");
 }
 

@@ -108,6 +108,9 @@ hipError_t launch_prefill_generic(const PrefillParams& p, hipStream_t s);
 // hipErrorNotSupported when no tuned instance covers the arguments.
 bool prefill_mfma_supported(const goda_prefill_args& a);
 int64_t prefill_mfma_workspace_bytes(const goda_prefill_args& a);
+// What it runs with at the least: the K/V tile images, without the room for the
+// sums of items whose keys are cut (then none are).
+int64_t prefill_mfma_least_bytes(const goda_prefill_args& a);
 hipError_t launch_prefill_mfma(const PrefillParams& p, hipStream_t s);
 
 // fp32 prefill on the matrix cores with operands streamed from L2: head_dim

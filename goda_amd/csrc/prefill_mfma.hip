@@ -1485,7 +1485,8 @@ hipError_t launch_attn(PrefillParams p, hipStream_t s) {
   hipError_t e;
   if constexpr (!MASK && sizeof(T) == 2) {
     const KeyPieces k = key_pieces(a);
-    if (k.ksplit > 1) {
+    // (a workspace that holds the tile images alone is enough for uncut items)
+    if (k.ksplit > 1 && a.workspace_bytes >= prefill_mfma_workspace_bytes(a)) {
       p.ksplit = k.ksplit;
       p.piece_tiles = k.tiles;
       p.min_piece = k.min_piece;
@@ -1570,6 +1571,8 @@ bool prefill_mfma_supported(const goda_prefill_args& a) {
   if (a.dtype != GODA_DTYPE_BF16 && a.dtype != GODA_DTYPE_F16) return false;
   return a.head_dim == 64 || a.head_dim == 128 || a.head_dim == 256;
 }
+
+int64_t prefill_mfma_least_bytes(const goda_prefill_args& a) { return image_bytes(a); }
 
 int64_t prefill_mfma_workspace_bytes(const goda_prefill_args& a) {
   const KeyPieces k = key_pieces(a);

@@ -509,3 +509,23 @@ def test_prefill_split_keys_lengths_on_the_device(dtype, d, hq, hkv, lens):
         o_ref, lse_ref = ref.attention_rows(q[i : i + 1].float(), k[i : i + 1, :n].float(), v[i : i + 1, :n].float(), rows, causal=True)
         assert max_err(o[i : i + 1, first:], o_ref) <= TOL[dtype]
         assert lse_err(lse[i : i + 1, :, first:], lse_ref) <= 5e-3
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_prefill_split_keys_with_room_for_the_images_alone(d):
+    """A workspace without room for the pieces' sums: the items are not cut, and
+    the call gives the same result. One that is too small for the tile images
+    stays refused."""
+    q, k, v = (_rand((1, t, h, d), torch.bfloat16, s).to(DEV) for t, h, s in ((40, 8, 1), (4096, 2, 2), (4096, 2, 3)))
+    plan = ops.plan_prefill(q, k, v, causal=True)
+    want = plan().clone()
+    images = 2 * 4096 * 2 * d * 2
+    assert plan.args.workspace_bytes > images  # (cut)
+    plan.args.workspace_bytes = images
+    plan.result.zero_()
+    got = plan()
+    torch.cuda.synchronize()
+    assert max_err(got, want) <= TOL[torch.bfloat16]
+    plan.args.workspace_bytes = images - 1
+    with pytest.raises(Exception, match="workspace"):
+        plan()
