@@ -101,6 +101,17 @@ constexpr int kVarlenXcdGroup = 8;
 // (the more sequences interleave, the more of their K/V tiles miss L2; a
 // schedule simulation without that cost gave 539 -> 521 / 505 / 500 / 500).
 constexpr int kPackedTailNum = 1, kPackedTailDen = 4;
+// Packed batches whose longest sequence has at most this many query tiles per
+// XCD: tile qt of the pair at place i of the walk goes to XCD (qt - i) mod 8.
+// With qt mod 8 the first XCDs took nearly all tiles of short sequences (of a
+// batch with one tile each, XCD 0 all). Packed prefill, us, before / now, 4
+// to 48 sequences of 1/16 .. all of the longest, causal:
+//   longest, tiles      1          4          8         16         24        32
+//   16/16 D=64    275 / 191  220 / 169  147 / 129  225 / 206  247 / 248  502 / 458
+//   32/8 D=128    143 / 100  164 / 121  195 / 172  277 / 258  226 / 231  376 / 359
+//   8/1 D=256      34 /  21   42 /  28   47 /  41   77 /  70   85 /  89  120 / 106
+// (24 and 32 tiles turned as well: the tail's order, below, is then lost.)
+constexpr int kRotateTiles = 2;
 // Move each tile in two halves through half the staging registers: register
 // relief for D = 256 (whose two-waves-per-SIMD form is at the limit), and at
 // D = 128 half of the LDS stores move from the end of the interval, where
@@ -382,7 +393,9 @@ __device__ __forceinline__ void grid_item(const PrefillParams& p, const int lin,
     const int per = nqt / kXg;                 // query tiles of one pair on one XCD
     const int pg = npairs / (8 / kXg);         // pairs of one XCD group
     pair = (x / kXg) * pg + s / per;
-    qt = (per - 1 - s % per) * kXg + x % kXg;
+    // Short sequences: turned by the pair's place in the walk (kRotateTiles).
+    const bool rotate = per <= kRotateTiles;
+    qt = (per - 1 - s % per) * kXg + (x + (rotate ? s / per : 0)) % kXg;
     if (a.batch <= 64) {
       // Longest sequences first, so the heaviest tiles are not the last ones
       // dispatched: position `pair` in the walk is served by the sequence of
@@ -403,7 +416,7 @@ __device__ __forceinline__ void grid_item(const PrefillParams& p, const int lin,
       // the next level down.
       // Level i of XCD x is query tile (per - 1 - i) * 8 + x; sequence r has
       // n_r = ceil((nq_r - x) / 8) tiles there, its levels per - n_r .. per - 1.
-      const int r0 = a.batch - (a.batch * kPackedTailNum) / kPackedTailDen;
+      const int r0 = rotate ? a.batch : a.batch - (a.batch * kPackedTailNum) / kPackedTailDen;
       const int s0 = r0 * per_seq * per;  // the tail's first slot on this XCD
       if (s < s0 || r0 >= a.batch) {
         const int r = pair / per_seq;
