@@ -386,16 +386,16 @@ __device__ __forceinline__ void grid_item(const PrefillParams& p, const int lin,
   // group, pair after pair, heaviest tile first: every XCD stays within ~3%
   // of the mean, and the XCDs work on the same pair at the same time, so each
   // XCD's L2 still serves one pair's K/V stream to all its workgroups.
-  constexpr int kXg = kVarlenXcdGroup;  // XCDs sharing one pair's query tiles
+  // XCDs sharing one pair's query tiles: fewer where a pair has fewer (packed_tiles)
+  const int kXg = min(nqt, kVarlenXcdGroup);
   const int npairs = nblk / nqt;
   if (a.cu_seqlens_q && nblk % 8 == 0 && nqt % kXg == 0 && npairs % (8 / kXg) == 0) {
     const int x = lin % 8, s = lin / 8;
     const int per = nqt / kXg;                 // query tiles of one pair on one XCD
-    const int pg = npairs / (8 / kXg);         // pairs of one XCD group
-    pair = (x / kXg) * pg + s / per;
+    pair = s / per * (8 / kXg) + x / kXg;      // place in the walk
     // Short sequences: turned by the pair's place in the walk (kRotateTiles).
     const bool rotate = per <= kRotateTiles;
-    qt = (per - 1 - s % per) * kXg + (x + (rotate ? s / per : 0)) % kXg;
+    qt = (per - 1 - s % per) * kXg + (x + (rotate ? pair : 0)) % kXg;
     if (a.batch <= 64) {
       // Longest sequences first, so the heaviest tiles are not the last ones
       // dispatched: position `pair` in the walk is served by the sequence of
@@ -1480,6 +1480,18 @@ int64_t piece_bytes(int d) {
   return d == 64 ? kPieceBytes<64> : d == 128 ? kPieceBytes<128> : kPieceBytes<256>;
 }
 
+// Query tiles per pair of a packed grid: whole rounds over the 8 XCDs (extra
+// tiles exit at once), or 1, 2 or 4 where the longest sequence has no more and
+// the pairs divide over the XCDs' groups: the extra tiles would be up to seven
+// in eight workgroups, some 4 us each. Packed prefill, 8 tiles / this: longest
+// sequence of 1 tile, 16/16 D=64 191 / 57 us, 32/8 D=128 100 / 30; of 4 tiles
+// 170 / 144 and 121 / 99 (longer ones: within 1.5%).
+int packed_tiles(int nqt, int64_t pairs) {
+  for (int g = 1; g < 8; g *= 2)
+    if (nqt <= g && pairs % (8 / g) == 0) return g;
+  return (nqt + 7) / 8 * 8;
+}
+
 template <typename T, int D, bool ALIBI, bool MASK>
 hipError_t launch_attn(PrefillParams p, hipStream_t s) {
   typedef Config<T, D> C;
@@ -1488,7 +1500,7 @@ hipError_t launch_attn(PrefillParams p, hipStream_t s) {
   p.heads_per_wg = hg;
   const int qb_rows = (C::WAVES / hg) * 32 * C::NT;
   int nqt = (a.seqlen_q + qb_rows - 1) / qb_rows;
-  if (a.cu_seqlens_q) nqt = (nqt + 7) / 8 * 8;  // whole rounds over the 8 XCDs (extra tiles exit at once)
+  if (a.cu_seqlens_q) nqt = packed_tiles(nqt, (int64_t)a.batch * a.heads_kv * (p.group / hg));
   p.qtiles = nqt;
   const int64_t nblk = (int64_t)nqt * a.batch * a.heads_kv * (p.group / hg);
   if (nblk <= 0) return hipSuccess;
