@@ -92,13 +92,22 @@ def _padded(q, k, v, options: dict) -> torch.Tensor:
     rq, rk = opts.pop("rope_q", False), opts.pop("rope_k", False)
     qo, ko = int(opts.pop("rope_q_offset", 0)), int(opts.pop("rope_k_offset", 0))
     pabs = bool(opts.pop("rope_pos_abs", False))
+    packed = bool(opts.pop("rope_packed_rows", False))
     if (rq or rk) and cos is None:
         raise ValueError("goda_amd: rope_q/rope_k need rope_cos and rope_sin")
     varlen = opts.get("cu_seqlens_q") is not None
+    if (rq or rk) and packed and not varlen:
+        raise ValueError("goda_amd: rope_packed_rows needs packed rows (cu_seqlens)")
     if rq or rk:
         cos = cos.reshape(-1, d // 2).float()
         sin = sin.reshape(-1, d // 2).float()
-        if varlen:
+        if packed:
+            # the packed row index modulo the table length, as in the kernels
+            if rq:
+                q = headdim.rotate(q[None], cos, sin, torch.arange(q.shape[0], device=q.device) % cos.shape[0])[0]
+            if rk:
+                k = headdim.rotate(k[None], cos, sin, torch.arange(k.shape[0], device=k.device) % cos.shape[0])[0]
+        elif varlen:
             cu_q, cu_k = opts["cu_seqlens_q"], opts["cu_seqlens_k"]
             iq = _row_positions(cu_q, q.shape[0])
             jk = _row_positions(cu_k, k.shape[0])

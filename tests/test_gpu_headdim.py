@@ -9,6 +9,7 @@ import math
 import pytest
 import torch
 
+from goda_amd import autograd
 from goda_amd import workloads as wl
 from goda_amd.kernels_ import FlashAttentionGQAKernel, FlashAttentionMQAKernel
 from goda_amd.mint.kvcache import KVCache
@@ -119,3 +120,25 @@ def test_layer_with_head_dim_80_and_fused_norm_options():
     y2.sum().backward()
     torch.cuda.synchronize()
     assert all(torch.isfinite(p.grad).all() for p in layer.parameters())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_packed_row_rope_forward_and_backward(dtype):
+    """rope_packed_rows at head dim 96: documents of two rows of 70 tokens
+    rotate at their position in the row, forward and gradients."""
+    d, row, hq, hkv = 96, 70, 4, 2
+    starts = [0, 33, 70, 140]
+    q, k, v, d_o = (_rand((2 * row, h, d), dtype, s) for s, h in enumerate((hq, hkv, hkv, hq)))
+    cos, sin = wl.rope_tables(row, d, 10000.0)
+    cu = torch.tensor(starts, dtype=torch.int32, device=DEV)
+    x = [y.to(DEV).requires_grad_(True) for y in (q, k, v)]
+    o = autograd.attention_prefill(*x, causal=True, cu_seqlens_q=cu, cu_seqlens_k=cu, max_seqlen_q=70, max_seqlen_k=70,
+                                   rope_cos=cos.to(DEV), rope_sin=sin.to(DEV), rope_q=True, rope_k=True, rope_packed_rows=True)
+    o.backward(d_o.to(DEV))
+    for lo, hi in zip(starts, starts[1:]):
+        pos = torch.arange(lo, hi) % row
+        qs, ks, vs, gs = (y[None, lo:hi].float() for y in (q, k, v, d_o))
+        o_ref = ref.attention(ref.apply_rope(qs, cos, sin, pos), ref.apply_rope(ks, cos, sin, pos), vs, causal=True)
+        assert max_err(o[None, lo:hi].detach(), o_ref) <= TOL[dtype]
+        refs = ref.attention_grads(qs, ks, vs, gs, causal=True, rope=(cos, sin, pos, pos))
+        _check(tuple(y.grad[None, lo:hi] for y in x), refs, dtype, f"packed rows {dtype} {lo}")

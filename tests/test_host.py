@@ -8,7 +8,7 @@ import math
 import pytest
 import torch
 
-from goda_amd import ops
+from goda_amd import autograd, ops
 from goda_amd import workloads as wl
 from goda_amd.mint.kvcache import KVCache
 from goda_amd.mint.nn import FlashAttention, LinearScaledRoPE, RoPE, alibi_slopes
@@ -190,3 +190,29 @@ def test_head_dim_padding_helpers():
     pb = torch.stack([pos, pos + 3])
     r = headdim.rotate(x, cos, sin, pb)
     assert torch.allclose(r[1], ref.apply_rope(x[1:2], cos, sin, pos + 3)[0], atol=1e-6)
+
+
+def test_packed_row_rope_at_a_padded_head_dim(monkeypatch):
+    """rope_packed_rows at a head dim without kernels: q and k rotate at their
+    packed row index modulo the table length (not at the document's position)
+    before the padding, and no RoPE option goes on to the kernels."""
+    seen = {}
+
+    def capture(q, k, v, **kw):
+        seen.update(kw, q=q, k=k)
+        return torch.zeros_like(q)
+
+    monkeypatch.setattr(ops, "attention_prefill", capture)
+    d, n, row = 96, 140, 70
+    g = torch.Generator().manual_seed(5)
+    q, k, v = torch.randn(n, 4, d, generator=g), torch.randn(n, 2, d, generator=g), torch.randn(n, 2, d, generator=g)
+    cos, sin = ref.rope_tables(row, d, 10000.0)
+    cu = torch.tensor([0, 33, 70, 140], dtype=torch.int32)
+    kw = dict(causal=True, rope_cos=cos, rope_sin=sin, rope_q=True, rope_k=True, rope_packed_rows=True)
+    autograd.attention_prefill(q, k, v, cu_seqlens_q=cu, cu_seqlens_k=cu, max_seqlen_q=70, max_seqlen_k=70, **kw)
+    pos = torch.arange(n) % row
+    assert torch.allclose(seen["q"][..., :d], ref.apply_rope(q[None], cos, sin, pos)[0], atol=1e-6)
+    assert torch.allclose(seen["k"][..., :d], ref.apply_rope(k[None], cos, sin, pos)[0], atol=1e-6)
+    assert not any(name.startswith("rope") for name in seen)
+    with pytest.raises(ValueError, match="packed rows"):
+        autograd.attention_prefill(q[None], k[None], v[None], **kw)
