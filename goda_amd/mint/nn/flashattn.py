@@ -171,8 +171,9 @@ class FlashAttention(nn.Module):
                 segments = None  # an id recurs in separate runs of a row: the dense mask below
         if segments is not None:
             kw = _norm_kwargs(qk_norm, q=True, k=True)
-            if not headdim.is_native(d):
-                # norm and RoPE as torch ops, before the zero-padding
+            if not headdim.is_native(d) or _rope_in_torch(rope, t):
+                # norm and RoPE as torch ops, before the packing (and the
+                # zero-padding of a head dim without kernels)
                 if qk_norm is not None:
                     q, k = headdim.rms_norm(q, qk_norm[0], qk_norm[2]), headdim.rms_norm(k, qk_norm[1], qk_norm[2])
                     kw = {}
@@ -288,8 +289,14 @@ def _norm_kwargs(qk_norm, *, q: bool, k: bool) -> dict:
     return kw
 
 
+def _rope_in_torch(rope, t: int) -> bool:
+    """Documents' RoPE that the kernels do not take: tables that receive
+    gradients, and a single position for every row."""
+    return rope is not None and (_needs_grad(*rope) or (t > 1 and any(x.shape[0] == 1 for x in rope)))
+
+
 def _rotate(x: torch.Tensor, rope: tuple[torch.Tensor, torch.Tensor], start_pos: int) -> torch.Tensor:
-    # (documents of a head dim without kernels)
+    # (documents whose RoPE does not run in the kernels)
     t = x.shape[1]
     cos = rope[0][start_pos : start_pos + t][None, :, None, :].to(x.dtype)
     sin = rope[1][start_pos : start_pos + t][None, :, None, :].to(x.dtype)

@@ -216,3 +216,37 @@ def test_packed_row_rope_at_a_padded_head_dim(monkeypatch):
     assert not any(name.startswith("rope") for name in seen)
     with pytest.raises(ValueError, match="packed rows"):
         autograd.attention_prefill(q[None], k[None], v[None], **kw)
+
+
+def test_documents_rope_tables_that_receive_gradients(monkeypatch):
+    """Packed documents under RoPE tables that require grad: the rotation is a
+    torch op (after the QK-norm), so that the tables get their gradients; one
+    position for every row is broadcast; other calls leave both to the kernels."""
+    seen = {}
+
+    def capture(q, k, v, **kw):
+        seen.clear()
+        seen.update(kw)
+        return q
+
+    monkeypatch.setattr(autograd, "attention_prefill", capture)
+    b, t, h, d = 2, 70, 2, 64
+    g = torch.Generator().manual_seed(3)
+    q = torch.randn(b, t, h, d, generator=g)
+    w = torch.randn(d, generator=g) * 0.1
+    docs = (torch.arange(t) // 30).expand(b, t)
+    cos, sin = (x.requires_grad_(True) for x in ref.rope_tables(t, d, 10000.0))
+    fa = FlashAttention()
+    o = fa(q, q, q, causal=True, doc_ids=docs, rope=(cos, sin), qk_norm=(w, w, 1e-6))
+    assert "rope_cos" not in seen and "q_norm_weight" not in seen
+    n = ref.rms_norm(q, w)
+    assert torch.allclose(o, ref.apply_rope(n, cos, sin, torch.arange(t)), atol=1e-5)
+    o.sum().backward()
+    # d/dcos of x1 cos - x2 sin and x1 sin + x2 cos, summed: x1 + x2
+    assert torch.allclose(cos.grad, (n[..., : d // 2] + n[..., d // 2 :]).sum((0, 2)), atol=1e-4)
+    assert sin.grad is not None
+    with torch.no_grad():
+        fa(q, q, q, causal=True, doc_ids=docs, rope=(cos, sin), qk_norm=(w, w, 1e-6))
+        assert seen["rope_packed_rows"] and "q_norm_weight" in seen
+        one = fa(q, q, q, causal=True, doc_ids=docs, rope=(cos[:1], sin[:1]))
+    assert "rope_cos" not in seen and torch.equal(one, q)  # (position 0: the identity)
