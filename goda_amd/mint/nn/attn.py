@@ -6,10 +6,12 @@ ALiBi `pos_embeddings` from `goda_amd.mint.nn.pos` is fused into the
 attention kernels (q and k are rotated while the kernels stage them; ALiBi is
 added to the scores) instead of running as separate elementwise passes, and
 ALiBi is actually applied (the reference asserts it away, mint/nn/attn.py:62).
-Without autograd (generation, evaluation) the QK-RMSNorm (mint/nn/attn.py:57-58)
-is fused too, so q and k reach the kernels straight from the projections;
-under autograd it stays a differentiable torch op. Any other `pos_embeddings`
-module is called as in the reference and must not return a bias.
+The QK-RMSNorm (mint/nn/attn.py:57-58) is fused too, forward and backward, so q
+and k reach the kernels straight from the projections without a call of the
+`q_norm` / `k_norm` modules; under autograd over a KV cache, and for packed
+documents when those modules carry hooks, they are called as differentiable
+torch ops. Any other `pos_embeddings` module is called as in the reference and
+must not return a bias.
 """
 
 from __future__ import annotations
@@ -34,6 +36,11 @@ class RMSNorm(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         return headdim.rms_norm(x, self.scale, self.eps, self.shift)
+
+
+def _hooked(m: nn.Module) -> bool:
+    own = (m._forward_hooks, m._forward_pre_hooks, m._backward_hooks, m._backward_pre_hooks)
+    return any(own) or nn.modules.module._has_any_global_hook()
 
 
 class GroupedQueryAttention(nn.Module):
@@ -78,8 +85,10 @@ class GroupedQueryAttention(nn.Module):
         fusable = isinstance(self.pos_embeddings, (RoPE, ALiBiPositionalBias))
         norms_plain = self.q_norm.shift is None and self.k_norm.shift is None and self.q_norm.eps == self.k_norm.eps
         # The fused norm also trains (the backward returns the weights'
-        # gradients), except over a KV cache.
-        if fusable and norms_plain and (not torch.is_grad_enabled() or kv_cache is None):
+        # gradients), except over a KV cache, and for packed documents where
+        # the norm modules carry hooks, which then have to run.
+        hooked = doc_ids is not None and (_hooked(self.q_norm) or _hooked(self.k_norm))
+        if fusable and norms_plain and (not torch.is_grad_enabled() or (kv_cache is None and not hooked)):
             fused["qk_norm"] = (self.q_norm.scale, self.k_norm.scale, self.q_norm.eps)
         else:
             q = self.q_norm(q)

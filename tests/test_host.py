@@ -11,7 +11,7 @@ import torch
 from goda_amd import autograd, ops
 from goda_amd import workloads as wl
 from goda_amd.mint.kvcache import KVCache
-from goda_amd.mint.nn import FlashAttention, LinearScaledRoPE, RoPE, alibi_slopes
+from goda_amd.mint.nn import FlashAttention, GroupedQueryAttention, LinearScaledRoPE, RoPE, alibi_slopes
 from goda_amd.mint.nn.flashattn import _bool_base_mask, _segments
 from oracle import attention as ref
 
@@ -250,3 +250,28 @@ def test_documents_rope_tables_that_receive_gradients(monkeypatch):
         assert seen["rope_packed_rows"] and "q_norm_weight" in seen
         one = fa(q, q, q, causal=True, doc_ids=docs, rope=(cos[:1], sin[:1]))
     assert "rope_cos" not in seen and torch.equal(one, q)  # (position 0: the identity)
+
+
+def test_documents_call_hooked_norm_modules():
+    """Packed documents under grad: q_norm / k_norm modules that carry hooks are
+    called; without hooks the norm is left to the kernels."""
+    t, d = 12, 64
+    layer = GroupedQueryAttention(2, 1, d, 32, RoPE(seq_len=t, head_dim=d, rope_base_theta=10000), torch.float32)
+    seen = {}
+
+    class Stub(torch.nn.Module):
+        def forward(self, q, k, v, **kw):
+            seen.clear()
+            seen.update(kw)
+            return q
+
+    layer.attention = Stub()
+    x = torch.randn(1, t, 32)
+    docs = torch.zeros(1, t, dtype=torch.long)
+    layer(x, doc_ids=docs)
+    assert "qk_norm" in seen
+    calls = []
+    layer.k_norm.register_forward_hook(lambda *a: calls.append("fwd"))
+    layer.q_norm.register_full_backward_hook(lambda *a: calls.append("bwd"))
+    layer(x, doc_ids=docs).sum().backward()
+    assert "qk_norm" not in seen and sorted(calls) == ["bwd", "fwd"]
