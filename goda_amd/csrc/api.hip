@@ -297,7 +297,8 @@ int32_t goda_attn_pack_mask(const goda_pack_mask_args* a, void* stream) {
     return fail(GODA_ERR_INVALID_ARG, "pack_mask: bad sizes (batch %d, heads %d, rows %d, keys %d, mask_keys %d)", a->batch,
                 a->heads, a->rows, a->keys, a->mask_keys);
   if ((int64_t)a->batch * a->heads * a->rows * a->keys == 0) return ok();
-  if (!a->mask || !a->bits || (reinterpret_cast<uintptr_t>(a->bits) & 7) != 0)
+  // (a mask of no keys is not read: it hides every key)
+  if ((!a->mask && a->mask_keys > 0) || !a->bits || (reinterpret_cast<uintptr_t>(a->bits) & 7) != 0)
     return fail(GODA_ERR_INVALID_ARG, "pack_mask: mask is NULL or bits not an 8-byte aligned pointer");
   return hip_status(goda::launch_pack_mask(*a, reinterpret_cast<hipStream_t>(stream)), "pack_mask");
 }

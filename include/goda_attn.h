@@ -331,7 +331,8 @@ int32_t goda_attn_kv_append(const goda_kv_append_args* args, void* stream);
 /* Bit-packs a boolean mask (one byte a key, any nonzero byte visible) of any
  * byte strides into the words of goda_prefill_args.mask_bits: bits receives
  * [batch][heads][rows][2 * ceil(keys / 64)] contiguous words; key j >= mask_keys
- * is hidden. stride_k 0 with mask_keys = keys broadcasts one byte to every key. */
+ * is hidden (mask_keys 0: every key, and mask may be NULL). stride_k 0 with
+ * mask_keys = keys broadcasts one byte to every key. */
 typedef struct goda_pack_mask_args {
   const void* mask;
   int64_t stride_b, stride_h, stride_q, stride_k; /* bytes */

@@ -205,6 +205,15 @@ def test_pack_mask_kernel_matches_the_cpu_form(shape, form):
     assert torch.equal(full(got), full(want))
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 1, 0), (2, 3, 5, 0), (0,)])
+def test_pack_mask_of_no_keys_hides_every_key(shape):
+    """A mask over an empty prefix of the keys (allow_short_keys)."""
+    m = torch.ones(shape, dtype=torch.bool)
+    packed = ops.pack_mask(m.to(DEV), 2, 3, 5, 70, DEV, allow_short_keys=True)
+    want = ops.pack_mask(m, 2, 3, 5, 70, "cpu", allow_short_keys=True)
+    assert packed.bits.shape == want.bits.shape and torch.count_nonzero(packed.bits) == 0
+
+
 @pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.bfloat16, 128), (torch.float16, 256), (torch.float32, 128)])
 @pytest.mark.parametrize("causal,alibi", [(True, False), (False, False), (False, True)])
 @pytest.mark.parametrize("tk", [64, 65, 330, 2100])
