@@ -17,7 +17,7 @@ from pathlib import Path
 _LIB_ENV = "GODA_ATTN_LIB"
 _DEFAULT = Path(__file__).resolve().parent / "lib" / "libgoda_attn.so"
 
-ABI_VERSION = 5
+ABI_VERSION = 6
 
 DTYPE_F32 = 0
 DTYPE_F16 = 1
@@ -82,6 +82,7 @@ class PrefillArgs(ctypes.Structure):
         ("rope_k_offset", _i32),
         ("norm_eps", _f32),
         ("rope_pos_abs", _i32),
+        ("rope_packed_rows", _i32),
         ("q_norm_weight", _vp),
         ("k_norm_weight", _vp),
         ("mask_bits", _vp),

@@ -75,15 +75,15 @@ int32_t check_prefill(const goda_prefill_args* a, bool need_ptrs) {
     // rope_q_offset + i); k rows at rope_k_offset + j.
     const int64_t qmax = (int64_t)a->rope_q_offset + (a->rope_pos_abs ? a->seqlen_q : a->seqlen_k) - 1;
     const int64_t kmax = (int64_t)a->rope_k_offset + a->seqlen_k - 1;
-    if (a->rope_pos_abs == 2) {  // packed row index modulo rope_len: always inside the table
+    if (a->rope_packed_rows) {  // packed row index modulo rope_len: always inside the table
       if (!a->cu_seqlens_q)
-        return fail(GODA_ERR_INVALID_ARG, "prefill: rope_pos_abs 2 needs packed rows (cu_seqlens)");
+        return fail(GODA_ERR_INVALID_ARG, "prefill: rope_packed_rows needs packed rows (cu_seqlens)");
       if (a->rope_len < 64)
-        return fail(GODA_ERR_INVALID_ARG, "prefill: rope_pos_abs 2 needs tables of at least 64 positions (got %d)", a->rope_len);
+        return fail(GODA_ERR_INVALID_ARG, "prefill: rope_packed_rows needs tables of at least 64 positions (got %d)", a->rope_len);
     } else if (a->rope_q && (a->rope_q_offset < 0 || qmax >= a->rope_len))
       return fail(GODA_ERR_INVALID_ARG, "prefill: q positions up to %lld exceed rope_len %d",
                   (long long)qmax, a->rope_len);
-    if (a->rope_pos_abs != 2 && a->rope_k && (a->rope_k_offset < 0 || kmax >= a->rope_len))
+    if (!a->rope_packed_rows && a->rope_k && (a->rope_k_offset < 0 || kmax >= a->rope_len))
       return fail(GODA_ERR_INVALID_ARG, "prefill: k positions up to %lld exceed rope_len %d",
                   (long long)kmax, a->rope_len);
     if (a->rope_q && !a->rope_pos_abs && !a->cu_seqlens_q && a->seqlen_q > a->seqlen_k && !a->seqused_k)

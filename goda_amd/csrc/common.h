@@ -182,9 +182,9 @@ __device__ __forceinline__ SeqGeom seq_geom(int b, int seqlen_q, int seqlen_k,
 
 // RoPE positions of the query or key rows r0 + l, l < 64 (r0 wave-uniform,
 // 0-based within the sequence; diag = Lk - Lq): rope_q_offset + diag + row, or
-// rope_q_offset + row with rope_pos_abs 1 (a caller-given start position), and
+// rope_q_offset + row with rope_pos_abs (a caller-given start position), and
 // rope_k_offset + row for keys, clamped into the table the host validated; with
-// rope_pos_abs 2 the packed row index modulo rope_len (its position in the row
+// rope_packed_rows the packed row index modulo rope_len (its position in the row
 // of documents it was packed from). One division per tile and rope_len >= 64
 // there: a division per row cost the smallest calls 2%.
 struct RopePos {
@@ -198,7 +198,7 @@ struct RopePos {
 };
 __device__ __forceinline__ RopePos rope_rows(const goda_prefill_args& a, int64_t seq_row0, int offset, int r0) {
   // (out of the way of the usual case: smallest calls wait for every line of code)
-  if (__builtin_expect(a.rope_pos_abs != 2 || a.rope_len <= 0, 1)) return RopePos{offset + r0, a.rope_len, false};
+  if (__builtin_expect(!a.rope_packed_rows || a.rope_len <= 0, 1)) return RopePos{offset + r0, a.rope_len, false};
   const uint32_t row = (uint32_t)__builtin_amdgcn_readfirstlane((int)(seq_row0 + r0));
   return RopePos{(int)(row % (uint32_t)a.rope_len), a.rope_len, true};
 }

@@ -357,7 +357,7 @@ def _prefill_args(
     a.rope_cos, a.rope_sin, a.rope_len = _ptr(cos), _ptr(sin), rope_len
     a.rope_q, a.rope_k = int(bool(rope_q)), int(bool(rope_k))
     a.rope_q_offset, a.rope_k_offset = int(rope_q_offset), int(rope_k_offset)
-    a.rope_pos_abs = 2 if rope_packed_rows else int(bool(rope_pos_abs))
+    a.rope_pos_abs, a.rope_packed_rows = int(bool(rope_pos_abs)), int(bool(rope_packed_rows))
     qn = _f32_vec("q_norm_weight", q_norm_weight, d, dev)
     kn = _f32_vec("k_norm_weight", k_norm_weight, d, dev)
     a.q_norm_weight, a.k_norm_weight, a.norm_eps = _ptr(qn), _ptr(kn), float(norm_eps)

@@ -55,7 +55,7 @@
 extern "C" {
 #endif
 
-#define GODA_ATTN_ABI_VERSION 5
+#define GODA_ATTN_ABI_VERSION 6
 
 /* element types */
 #define GODA_DTYPE_F32 0
@@ -112,13 +112,14 @@ typedef struct goda_prefill_args {
   int32_t rope_pos_abs;        /* 1: query row i rotates at rope_q_offset + i
                                   (a caller-given start position, as goda's
                                   RoPE(q, k, start_pos), mint/nn/pos.py:100-112);
-                                  0: at rope_q_offset + (Lk - Lq) + i;
-                                  2 (packed rows, cu_seqlens): query and key
+                                  0: at rope_q_offset + (Lk - Lq) + i */
+  int32_t rope_packed_rows;    /* 1 (packed rows, cu_seqlens): query and key
                                   rows rotate at their packed row index modulo
-                                  rope_len (at least 64), the offsets unused:
-                                  documents packed from rows of rope_len tokens
-                                  keep their positions in the row (shorter rows:
-                                  tables that repeat) */
+                                  rope_len (at least 64), the offsets and
+                                  rope_pos_abs unused: documents packed from
+                                  rows of rope_len tokens keep their positions
+                                  in the row (shorter rows: tables that
+                                  repeat). ABI 6: what was padding before. */
 
   /* Fused QK-RMSNorm weights, fp32 [head_dim] each, or NULL (no norm on
    * that side; goda's q_norm / k_norm, mint/nn/norm.py:17-27, weight

@@ -102,6 +102,21 @@ def test_prefill_rejects_bad_arguments(lib, over, code, needle):
     assert lib.goda_attn_prefill_fwd(ctypes.byref(a), None) == code
 
 
+def test_rope_position_flags(lib):
+    """Any nonzero rope_pos_abs names the same rule; packed rows have a flag of
+    their own, which needs cu_seqlens and tables of at least 64 positions."""
+    table = ctypes.addressof(ctypes.create_string_buffer(16))  # (sizes only: not read)
+    rope = dict(rope_cos=table, rope_sin=table, rope_len=64, rope_q=1, rope_k=1)
+    size = lambda **kw: lib.goda_attn_prefill_workspace_size(ctypes.byref(_prefill_args(**rope | kw)))  # noqa: E731
+    assert size(rope_pos_abs=1) == size(rope_pos_abs=2) == size(rope_pos_abs=-1) > 0
+    assert size(rope_pos_abs=2, rope_q_offset=1) == _lib.ERR_INVALID_ARG  # past the table
+    assert size(rope_packed_rows=1) == _lib.ERR_INVALID_ARG
+    assert "packed rows" in lib.goda_attn_last_error().decode()
+    cu = dict(cu_seqlens_q=table, cu_seqlens_k=table, rope_packed_rows=1)
+    assert size(**cu, rope_q_offset=1) > 0
+    assert size(**cu, rope_len=63) == _lib.ERR_INVALID_ARG
+
+
 def test_prefill_rejects_null_tensors(lib):
     a = _prefill_args()
     assert lib.goda_attn_prefill_fwd(ctypes.byref(a), None) == _lib.ERR_INVALID_ARG
