@@ -29,9 +29,17 @@ constexpr int kWaves = 4;
 // Chunks in flight (4 registers and 256 clocks of products each, times the
 // waves of a SIMD): 2048 clocks and more cover a load that misses L2.
 constexpr int kRing = 8;
-// Rescale margin in log2 units (see the 16-bit kernel: fp32 accumulators hold
-// rows of 2^20 keys at 2^60).
-constexpr float kRescaleThresh = 60.f;
+// Rescale margin in log2 units: at head_dim 64 and 128 that of the LDS-ring
+// kernel, which larger calls run on (fp32 accumulators hold rows of 2^20 keys at
+// 2^60). At 256 the vector-ALU kernel runs beside this one, whose probabilities
+// are at most 1, so that values up to the type's largest over the number of keys
+// stay finite: here they are at most 2^8 and the v image holds v * 2^-8, which
+// the division by the row sum takes back. (A margin of 0 rescaled at most tiles:
+// 315 -> 333 us at B=1, T=2048, 16/1 heads, causal.)
+template <int D>
+constexpr float kRescaleThresh = D == 256 ? 8.f : 60.f;
+template <int D>
+constexpr float kValueScale = D == 256 ? 1.f / 256.f : 1.f;
 
 template <int D>
 constexpr int kWavesPerSimd = D <= 128 ? 2 : 1;
@@ -44,7 +52,7 @@ __device__ __forceinline__ int64_t kv_tile(int b, int j, int hk, int ntiles, int
 }
 
 // Per (key tile, KV head, sequence): the row image of k (normalized, rotated)
-// and the transposed image of v, rows past the sequence zero.
+// and the transposed image of v (times kValueScale), rows past the sequence zero.
 template <int D>
 __global__ void __launch_bounds__(256) pack_kv_f32_kernel(const PrefillParams p) {
   const goda_prefill_args& a = p.a;
@@ -77,8 +85,8 @@ __global__ void __launch_bounds__(256) pack_kv_f32_kernel(const PrefillParams p)
                      a.rope_sin);
     st_vec<f32x4>(&krows[r][c], k1);
     st_vec<f32x4>(&krows[r][c + D / 2], k2);
-    st_vec<f32x4>(&vrows[r][c], v1);
-    st_vec<f32x4>(&vrows[r][c + D / 2], v2);
+    st_vec<f32x4>(&vrows[r][c], v1 * kValueScale<D>);
+    st_vec<f32x4>(&vrows[r][c + D / 2], v2 * kValueScale<D>);
   }
   __syncthreads();
   unsigned char* tile = reinterpret_cast<unsigned char*>(a.workspace) +
@@ -272,7 +280,7 @@ __global__ void __launch_bounds__(kWaves * 64, kWavesPerSimd<D>) prefill_f32_ker
       const float alpha = (m_run == kNegInf) ? 0.f : fast_exp2(m_run - mn);
       const float shift = (mn == kNegInf) ? 0.f : mn - mq;
       m_run = mn;
-      gthr = (mn == kNegInf) ? kNegInf : kRescaleThresh;
+      gthr = (mn == kNegInf) ? kNegInf : kRescaleThresh<D>;
       l_run *= alpha;
 #pragma unroll
       for (int md = 0; md < MD; ++md) oacc[md] *= alpha;
@@ -307,7 +315,7 @@ __global__ void __launch_bounds__(kWaves * 64, kWavesPerSimd<D>) prefill_f32_ker
   float l = half_sum(l_run);
   if (split == 1) {
     if (!row_ok) return;
-    const float inv = l > 0.f ? 1.f / l : 0.f;
+    const float inv = l > 0.f ? 1.f / (l * kValueScale<D>) : 0.f;
     float* orow = obase + qi * a.o_stride_t;
 #pragma unroll
     for (int md = 0; md < MD; ++md)
@@ -342,7 +350,7 @@ __global__ void __launch_bounds__(kWaves * 64, kWavesPerSimd<D>) prefill_f32_ker
       o += ld_vec<f32x4>(&sm.o[w0 + w][r][4 * (lane % CPR)]);
     }
     if (live && qr0 + r < g.lq) {
-      st_vec<f32x4>(obase + (int64_t)(qr0 + r) * a.o_stride_t + 4 * (lane % CPR), o * (ls > 0.f ? 1.f / ls : 0.f));
+      st_vec<f32x4>(obase + (int64_t)(qr0 + r) * a.o_stride_t + 4 * (lane % CPR), o * (ls > 0.f ? 1.f / (ls * kValueScale<D>) : 0.f));
       if (lse && lane % CPR == 0) {
         float mr = kNegInf;
         for (int w = 0; w < split; ++w) mr = fmaxf(mr, sm.m[w0 + w][r]);

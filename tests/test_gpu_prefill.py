@@ -477,6 +477,23 @@ def test_prefill_fp32_wide_without_workspace(tk):
     assert max_err(got, want) <= 1e-5
 
 
+@pytest.mark.parametrize("tk", [64, 96, 2048])
+def test_prefill_fp32_wide_large_values(tk):
+    """fp32 at head_dim 256: values of 1e30 under scores that grow by up to 40
+    (58 log2 units) along the keys stay finite, whichever kernel runs: no
+    probability passes 1, so that an output is at most the largest value. Two
+    roundings of a score of 58 log2 units change a probability by 2 * 58 * 2^-24
+    * ln 2 = 4.8e-6 of itself, the bound is twice that."""
+    d = 256
+    q, v = torch.zeros(1, 4, 2, d), _rand((1, tk, 2, d), torch.float32, 3) * 1e30
+    k = torch.zeros(1, tk, 2, d)
+    q[..., 0] = 1.0
+    k[..., 0] = torch.linspace(0.0, 40.0, tk)[None, :, None]
+    o = ops.attention_prefill(q.to(DEV), k.to(DEV), v.to(DEV), causal=False, softmax_scale=1.0)
+    want = ref.attention(q.double(), k.double(), v.double(), causal=False, scale=1.0, dtype=torch.float64)
+    assert (o.cpu().double() - want).abs().max().item() <= 1e-5 * v.abs().max().item()
+
+
 @pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.bfloat16, 128), (torch.float16, 256)])
 @pytest.mark.parametrize("b,tq,tk,hq,hkv,causal,window,alibi", [
     (1, 1500, 1500, 4, 2, True, -1, False),  # few items of unequal length
