@@ -41,7 +41,9 @@ bool dtype_ok(int32_t d) { return d == GODA_DTYPE_F32 || d == GODA_DTYPE_F16 || 
 bool head_dim_ok(int32_t d) { return d == 64 || d == 128 || d == 256; }
 
 // Checks shared by prefill; returns GODA_OK or a failure status. The
-// workspace query passes need_ptrs = false: it depends on sizes only.
+// workspace query passes need_ptrs = false: it depends on the sizes and options
+// (of the pointers only on which are set and, in the backward, on whether both
+// cu_seqlens are one array).
 int32_t check_prefill(const goda_prefill_args* a, bool need_ptrs) {
   if (!a) return fail(GODA_ERR_INVALID_ARG, "prefill: args is NULL");
   if (!dtype_ok(a->dtype)) return fail(GODA_ERR_INVALID_ARG, "prefill: unknown dtype %d", a->dtype);
@@ -211,7 +213,7 @@ int32_t goda_attn_prefill_bwd(const goda_prefill_args* a, const goda_prefill_gra
   if (!a->q || !a->k || !a->v || !a->o || !g->d_o || !g->dq || !g->dk || !g->dv)
     return fail(GODA_ERR_INVALID_ARG, "prefill_bwd: NULL tensor pointer");
   if (!a->lse) return fail(GODA_ERR_INVALID_ARG, "prefill_bwd: the forward's lse is required");
-  const int64_t need = goda::prefill_bwd_workspace_bytes(*a);
+  const int64_t need = goda::prefill_bwd_least_bytes(*a);
   if (need > 0 && (!g->workspace || g->workspace_bytes < need))
     return fail(GODA_ERR_WORKSPACE, "prefill_bwd: workspace of %lld bytes needed, %lld given", (long long)need,
                 (long long)g->workspace_bytes);

@@ -18,8 +18,10 @@
 //   4. bwd_dq_f32_kernel: a wave owns 32 query rows of a head (or shares them
 //      with others of its workgroup, which take every split-th key tile):
 //        dQ^T [d][rows] += K^T dS^T         A = k^T image, B = stored dS
-//      Where the dS tiles would pass kDsMaxBytes it forms S and dP again
-//      (RECOMPUTE: three products per tile instead of one).
+//      3 and 4 run in turn for as many (sequence, KV head) pairs as the buffer of
+//      dS tiles holds. Where those of one pair pass kDsMaxBytes, or the workspace
+//      has no room for them, 4 forms S and dP again (RECOMPUTE: three products
+//      per tile instead of one).
 //
 // Bound by the fp32 products (154 TFLOP/s reached by a large matrix product).
 // Whole backward, us, before (LDS rings with one wave per SIMD at head_dim 64
@@ -40,7 +42,18 @@ namespace {
 
 constexpr int kWaves = 4;
 constexpr int kRing = 8;  // chunks in flight, as in the forward
+// dS tiles held at a time: all up to kDsMaxBytes, else as many (sequence, KV
+// head) pairs as kDsChunkBytes hold, or one pair up to kDsMaxBytes. Whole
+// backward, ms, with S and dP formed again / with the tiles of a part at a time:
+//   B=8 T=4096 32/8 D=128 causal   32.6 / 25.3     B=1 T=16384 32/8 D=128   63.1 / 49.1
+//   B=2 T=16384 8/8 D=64 causal    17.6 / 13.6     the same, window 128     1.82 / 1.46
+//   packed 8192 + 16 x 200 rows, 16/4 D=128                                 15.8 / 7.9
+// Every run ends with its longest workgroups: B=1 T=11264 32/8 D=128 23.4 at
+// once, 24.1 in two runs, hence the larger limit for all. (Past both, the dq
+// kernel that forms S and dP again is 3% slower than the LDS-ring kernels that
+// it replaced at head_dim 128 and 9% at 64.)
 constexpr int64_t kDsMaxBytes = 8ll << 30;
+constexpr int64_t kDsChunkBytes = 4ll << 30;
 constexpr int kDsTile = kF32Rows * kF32Rows * 4;
 template <int D>
 constexpr int kWavesPerSimd = D <= 128 ? 2 : 1;
@@ -66,10 +79,16 @@ template <int D>
 __device__ __forceinline__ const unsigned char* k_tile(const BwdParams& p, int b, int kt, int hk) {
   return p.kvimg + (((int64_t)b * p.ntk + kt) * p.a.heads_kv + hk) * KTile<D>::BYTES;
 }
-// dS tile: for key group g and lane half h, row l's keys 8 g + 4 h + e at
-// (64 g + 32 h + l) 16 + 4 e.
-__device__ __forceinline__ unsigned char* ds_tile(const BwdParams& p, int b, int qt, int kt, int hq) {
-  return p.ds + (((int64_t)b * p.ds_per_b + ds_row_off(qt, p.ntk, p.ds_c, p.ds_tri != 0) + kt) * p.a.heads_q + hq) * kDsTile;
+// dS tile of query head h of a pair's group (pair: of this launch; diag = Lk -
+// Lq of the sequence): for key group g and lane half l / 32, row l % 32's keys
+// 8 g + 4 (l / 32) + e at (64 g + l) 16 + 4 e.
+__device__ __forceinline__ unsigned char* ds_tile(const BwdParams& p, int pair, int diag, int qt, int kt, int h) {
+  int64_t at;
+  if (p.ds_band > 0)
+    at = (int64_t)qt * p.ds_band + kt - max(0, diag + qt * kF32Rows - p.a.window_left) / kF32Rows;
+  else
+    at = ds_row_off(qt, p.ntk, p.ds_c, p.ds_tri != 0) + kt;
+  return p.ds + ((pair * p.ds_per_pair + at) * p.group + h) * kDsTile;
 }
 
 __device__ __forceinline__ const float* row_of(const void* base, int64_t sb, int64_t st, int64_t sh, bool varlen, int b,
@@ -209,17 +228,12 @@ __global__ void __launch_bounds__(kWaves * 64, kWavesPerSimd<D>) bwd_dkv_f32_ker
   static_assert(2 * KS % kRing == 0, "a ring slot is a compile-time constant of the chunk");
   extern __shared__ __align__(16) unsigned char smem[];
   const goda_prefill_args& a = p.a;
-  // Workgroup order of backward_mfma.hip: units (KV head, share of the walk,
-  // sequence) in chunks, the key tile most rows see first.
-  int kt, by, b;
-  {
-    const int lin = (int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
-    int unit;
-    chunked_order(lin, (int)gridDim.x, (int)(gridDim.y * gridDim.z), unit, kt);
-    by = unit % (int)gridDim.y;
-    b = unit / (int)gridDim.y;
-  }
-  const int hk = by / p.nsplit, split = by % p.nsplit;
+  // Workgroup order of backward_mfma.hip: units (sequence, KV head, share of the
+  // walk) in chunks, the key tile most rows see first.
+  int unit, kt;
+  chunked_order((int)blockIdx.x, p.ntk, p.npairs * p.nsplit, unit, kt);
+  const int pair = unit / p.nsplit, split = unit % p.nsplit;  // (pair: of this launch)
+  const int b = (p.pair0 + pair) / a.heads_kv, hk = (p.pair0 + pair) % a.heads_kv;
   const SeqGeom g = seq_geom(b, a.seqlen_q, a.seqlen_k, a.cu_seqlens_q, a.cu_seqlens_k, a.seqused_k);
   const bool varlen = a.cu_seqlens_k != nullptr;
   const int kend = varlen ? g.lk : a.seqlen_k;  // rows this launch writes
@@ -334,7 +348,7 @@ __global__ void __launch_bounds__(kWaves * 64, kWavesPerSimd<D>) bwd_dkv_f32_ker
       }
     }
     if (p.ds) {
-      unsigned char* dst = ds_tile(p, b, qt, kt, hq) + ds_lane;
+      unsigned char* dst = ds_tile(p, pair, diag, qt, kt, hq - hk * p.group) + ds_lane;
 #pragma unroll
       for (int r = 0; r < 16; ++r) *reinterpret_cast<float*>(dst + (8 * (r >> 2) + (r & 3)) * 16) = dp[r];
     }
@@ -457,9 +471,9 @@ __global__ void __launch_bounds__(kWaves * 64, (RECOMPUTE && D == 128 ? 1 : kWav
   const int split = p.key_split;  // waves sharing an item's key tiles
   const int per_wg = kWaves / split;
   const int nblk = (p.ntq * p.group + per_wg - 1) / per_wg;
-  int pair, blk;
-  chunked_order((int)blockIdx.x, nblk, a.batch * a.heads_kv, pair, blk);
-  const int b = pair / a.heads_kv, hk = pair % a.heads_kv;
+  int pair, blk;  // (pair: of this launch)
+  chunked_order((int)blockIdx.x, nblk, p.npairs, pair, blk);
+  const int b = (p.pair0 + pair) / a.heads_kv, hk = (p.pair0 + pair) % a.heads_kv;
   const int item = blk * per_wg + wave / split;
   const int part = wave % split;
   const int qt = p.ntq - 1 - item / p.group;
@@ -495,7 +509,7 @@ __global__ void __launch_bounds__(kWaves * 64, (RECOMPUTE && D == 128 ? 1 : kWav
 #pragma unroll
     for (int c = 0; c < kRing; ++c) ring[c] = chunk(cur, c);
     if constexpr (!RECOMPUTE) {
-      const unsigned char* t = ds_tile(p, b, qt, j_lo + part, hq);
+      const unsigned char* t = ds_tile(p, pair, diag, qt, j_lo + part, item % p.group);
 #pragma unroll
       for (int k = 0; k < 4; ++k) dsb[k] = img_chunk(t, k, lane16);
     }
@@ -561,7 +575,7 @@ __global__ void __launch_bounds__(kWaves * 64, (RECOMPUTE && D == 128 ? 1 : kWav
 #pragma unroll
       for (int k = 0; k < 4; ++k) db[k] = acc_chunk(dp, k);
     } else {
-      const unsigned char* tn = ds_tile(p, b, qt, more ? kt + split : kt, hq);
+      const unsigned char* tn = ds_tile(p, pair, diag, qt, more ? kt + split : kt, item % p.group);
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         db[k] = dsb[k];
@@ -609,10 +623,11 @@ __global__ void __launch_bounds__(kWaves * 64, (RECOMPUTE && D == 128 ? 1 : kWav
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-// Workgroups per key tile of the dk/dv kernel: enough that the grid holds
-// ~1024, at most 8, and four steps of the walk (one per wave) each.
-int dkv_splits(const goda_prefill_args& a) {
-  const int64_t wgs = (int64_t)((a.seqlen_k + kF32Rows - 1) / kF32Rows) * a.heads_kv * a.batch;
+// Workgroups per key tile of the dk/dv kernel: enough that the grid over `pairs`
+// (sequence, KV head) pairs holds ~1024, at most 8, and four steps of the walk
+// (one per wave) each.
+int dkv_splits(const goda_prefill_args& a, int64_t pairs) {
+  const int64_t wgs = (int64_t)((a.seqlen_k + kF32Rows - 1) / kF32Rows) * pairs;
   if (wgs <= 0) return 1;
   const int64_t steps = (int64_t)(a.heads_q / a.heads_kv) * ((a.seqlen_q + kF32Rows - 1) / kF32Rows);
   const int64_t ns = std::min<int64_t>((1024 + wgs - 1) / wgs, steps / kWaves);
@@ -622,36 +637,71 @@ int dkv_splits(const goda_prefill_args& a) {
 int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
 
 // Workspace: query tiles, key tiles, dk/dv partials, key-major mask words, dS
-// tiles (ds < 0: none).
+// tiles of ds_pairs pairs (ds < 0: none).
 struct Layout {
-  int ntq, ntk, nsplit, ds_c, ds_tri;
-  int64_t kvimg, part, mask, ds, ds_per_b, total;
+  int ntq, ntk, nsplit, ds_c, ds_tri, ds_band;
+  int64_t kvimg, part, mask, ds, ds_per_pair, ds_pairs, total;
 };
+int64_t ds_pair_bytes(const goda_prefill_args& a, const Layout& l) {
+  return l.ds_per_pair * (a.heads_q / a.heads_kv) * kDsTile;
+}
+// The layout with dS tiles of `pairs` pairs (0: none).
 template <int D>
-Layout layout(const goda_prefill_args& a) {
+Layout layout_with(const goda_prefill_args& a, int nsplit, int64_t pairs) {
   Layout l{};
   l.ntq = (a.seqlen_q + kF32Rows - 1) / kF32Rows;
   l.ntk = (a.seqlen_k + kF32Rows - 1) / kF32Rows;
-  l.nsplit = dkv_splits(a);
+  l.nsplit = nsplit;
   l.kvimg = (int64_t)a.batch * l.ntq * a.heads_q * QTile<D>::BYTES;
   l.part = l.kvimg + (int64_t)a.batch * l.ntk * a.heads_kv * KTile<D>::BYTES;
   l.mask = l.part;
   if (l.nsplit > 1) l.mask += (int64_t)l.nsplit * 2 * a.batch * a.seqlen_k * a.heads_kv * D * 4;
   l.mask = align256(l.mask);
   l.total = l.mask + 4 * bwd_mask_t_words(a);
-  // causal batches of equal lengths keep only the visible key tiles
-  const bool varlen = a.cu_seqlens_q != nullptr || a.cu_seqlens_k != nullptr;
-  const int diag = a.seqlen_k - a.seqlen_q;
-  l.ds_tri = a.causal && !varlen && diag >= 0;
-  l.ds_c = l.ds_tri ? (diag + kF32Rows - 1) / kF32Rows : 0;
-  l.ds_per_b = ds_row_off(l.ntq, l.ntk, l.ds_c, l.ds_tri != 0);
-  const int64_t bytes = (int64_t)a.batch * l.ds_per_b * a.heads_q * kDsTile;
+  // A causal batch keeps only the key tiles that a query tile can see: up to the
+  // diagonal where every sequence's keys run the same way past its queries (equal
+  // lengths, or the same packed rows: then past them only as far as the clamp to
+  // the launch's sizes leaves), and those of the left window.
+  l.ds_tri = a.causal && (!a.cu_seqlens_q || a.cu_seqlens_q == a.cu_seqlens_k);
+  l.ds_c = l.ds_tri ? (std::max(0, a.seqlen_k - a.seqlen_q) + kF32Rows - 1) / kF32Rows : 0;
+  l.ds_per_pair = ds_row_off(l.ntq, l.ntk, l.ds_c, l.ds_tri != 0);
+  if (a.window_left >= 0 && (a.causal || a.seqlen_q == 1)) {
+    // keys from W before a tile's first row to its last row: W + 32 positions
+    const int64_t band = ((int64_t)a.window_left + 2 * (kF32Rows - 1)) / kF32Rows + 1;
+    if (band < l.ntk && l.ntq * band < l.ds_per_pair) {
+      l.ds_band = (int)band;
+      l.ds_per_pair = l.ntq * band;
+    }
+  }
+  l.ds_pairs = pairs;
   l.ds = -1;
-  if (bytes <= kDsMaxBytes) {
+  if (pairs > 0) {
     l.ds = align256(l.total);
-    l.total = l.ds + bytes;
+    l.total = l.ds + pairs * ds_pair_bytes(a, l);
   }
   return l;
+}
+// The layout for a workspace of `room` bytes. Where it does not hold the dS tiles
+// wanted, those of fewer pairs (a grid of 512 key tiles at least: fewer leave the
+// GPU idle), then none, then no split walk of dk/dv. The last is the least that a
+// launch runs with, and grows with every size.
+template <int D>
+Layout layout(const goda_prefill_args& a, int64_t room) {
+  const int64_t pairs = (int64_t)a.batch * a.heads_kv;
+  const int nsplit = dkv_splits(a, pairs);
+  const Layout none = layout_with<D>(a, nsplit, 0);
+  const int64_t bytes = ds_pair_bytes(a, none);
+  int64_t n = pairs;
+  if (bytes * pairs > kDsMaxBytes) n = bytes > kDsMaxBytes ? 0 : std::max<int64_t>(1, kDsChunkBytes / bytes);
+  if (n > 0) {
+    Layout l = layout_with<D>(a, dkv_splits(a, n), n);
+    if (l.total <= room) return l;
+    for (n = std::min(n, (room - none.total) / std::max<int64_t>(bytes, 1)); n > 0 && n * l.ntk >= 512; n = n * 7 / 8) {
+      l = layout_with<D>(a, dkv_splits(a, n), n);
+      if (l.total <= room) return l;
+    }
+  }
+  return none.total <= room ? none : layout_with<D>(a, 1, 0);
 }
 
 template <int D, bool ALIBI, bool MASK>
@@ -660,35 +710,48 @@ hipError_t launch_main(BwdParams p, hipStream_t s) {
   hipError_t e;
   constexpr int lds = (int)std::max<size_t>(sizeof(SumSmem<D>), 2 * kF32Img<D>);
   if ((e = record_timing(p.g.timing_begin, s)) != hipSuccess) return e;
-  if (p.ntk > 0) {
-    auto kern = bwd_dkv_f32_kernel<D, ALIBI, MASK>;
-    if ((e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds)) != hipSuccess) return e;
-    kern<<<dim3(p.ntk, a.heads_kv * p.nsplit, a.batch), kWaves * 64, lds, s>>>(p);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    if (p.nsplit > 1) {
-      const int64_t threads = (int64_t)a.seqlen_k * (D / 8);
-      bwd_dkv_reduce_f32_kernel<D><<<dim3((unsigned)((threads + 255) / 256), a.heads_kv, a.batch), 256, 0, s>>>(p);
+  auto dkv = bwd_dkv_f32_kernel<D, ALIBI, MASK>;
+  auto dq = p.ds ? bwd_dq_f32_kernel<D, false, false, false> : bwd_dq_f32_kernel<D, true, ALIBI, MASK>;
+  constexpr int sums = (int)sizeof(SumSmem<D>);
+  if ((e = hipFuncSetAttribute((const void*)dkv, hipFuncAttributeMaxDynamicSharedMemorySize, lds)) != hipSuccess) return e;
+  if ((e = hipFuncSetAttribute((const void*)dq, hipFuncAttributeMaxDynamicSharedMemorySize, sums)) != hipSuccess) return e;
+  // Equal runs of pairs, no more than the dS tiles have room for, in whole
+  // rounds over the XCDs (chunked_order) where that allows.
+  const int pairs = a.batch * a.heads_kv;
+  int most = p.npairs;
+  if (most < pairs && most >= kOrderChunk) most = most / kOrderChunk * kOrderChunk;
+  const int runs = (pairs + most - 1) / most;
+  int run = (pairs + runs - 1) / runs;
+  if (run < pairs && run >= kOrderChunk) run = (run + kOrderChunk - 1) / kOrderChunk * kOrderChunk;
+  for (p.pair0 = 0; p.pair0 < pairs; p.pair0 += run) {
+    p.npairs = std::min(run, pairs - p.pair0);
+    if (p.ntk > 0) {
+      const int64_t nblk = (int64_t)p.ntk * p.npairs * p.nsplit;
+      if (nblk > 0x7fffffff) return hipErrorInvalidValue;
+      dkv<<<dim3((unsigned)nblk), kWaves * 64, lds, s>>>(p);
+      if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
+    if (p.ntq > 0) {
+      p.key_split = f32_key_split(a, (int64_t)p.ntq * p.group * p.npairs);
+      const int per_wg = kWaves / p.key_split;
+      const int64_t nblk = ((int64_t)p.ntq * p.group + per_wg - 1) / per_wg * p.npairs;
+      if (nblk > 0x7fffffff) return hipErrorInvalidValue;
+      dq<<<dim3((unsigned)nblk), kWaves * 64, sums, s>>>(p);
       if ((e = hipGetLastError()) != hipSuccess) return e;
     }
   }
-  if (p.ntq > 0) {
-    p.key_split = f32_key_split(a, (int64_t)p.ntq * a.heads_q * a.batch);
-    const int per_wg = kWaves / p.key_split;
-    const int64_t nblk = ((int64_t)p.ntq * p.group + per_wg - 1) / per_wg * a.heads_kv * a.batch;
-    if (nblk > 0x7fffffff) return hipErrorInvalidValue;
-    auto kern = p.ds ? bwd_dq_f32_kernel<D, false, false, false> : bwd_dq_f32_kernel<D, true, ALIBI, MASK>;
-    constexpr int sums = (int)sizeof(SumSmem<D>);
-    if ((e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, sums)) != hipSuccess) return e;
-    kern<<<dim3((unsigned)nblk), kWaves * 64, sums, s>>>(p);
+  if (p.ntk > 0 && p.nsplit > 1) {
+    const int64_t threads = (int64_t)a.seqlen_k * (D / 8);
+    bwd_dkv_reduce_f32_kernel<D><<<dim3((unsigned)((threads + 255) / 256), a.heads_kv, a.batch), 256, 0, s>>>(p);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   return record_timing(p.g.timing_end, s);
 }
 
 template <int D>
-hipError_t launch_d(BwdParams p, hipStream_t s) {
+hipError_t launch_d(BwdParams p, int64_t room, hipStream_t s) {
   const goda_prefill_args& a = p.a;
-  const Layout l = layout<D>(a);
+  const Layout l = layout<D>(a, room);
   p.ntq = l.ntq;
   p.ntk = l.ntk;
   p.nsplit = l.nsplit;
@@ -696,9 +759,11 @@ hipError_t launch_d(BwdParams p, hipStream_t s) {
   p.kvimg = p.qimg + l.kvimg;
   p.part = reinterpret_cast<float*>(p.qimg + l.part);
   p.ds = l.ds >= 0 ? p.qimg + l.ds : nullptr;
-  p.ds_per_b = l.ds_per_b;
+  p.ds_per_pair = l.ds_per_pair;
   p.ds_c = l.ds_c;
   p.ds_tri = l.ds_tri;
+  p.ds_band = l.ds_band;
+  p.npairs = p.ds ? (int)l.ds_pairs : a.batch * a.heads_kv;
   hipError_t e;
   if (a.mask_bits) {
     p.mask_t = reinterpret_cast<uint32_t*>(p.qimg + l.mask);
@@ -718,18 +783,18 @@ hipError_t launch_d(BwdParams p, hipStream_t s) {
 
 }  // namespace
 
-int64_t prefill_bwd_f32_workspace_bytes(const goda_prefill_args& a) {
-  return a.head_dim == 64 ? layout<64>(a).total : a.head_dim == 128 ? layout<128>(a).total : layout<256>(a).total;
+int64_t prefill_bwd_f32_workspace_bytes(const goda_prefill_args& a, int64_t room) {
+  return a.head_dim == 64 ? layout<64>(a, room).total : a.head_dim == 128 ? layout<128>(a, room).total : layout<256>(a, room).total;
 }
 
-hipError_t launch_prefill_bwd_f32(const BwdParams& p, hipStream_t s) {
+hipError_t launch_prefill_bwd_f32(const BwdParams& p, int64_t room, hipStream_t s) {
   switch (p.a.head_dim) {
     case 64:
-      return launch_d<64>(p, s);
+      return launch_d<64>(p, room, s);
     case 128:
-      return launch_d<128>(p, s);
+      return launch_d<128>(p, room, s);
     case 256:
-      return launch_d<256>(p, s);
+      return launch_d<256>(p, room, s);
     default:
       return hipErrorNotSupported;
   }

@@ -68,6 +68,12 @@ struct BwdParams {
   unsigned char* ds;
   int64_t ds_per_b;
   int64_t ds_sink;       // byte offset past the tiles: 2 KB that only take writes
+  // fp32: the (sequence, KV head) pairs of this launch, whose dS tiles the
+  // buffer holds, and a pair's tiles per query head. ds_band > 0: query tile q
+  // holds ds_band key tiles from the first that its window reaches.
+  int pair0, npairs;
+  int ds_band;
+  int64_t ds_per_pair;
   int ds_c, ds_tri;
   int ds_hpw;            // query heads per workgroup of the dq-from-dS kernel
 };
@@ -81,8 +87,10 @@ __host__ __device__ __forceinline__ int64_t ds_row_off(int qt, int ntk, int c, b
   const int q1 = qt < m ? qt : m;
   return (int64_t)q1 * (q1 - 1) / 2 + (int64_t)q1 * (c + 1) + (int64_t)(qt - q1) * ntk;
 }
-// Backward: workspace bytes and the launch.
+// Backward: workspace bytes (the most that a launch uses, the least that it
+// runs with) and the launch.
 int64_t prefill_bwd_workspace_bytes(const goda_prefill_args& a);
+int64_t prefill_bwd_least_bytes(const goda_prefill_args& a);
 hipError_t launch_prefill_bwd(const BwdParams& p, hipStream_t s);
 // Fused QK-RMSNorm backward (norm_bwd.hip): fp32 dw partials' bytes, and dx /
 // dw from the attention backward's dq / dk (gradients of the normalized rows).
@@ -95,9 +103,10 @@ hipError_t launch_norm_bwd(const goda_prefill_args& a, const goda_prefill_grads&
 // p.mask_t and sets their strides.
 int64_t bwd_mask_t_words(const goda_prefill_args& a);
 hipError_t launch_bwd_mask_t(BwdParams& p, hipStream_t s);
-// fp32 backward with operands streamed from L2.
-int64_t prefill_bwd_f32_workspace_bytes(const goda_prefill_args& a);
-hipError_t launch_prefill_bwd_f32(const BwdParams& p, hipStream_t s);
+// fp32 backward with operands streamed from L2: bytes of the largest layout
+// that `room` bytes hold, or of the smallest.
+int64_t prefill_bwd_f32_workspace_bytes(const goda_prefill_args& a, int64_t room);
+hipError_t launch_prefill_bwd_f32(const BwdParams& p, int64_t room, hipStream_t s);
 int64_t prefill_bwd_mfma_workspace_bytes(const goda_prefill_args& a);
 hipError_t launch_prefill_bwd_mfma(BwdParams p, hipStream_t s);
 

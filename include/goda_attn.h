@@ -283,8 +283,11 @@ int64_t goda_attn_prefill_workspace_size(const goda_prefill_args* args);
  * the packed varlen call of mint/nn/flashattn.py:123-133 (cu_seqlens). */
 int32_t goda_attn_prefill_fwd(const goda_prefill_args* args, void* stream);
 
-/* Workspace needed by goda_attn_prefill_bwd for these forward arguments
- * (bytes, >= 0), or a negative status if they are rejected. */
+/* Workspace of goda_attn_prefill_bwd for these forward arguments (bytes, >= 0),
+ * or a negative status if they are rejected. fp32 calls also run, somewhat
+ * slower, in a smaller one that holds their operand images (the status
+ * GODA_ERR_WORKSPACE names that size): one workspace sized for a program's
+ * largest batch serves its smaller ones. */
 int64_t goda_attn_prefill_bwd_workspace_size(const goda_prefill_args* fwd);
 
 /* Backward of goda_attn_prefill_fwd: dq, dk, dv from d_o and the forward's

@@ -199,3 +199,24 @@ def test_missing_library_is_a_loud_error(tmp_path):
     env = dict(os.environ, GODA_ATTN_LIB=str(tmp_path / "nope" / "libgoda_attn.so"))
     out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, env=env, timeout=300, cwd=str(ROOT))
     assert "raised:" in out.stdout and "no non-HIP fallback" in out.stdout, out.stdout + out.stderr
+
+
+def test_backward_fp32_workspace_of_windows_and_batches(lib):
+    """fp32 dS tiles: a left window holds its band alone, packed rows of one
+    cu_seqlens array a triangle, and a batch whose tiles pass 8 GiB keeps those
+    of a part of it (here 4 GiB)."""
+    size = lambda **kw: lib.goda_attn_prefill_bwd_workspace_size(ctypes.byref(_prefill_args(dtype=_lib.DTYPE_F32, **kw)))  # noqa: E731
+    long = dict(batch=1, heads_q=32, heads_kv=8, seqlen_q=8192, seqlen_k=8192)
+    images = 256 * (32 * (4 * 128 * 32 * 4 + 256) + 8 * 3 * 128 * 32 * 4)
+    band = (128 + 62) // 32 + 1
+    assert size(**long, window_left=128) <= images + 256 * band * 32 * 4096 + 512
+    buffers = [ctypes.create_string_buffer(16) for _ in range(2)]
+    table = [ctypes.addressof(x) for x in buffers]
+    packed = dict(batch=4, heads_q=8, heads_kv=8, seqlen_q=2048, seqlen_k=2048)
+    one = size(**packed, cu_seqlens_q=table[0], cu_seqlens_k=table[0])
+    two = size(**packed, cu_seqlens_q=table[0], cu_seqlens_k=table[1])
+    assert one == size(**packed) and two - one == 4 * 8 * (64 * 64 - 64 * 65 // 2) * 4096
+    square = dict(heads_q=32, heads_kv=8, seqlen_q=4096, seqlen_k=4096)
+    one, images = 128 * 129 // 2 * 4 * 4096, 128 * (32 * (4 * 128 * 32 * 4 + 256) + 8 * 3 * 128 * 32 * 4)  # a pair, a sequence
+    assert size(batch=4, **square) - 4 * images - 32 * one in range(256)
+    assert size(batch=8, **square) - 8 * images - (4 << 30) // one * one in range(256)

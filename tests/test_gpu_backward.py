@@ -12,6 +12,7 @@ cannot hold x more closely than its rounding.
 from __future__ import annotations
 
 import math
+import re
 
 import numpy as np
 import pytest
@@ -470,9 +471,103 @@ def test_backward_fp32_streamed(d, b, tq, tk, hq, hkv, causal, window):
     _case(b, tq, tk, hq, hkv, d, torch.float32, causal=causal, seed=d + tq, window=window)
 
 
+def _least_workspace(plan) -> int:
+    """The bytes that a refused workspace is told it needs; the plan is left
+    with a workspace of just that."""
+    plan.grads.workspace_bytes = 0
+    with pytest.raises(Exception, match="workspace of") as e:
+        plan()
+    plan.grads.workspace_bytes = int(re.search(r"workspace of (\d+) bytes", str(e.value))[1])
+    return plan.grads.workspace_bytes
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("b,tq,tk,hq,hkv,causal,window,alibi,masked", [
+    (2, 97, 97, 4, 2, True, -1, False, False),
+    (1, 40, 130, 6, 1, True, -1, True, False),  # the diagonal 90 keys in
+    (1, 130, 40, 2, 2, True, -1, False, True),  # rows without a key
+    (1, 300, 300, 3, 1, True, 0, False, False),  # one key a row: bands of two tiles
+    (1, 300, 300, 2, 1, True, 1, True, False),
+    (1, 290, 323, 2, 2, True, 34, False, True),
+    (1, 300, 300, 2, 1, True, 290, False, False),  # a window that leaves no band
+    (2, 1, 300, 4, 1, False, 70, False, False),
+    (1, 70, 100, 4, 4, False, -1, True, True),
+])
+def test_backward_fp32_stored_and_recomputed(d, b, tq, tk, hq, hkv, causal, window, alibi, masked):
+    """dq from stored dS tiles (a triangle, a window's band, or all of them) and,
+    in the least workspace the call accepts, from S and dP formed again, with a
+    walk of dk/dv that is not split: both within the oracle's bounds. A byte less
+    is refused."""
+    q, k, v, d_o = (_rand((b, t, h, d), torch.float32, s) for s, (t, h) in enumerate(((tq, hq), (tk, hkv), (tk, hkv), (tq, hq))))
+    kw, okw = dict(causal=causal, window_left=window), dict(causal=causal, window_size=(window, -1))
+    if alibi:
+        okw["alibi_slopes"] = torch.tensor(wl.alibi_slopes(hq), dtype=torch.float32)
+        kw["alibi_slopes"] = okw["alibi_slopes"].to(DEV)
+    if masked:
+        okw["base_attn_mask"] = torch.rand(b, 1, tq, tk, generator=torch.Generator().manual_seed(d)) < 0.8
+        kw["attn_mask"] = okw["base_attn_mask"].to(DEV)
+    x = [y.to(DEV) for y in (q, k, v)]
+    o, lse = ops.attention_prefill(*x, return_lse=True, **kw)
+    plan = ops.plan_prefill_bwd(*x, o, lse, d_o.to(DEV), **kw)
+    refs = ref.attention_grads(q, k, v, d_o, **okw)
+    _check(plan(), refs, torch.float32, f"stored d{d} {tq}/{tk}")
+    full, least = plan.grads.workspace_bytes, _least_workspace(plan)
+    assert least < full
+    for y in plan.result:
+        y.fill_(float("nan"))
+    _check(plan(), refs, torch.float32, f"recomputed d{d} {tq}/{tk}")
+    plan.grads.workspace_bytes = least - 1
+    with pytest.raises(Exception, match="workspace of"):
+        plan()
+
+
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("window", [-1, 20])
+@pytest.mark.parametrize("same", [True, False])  # one cu_seqlens array (a triangle of dS tiles), or two
+def test_backward_fp32_packed_in_a_smaller_workspace(same, window, norm):
+    """Packed documents in the workspace of a smaller call than the query's
+    (no dS tiles) and in the whole one: the same gradients, those of the norm
+    weights among them. The two forms differ in the order of fp32 sums."""
+    lens, hq, hkv, d = [70, 1, 160, 0, 33], 4, 2, 128
+    n, m = sum(lens), max(lens)
+    cu = torch.tensor([sum(lens[:i]) for i in range(len(lens) + 1)], dtype=torch.int32, device=DEV)
+    q, k, v, d_o = (_rand((n, h, d), torch.float32, s).to(DEV) for s, h in enumerate((hq, hkv, hkv, hq)))
+    kw = dict(causal=True, window_left=window, cu_seqlens_q=cu, cu_seqlens_k=cu if same else cu.clone(), max_seqlen_q=m, max_seqlen_k=m)
+    if norm:
+        kw.update(q_norm_weight=_rand((d,), torch.float32, 8).to(DEV), k_norm_weight=_rand((d,), torch.float32, 9).to(DEV))
+    o, lse = ops.attention_prefill(q, k, v, return_lse=True, **kw)
+    plan = ops.plan_prefill_bwd(q, k, v, o, lse, d_o, **kw)
+    full, want = plan.grads.workspace_bytes, [y.clone() for y in plan()]
+    assert _least_workspace(plan) < full
+    for got, w in zip(plan(), want):
+        assert (got - w).abs().max().item() <= 1e-5 * max(1.0, w.abs().max().item())
+
+
+def test_backward_fp32_workspace_of_the_largest_batch_serves_smaller_ones():
+    """One workspace, as the query gives it for the largest batch of a program,
+    at smaller batches: the split of dk/dv's walk, which the query's size turns
+    on, ends between 31 and 32 sequences, so that 31 ask for more than 32. None
+    is refused, and the gradients are those of a workspace of their own (up to
+    the order of fp32 sums)."""
+    t, d = 1024, 64
+    q, k, v, d_o = (_rand((32, t, 1, d), torch.float32, s).to(DEV) for s in range(4))
+    largest, sizes = None, []
+    for b in (32, 31, 5):
+        o, lse = ops.attention_prefill(q[:b], k[:b], v[:b], causal=True, return_lse=True)
+        plan = ops.plan_prefill_bwd(q[:b], k[:b], v[:b], o, lse, d_o[:b], causal=True)
+        sizes.append(plan.grads.workspace_bytes)
+        want = [y.clone() for y in plan()]
+        largest = largest or plan
+        plan.grads.workspace, plan.grads.workspace_bytes = largest.grads.workspace, sizes[0]
+        for got, w in zip(plan(), want):
+            assert (got - w).abs().max().item() <= 1e-5 * max(1.0, w.abs().max().item())
+    assert sizes[1] > sizes[0] > sizes[2]
+
+
 def test_backward_fp32_without_stored_ds():
-    """Past 8 GB of dS tiles the dq kernel forms S and dP again: the gradients
-    of the whole batch are those of its halves, which store them. The two forms
+    """Past 4 GiB of dS tiles the pairs of a batch run in several launches: the
+    gradients of the whole batch are those of its halves, and those of the dq
+    kernel that forms S and dP again, for want of room. The last two forms
     differ in the order of dq's fp32 sums and in the rounding of the exponents'
     bias terms: slopes of at most 0.707 / 64 over 4608 keys keep those under 74
     log2 units, so two roundings change a probability by 2 * 74 * 2^-24 * ln 2
@@ -484,15 +579,20 @@ def test_backward_fp32_without_stored_ds():
     slopes = torch.tensor(wl.alibi_slopes(hq), dtype=torch.float32, device=DEV) / 64
     mask = torch.rand(b, 1, 1, t, device=DEV, generator=g) < 0.9
 
-    def grads(rows):
+    def grads(rows, least=False):
         x = [y[rows].contiguous() for y in (q, k, v)]
         kw = dict(causal=False, alibi_slopes=slopes, attn_mask=mask[rows])
         o, lse = ops.attention_prefill(*x, return_lse=True, **kw)
         plan = ops.plan_prefill_bwd(*x, o, lse, d_o[rows].contiguous(), **kw)
-        return plan(), plan.grads.workspace_bytes
+        ws = plan.grads.workspace_bytes
+        if least:
+            assert _least_workspace(plan) < 1 << 30
+        return plan(), ws
 
     whole, ws = grads(slice(0, b))
     half, ws_half = grads(slice(0, 4))
-    assert ws < 8 << 30 and ws_half > 4 << 30  # recomputed / stored
+    assert ws < 8 << 30 and ws_half > 4 << 30  # (four launches, two)
+    for w, h in zip(whole, grads(slice(0, 4), least=True)[0]):
+        assert (w[:4] - h).abs().max().item() <= 1e-4 * max(1.0, h.abs().max().item())
     for w, h in zip(whole, half):
         assert (w[:4] - h).abs().max().item() <= 1e-4 * max(1.0, h.abs().max().item())
