@@ -26,6 +26,7 @@ struct PrefillParams {
   int piece_tiles;    // key tiles per piece; 0: from the lengths, on the device
   int min_piece;
   float* pieces;      // the pieces' sums, behind the tile images
+  uint64_t* marks;    // key tiles that 32 query rows see of the caller's mask, behind the images; or NULL
 };
 
 struct DecodeParams {
@@ -118,7 +119,8 @@ hipError_t launch_prefill_generic(const PrefillParams& p, hipStream_t s);
 bool prefill_mfma_supported(const goda_prefill_args& a);
 int64_t prefill_mfma_workspace_bytes(const goda_prefill_args& a);
 // What it runs with at the least: the K/V tile images, without the room for the
-// sums of items whose keys are cut (then none are).
+// sums of items whose keys are cut (then none are) and for a mask's marks (then
+// all tiles are walked).
 int64_t prefill_mfma_least_bytes(const goda_prefill_args& a);
 hipError_t launch_prefill_mfma(const PrefillParams& p, hipStream_t s);
 

@@ -126,10 +126,11 @@ template <int D>
 constexpr bool kPersistent = D <= 128;
 
 // With a caller's mask: key tiles that no row of the workgroup sees are not
-// walked. The tiles that are stand in a list behind the LDS ring, for up to
-// this many tiles (more: all are walked).
+// walked. The pre-pass marks, per 32 query rows, the tiles that one of them sees
+// (mark_tiles); a workgroup lists those of its rows behind the LDS ring, for up
+// to kListTiles tiles (more: all are walked).
 constexpr int kListTiles = 4096;
-constexpr int kListBytes = kListTiles * 2 + kListTiles / 8;
+constexpr int kListBytes = kListTiles * 2;
 
 // Split keys (KSPLIT instances): an item's key tiles are cut into pieces that
 // workgroups of their own walk, for dense batches whose items are too few to
@@ -168,11 +169,61 @@ __device__ __forceinline__ int64_t ws_tile(int b, int j, int hk, int ntiles, int
   return ((int64_t)b * ntiles + j) * hkv + hk;
 }
 
+// Bits of the caller's boolean mask for one key tile of one query row: 64
+// keys in one 8-byte word, 32 in a 4-byte one.
+template <int BKV>
+struct MaskWord;
+template <>
+struct MaskWord<64> {
+  typedef uint64_t t;
+  static constexpr t kAll = ~0ull;
+};
+template <>
+struct MaskWord<32> {
+  typedef uint32_t t;
+  static constexpr t kAll = ~0u;
+};
+
+// Marks of the caller's mask, [sequence][query head][32 query rows][64 key
+// tiles], one bit a tile; dimensions that the mask broadcasts have size 1.
+struct Marks {
+  int batch, heads, blocks, words;
+};
+__host__ __device__ __forceinline__ Marks marks_of(const goda_prefill_args& a, int ntiles) {
+  return Marks{a.mask_stride_b ? a.batch : 1, a.mask_stride_h ? a.heads_q : 1, a.mask_stride_q ? (a.seqlen_q + 31) / 32 : 1,
+               (ntiles + 63) / 64};
+}
+// One wave: the marks of block `u` of 32 rows. A lane holds a tile, so that a
+// row's words are one run of memory, and eight rows are in flight.
+template <int BKV>
+__device__ __forceinline__ void mark_tiles(const PrefillParams& p, int64_t u) {
+  typedef typename MaskWord<BKV>::t mword_t;
+  const goda_prefill_args& a = p.a;
+  const Marks k = marks_of(a, p.ntiles_k);
+  if (u >= (int64_t)k.batch * k.heads * k.blocks) return;
+  const int lane = threadIdx.x & 63;
+  const int block = (int)(u % k.blocks);
+  const int h = (int)(u / k.blocks % k.heads), b = (int)(u / k.blocks / k.heads);
+  const uint32_t* rows = mask_row(a, b, h, 32 * block);
+  const int last = a.mask_stride_q ? min(32, a.seqlen_q - 32 * block) - 1 : 0;
+  for (int w = 0; w < k.words; ++w) {
+    const int t = min(64 * w + lane, p.ntiles_k - 1);
+    mword_t any = 0;
+    for (int r0 = 0; r0 <= last; r0 += 8) {
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+        any |= reinterpret_cast<const mword_t*>(rows + min(r0 + r, last) * a.mask_stride_q)[t];
+    }
+    const uint64_t m = __builtin_amdgcn_ballot_w64(any != 0 && 64 * w + lane < p.ntiles_k);
+    if (lane == 0) p.marks[u * k.words + w] = m;
+  }
+}
 
 // ---------------------------------------------------------------------------
-// 1. pack K (rotated) and V^T into tile images
+// 1. pack K (rotated) and V^T into tile images; with a caller's mask, blocks
+// past the tiles mark what its rows see
 // ---------------------------------------------------------------------------
-template <typename T, int D, int BKV>
+template <typename T, int D, int BKV, bool MASK>
 __global__ void __launch_bounds__(256) pack_kv_kernel(const PrefillParams p) {
   typedef typename Vec<T>::v8 v8;
   typedef TileGeom<T, D, BKV, 1> TG;
@@ -180,6 +231,13 @@ __global__ void __launch_bounds__(256) pack_kv_kernel(const PrefillParams p) {
   const int j = blockIdx.x;
   const int hk = blockIdx.y;
   const int b = blockIdx.z;
+  if constexpr (MASK) {
+    if (j >= p.ntiles_k) {
+      const int64_t group = ((int64_t)b * a.heads_kv + hk) * (gridDim.x - p.ntiles_k) + j - p.ntiles_k;
+      mark_tiles<BKV>(p, 4 * group + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+      return;
+    }
+  }
   const SeqGeom g = seq_geom(b, a.seqlen_q, a.seqlen_k, a.cu_seqlens_q, a.cu_seqlens_k,
                              a.seqused_k);
   const int kv0 = j * BKV;
@@ -356,21 +414,6 @@ __device__ __forceinline__ float dot2_ones(f16x8 p, int i, float acc) {
   return __builtin_amdgcn_fdot2(v, one, acc, false);
 }
 
-// Bits of the caller's boolean mask for one key tile of one query row: 64
-// keys in one 8-byte word, 32 in a 4-byte one.
-template <int BKV>
-struct MaskWord;
-template <>
-struct MaskWord<64> {
-  typedef uint64_t t;
-  static constexpr t kAll = ~0ull;
-};
-template <>
-struct MaskWord<32> {
-  typedef uint32_t t;
-  static constexpr t kAll = ~0u;
-};
-
 // Non-persistent grid: the work item of workgroup `lin` of `nblk`.
 __device__ __forceinline__ void grid_item(const PrefillParams& p, const int lin, const int nblk, const int qb_rows,
                                           int& pair, int& qt) {
@@ -529,8 +572,10 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
 
   // ---- Q^T operand fragments (rotated) ---------------------------------------
   v8 qf[NT][KS];
-  // (invoked in the prologue, after the first tiles' copies are issued)
-  auto load_q = [&]() {
+  // (invoked in the prologue, after the first tiles' copies are issued; part 1:
+  // the loads alone, 2: what comes after them)
+  auto load_q = [&](auto part) {
+    constexpr int PART = decltype(part)::value;
     const T* qbase = reinterpret_cast<const T*>(a.q) +
                      (a.cu_seqlens_q ? 0 : (int64_t)b * a.q_stride_b) + (int64_t)hq * a.q_stride_h;
 #pragma unroll
@@ -538,9 +583,10 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
       const int qi = wrow0 + 32 * nt + l32;
       if (qi < g.lq) {
         const T* qr = qbase + (g.q_row0 + qi) * a.q_stride_t;
+        if constexpr (PART != 2)
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) qf[nt][ks] = ld_vec<v8>(qr + 16 * ks + 8 * hi);
-        {
+          for (int ks = 0; ks < KS; ++ks) qf[nt][ks] = ld_vec<v8>(qr + 16 * ks + 8 * hi);
+        if constexpr (PART != 1) {
           // fp32 round trip: fused QK-RMSNorm, then RoPE, then the softmax
           // scale in log2 units (scores come out of the MFMA ready for exp2),
           // one rounding.
@@ -587,7 +633,7 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
 #pragma unroll
             for (int e = 0; e < 8; ++e) qf[nt][ks][e] = (T)(xf[ks][e] * p.scale_log2);
         }
-      } else {
+      } else if constexpr (PART != 2) {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) qf[nt][ks] = v8{};
       }
@@ -595,10 +641,11 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
     // Pin the fragments in registers: without this the compiler treats the
     // (read-only) q loads as rematerializable and re-reads q from global
     // memory inside the key loop.
+    if constexpr (PART != 1)
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
+      for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[nt][ks]));
+        for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[nt][ks]));
   };
 
   // ---- key tile range ---------------------------------------------------------
@@ -623,16 +670,45 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
   // holds (nearly) every row's max and the lazy rescale seldom fires again;
   // in key order the max moved by the slope per key and rescaled often.
   // Stages and loop bounds stay in step order.
-  // With a caller's mask (and a tile list, below) step j is entry j of the list,
-  // whose tiles count from list_base.
-  const uint16_t* tile_list = nullptr;
-  int list_base = 0;
-  int j_rev = j_lo + j_hi - 1;
+  // With a caller's mask the steps are those of the tiles that some row sees,
+  // counted from 0, and a list in LDS has their tiles (`listed`: some tile is
+  // hidden). Lane i of `walk` holds the tile of step walk0 + i, so that a tile is
+  // read by one v_readlane, without a branch or a wait; head_dim 256, which has
+  // no register for it, reads the list. `ahead`: the tiles of the steps j .. j +
+  // kAhead, read one step before the first use.
+  constexpr bool WALK = D <= 128;
+  uint16_t* list = reinterpret_cast<uint16_t*>(smem + kStages * TG::BYTES);
+  bool listed = false;
+  const int first_tile = j_lo;
+  if constexpr (MASK) {
+    j_hi = max(j_hi - j_lo, 0);
+    j_lo = 0;
+  }
+  const int j_rev = j_lo + j_hi - 1;
+  int walk = 0, walk0 = 0, ahead[kAhead + 1];
+  // Lane i's tile of the 64 steps from j (the last ones' where there are fewer).
+  auto fill_walk = [&](int j) {
+    if constexpr (WALK) {
+      walk0 = j;
+      const int i = min(j + lane, j_hi - 1);
+      walk = first_tile + (listed ? (int)list[i] : ALIBI ? j_rev - i : i);
+    }
+  };
   auto tile_of = [&](int j) {
-    const int i = ALIBI ? j_rev - j : j;
-    if constexpr (MASK)
-      if (tile_list) return list_base + __builtin_amdgcn_readfirstlane((int)tile_list[i]);
-    return i;
+    if constexpr (MASK && WALK) return __builtin_amdgcn_readlane(walk, j - walk0);
+    if constexpr (MASK) {
+      const int i = min(j, j_hi - 1);
+      return first_tile + (listed ? __builtin_amdgcn_readfirstlane((int)list[i]) : ALIBI ? j_rev - i : i);
+    }
+    return ALIBI ? j_rev - j : j;
+  };
+  // The tile of step j in the key loop, j being `K` steps past the current one.
+  typedef std::integral_constant<int, 0> Now;
+  typedef std::integral_constant<int, 1> Next;
+  typedef std::integral_constant<int, kAhead> Copied;
+  auto tile_at = [&](auto k, int j) {
+    if constexpr (MASK) return ahead[decltype(k)::value];
+    return tile_of(j);
   };
 
   f32x16 oacc[MD][NT];
@@ -678,56 +754,6 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
       mrow[nt] = reinterpret_cast<const mword_t*>(mask_row(a, b, hq, min(wrow0 + 32 * nt + l32, g.lq - 1)));
       mw[nt] = MaskWord<BKV>::kAll;
     }
-    // The list of the tiles that hold a visible key: each wave marks those of
-    // its rows in a bit set, lanes l and l ^ 32 two tiles of a row at a time;
-    // then a tile's place is the number of marked tiles before it. (Masks of
-    // documents, prefixes or padding hide whole tiles, which otherwise cost
-    // as much as visible ones: B=4, T=2048, 16/4 heads, a prefix mask over
-    // half the tiles, 142 -> 121 us.)
-    const int ntl = j_hi - j_lo;
-    if (ntl > 0 && ntl <= kListTiles) {
-      uint16_t* list = reinterpret_cast<uint16_t*>(smem + kStages * TG::BYTES);
-      uint32_t* seen = reinterpret_cast<uint32_t*>(list + kListTiles);
-      const int nw = (ntl + 31) / 32;
-      for (int i = tid; i < nw; i += WAVES * 64) seen[i] = 0;
-      __syncthreads();
-      for (int t0 = 0; t0 < ntl; t0 += 8) {
-        bool any[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {  // (the loads of four pairs in flight)
-          const int u = t0 + 2 * k + hi;
-          any[k] = false;
-          if (u < ntl) {
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) any[k] = any[k] || mrow[nt][j_lo + u] != 0;
-          }
-        }
-        uint32_t bits = 0;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const uint64_t m = __builtin_amdgcn_ballot_w64(any[k]);
-          bits |= (((uint32_t)m != 0 ? 1u : 0u) | ((uint32_t)(m >> 32) != 0 ? 2u : 0u)) << (2 * k);
-        }
-        if (bits && lane == 0) atomicOr(&seen[t0 >> 5], bits << (t0 & 31));
-      }
-      __syncthreads();
-      int total = 0;
-      for (int t = tid; t < nw * 32; t += WAVES * 64) {
-        const uint32_t w = seen[t >> 5];
-        if ((w >> (t & 31)) & 1u) {
-          int at = __popc(w & ((1u << (t & 31)) - 1u));
-          for (int i = 0; i < (t >> 5); ++i) at += __popc(seen[i]);
-          list[at] = (uint16_t)t;
-        }
-      }
-      for (int i = 0; i < nw; ++i) total += __popc(seen[i]);
-      __syncthreads();
-      tile_list = list;
-      list_base = j_lo;
-      j_lo = 0;
-      j_hi = __builtin_amdgcn_readfirstlane(total);
-      j_rev = j_hi - 1;
-    }
   }
 
   // ---- tile ring ----------------------------------------------------------------
@@ -743,8 +769,8 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
   constexpr bool SPLIT = kSplitStaging<D> && WAVES == 8 && LOADS % 2 == 0;
   constexpr int NSTG = SPLIT ? LOADS / 2 : LOADS;
   v8 stg[NSTG];
-  auto tile_load_part = [&](int j, int part) {
-    const v8* src = reinterpret_cast<const v8*>(ws + ws_tile(b, tile_of(j), hk, ntiles_k, heads_kv) * TG::BYTES) +
+  auto tile_load_part = [&](int tile, int part) {
+    const v8* src = reinterpret_cast<const v8*>(ws + ws_tile(b, tile, hk, ntiles_k, heads_kv) * TG::BYTES) +
                     my_chunk0 + part * NSTG * 64;
 #pragma unroll
     for (int i = 0; i < NSTG; ++i) stg[i] = src[i * 64];
@@ -754,11 +780,11 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
 #pragma unroll
     for (int i = 0; i < NSTG; ++i) dst[i * 64] = stg[i];
   };
-  auto tile_load = [&](int j) {
-    tile_load_part(j, 0);
+  auto tile_load = [&](int j, int tile) {
+    tile_load_part(tile, 0);
     if constexpr (SPLIT) {
       tile_store_part(j, 0);
-      tile_load_part(j, 1);
+      tile_load_part(tile, 1);
     }
   };
   auto tile_store = [&](int j) { tile_store_part(j, SPLIT ? 1 : 0); };
@@ -779,9 +805,9 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
   static_assert(!DMA || LOADS == 2 || LOADS == 4, "DMA share of 2 or 4 blocks");
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   const unsigned lane_off = (unsigned)((wave_u * LOADS * 64 + lane) * 16);
-  auto tile_dma = [&](int j) {
+  auto tile_dma = [&](int j, int tile) {
     const unsigned long long base =
-        (unsigned long long)(uintptr_t)(ws + ws_tile(b, tile_of(j), hk, ntiles_k, heads_kv) * TG::BYTES);
+        (unsigned long long)(uintptr_t)(ws + ws_tile(b, tile, hk, ntiles_k, heads_kv) * TG::BYTES);
     const unsigned lds0 =
         (unsigned)(uintptr_t)(smem + ((j - j_lo) & (kStages - 1)) * TG::BYTES) + (unsigned)(wave_u * LOADS * 64 * 16);
     dma_blocks<LOADS>(lds0, lane_off, base);
@@ -802,10 +828,10 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
   // last step of a workgroup that does not peel it (head_dim 256), where j is
   // clamped for the mask words and the bias and the products read stage
   // j + 1 (whatever it holds; they are never used).
-  auto qk = [&](int j, f32x16 (&s)[MT][NT], int js) {
+  auto qk = [&](auto k, int j, f32x16 (&s)[MT][NT], int js) {
     if constexpr (MASK) {
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) mw[nt] = mrow[nt][tile_of(j)];
+      for (int nt = 0; nt < NT; ++nt) mw[nt] = mrow[nt][tile_at(k, j)];
     }
     const v8* kp = reinterpret_cast<const v8*>(smem + ((js - j_lo) & (kStages - 1)) * TG::BYTES) + hi * BKV + l32;
 #pragma unroll
@@ -813,7 +839,7 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
       const float m0 = (m_run[nt] == kNegInf) ? 0.f : -m_run[nt];
       if (ALIBI) {
         const int iabs = diag + wrow0 + 32 * nt + l32;
-        float bg = m0 + slope2 * (float)(tile_of(j) * BKV + 4 * hi - iabs);
+        float bg = m0 + slope2 * (float)(tile_at(k, j) * BKV + 4 * hi - iabs);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -843,8 +869,8 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
   // The scores arrive as exponents relative to the reference max the row had
   // when S(j) was issued (the same m_run as now: nothing updates it between
   // an S tile's products and its softmax).
-  auto vpart = [&](int j, f32x16 (&s)[MT][NT], v8 (&pf)[NT][KS2]) {
-    const int kvb = tile_of(j) * BKV;
+  auto vpart = [&](auto k, int j, f32x16 (&s)[MT][NT], v8 (&pf)[NT][KS2]) {
+    const int kvb = tile_at(k, j) * BKV;
     const bool need_mask = (kvb + BKV > g.lk) || (causal && kvb + BKV - 1 > diag + wrow0) ||
                            (use_window && kvb < diag + wrow0 + 32 * NT - 1 - window_left);
     if (need_mask) {
@@ -977,7 +1003,7 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
   auto mphase = [&](auto last, int j, const v8 (&pf)[NT][KS2], f32x16 (&s)[MT][NT]) {
     constexpr bool LAST = decltype(last)::value;
     pv_mfma(j, pf);
-    if constexpr (!LAST) qk(j + 1 < j_hi ? j + 1 : j, s, j + 1);
+    if constexpr (!LAST) qk(Next{}, j + 1 < j_hi ? j + 1 : j, s, j + 1);
     // counted in instructions: an fp32 step is 8 MFMAs and its 32-byte
     // operand two 16-byte LDS reads
     constexpr int kMfma = (KS2 * MD * NT + (LAST ? 0 : KS * MT * NT)) * kMfmaPerStep<T>;
@@ -1013,19 +1039,19 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
     if constexpr (DMA) {
       dma_barrier(j);
       if constexpr (!kDmaMid)
-        if (j + kAhead < j_hi) tile_dma(j + kAhead);
+        if (j + kAhead < j_hi) tile_dma(j + kAhead, tile_at(Copied{}, j + kAhead));
       return;
     }
     if ((j - j_lo) % kBarrierEvery == kBarrierEvery - 1) ring_barrier();  // the prologue's barrier opens interval j_lo
-    if (j + kAhead < j_hi) tile_load_part(j + kAhead, 0);
+    if (j + kAhead < j_hi) tile_load_part(tile_at(Copied{}, j + kAhead), 0);
   };
   auto ring_mid = [&](int j) {
     if constexpr (kDmaMid) {
-      if (j + kAhead < j_hi) tile_dma(j + kAhead);
+      if (j + kAhead < j_hi) tile_dma(j + kAhead, tile_at(Copied{}, j + kAhead));
     } else if constexpr (SPLIT && !DMA) {
       if (j + kAhead < j_hi) {
         tile_store_part(j + kAhead, 0);
-        tile_load_part(j + kAhead, 1);
+        tile_load_part(tile_at(Copied{}, j + kAhead), 1);
       }
     }
   };
@@ -1035,23 +1061,94 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
   };
 
   // ---- prologue: tiles j_lo .. j_lo + kAhead - 1 resident, scores of tile j_lo --------
+  // With a caller's mask, the tiles to walk: lane w takes word w of the marks of
+  // the workgroup's rows, and every wave writes the whole list, the same words
+  // from each. Meanwhile the tiles that are the first if none is hidden are
+  // copied, and the q rows loaded. bf16, us, every tile walked / this: B=4,
+  // T=2048, 16/4 heads, D=128: half the tiles hidden 133 / 83, a prefix mask
+  // 137 / 130, nothing hidden 139 / 141; B=1, T=8192, 32/8 heads: six documents
+  // 470 / 139, nothing hidden 929 / 940; small ones up to 1 us more (T=300: 14.3 /
+  // 15.4). With the marks taken in this kernel and the list read from LDS three
+  // times a step, nothing hidden was 156, 1074 and 16.1.
+  if constexpr (MASK) {
+    const int ntl = j_hi;
+    if (ntl > 0) {
+      fill_walk(0);
+      if constexpr (DMA)
+        for (int t = 0; t < kAhead && t < ntl; ++t) tile_dma(t, tile_of(t));
+      const int w0 = first_tile / 64, nw = (first_tile + ntl - 1) / 64 - w0 + 1;
+      const bool marked = p.marks && nw <= kListTiles / 64;
+      uint64_t m = 0;
+      if (marked && lane < nw) {
+        const Marks k = marks_of(a, ntiles_k);
+        const int64_t bh = (int64_t)(a.mask_stride_b ? b : 0) * k.heads;
+#pragma unroll
+        for (int i = 0; i < WAVES; ++i) {
+          const int h = a.mask_stride_h ? hk * p.group + sl * hg + i % hg : 0;
+          const int block = a.mask_stride_q ? min(qr0 / 32 + i / hg, k.blocks - 1) : 0;
+          m |= p.marks[((bh + h) * k.blocks + block) * k.words + w0 + lane];
+        }
+        // the tiles of the walk alone
+        const int lo = first_tile - 64 * (w0 + lane), n = first_tile + ntl - 64 * (w0 + lane);
+        if (lo > 0) m &= ~0ull << lo;
+        if (n < 64) m &= ~0ull >> (64 - n);
+      }
+      load_q(std::integral_constant<int, 1>{});
+      if (marked) {
+        int upto = __popcll(m);
+        if (nw > 1) {
+#pragma unroll
+          for (int o = 1; o < 64; o <<= 1) {
+            const int t = __shfl_up(upto, o, 64);
+            if (lane >= o) upto += t;
+          }
+        }
+        const int total = __builtin_amdgcn_readlane(upto, nw - 1);
+        if (total < ntl) {
+          for (int w = 0; w < nw; ++w) {
+            const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)m, w), up = __builtin_amdgcn_readlane((uint32_t)(m >> 32), w);
+            const int before = __builtin_amdgcn_readlane(upto, w) - __popc(lo) - __popc(up);
+            const int at = before + (int)__builtin_amdgcn_mbcnt_hi(up, __builtin_amdgcn_mbcnt_lo(lo, 0));
+            if (((lane < 32 ? lo : up) >> l32) & 1u)
+              list[ALIBI ? total - 1 - at : at] = (uint16_t)(64 * (w0 + w) + lane - first_tile);
+          }
+          j_hi = total;
+          listed = true;
+          if (total > 0) fill_walk(0);
+          // The first tiles are others than those copied: again, behind this
+          // wave's earlier copies to the same places. No tile at all: every
+          // wave's copies are done with before the stages serve the outputs.
+          bool same = total > 0;
+          for (int t = 0; t < kAhead && t < total; ++t) same = same && tile_of(t) == first_tile + (ALIBI ? j_rev - t : t);
+          if (DMA && !same) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            for (int t = 0; t < kAhead && t < total; ++t) tile_dma(t, tile_of(t));
+          }
+          if (total == 0) __syncthreads();
+        }
+      }
+      if (j_hi > 0)
+        for (int t = 0; t <= kAhead; ++t) ahead[t] = tile_of(t);
+    }
+  }
   const int ntile = j_hi - j_lo;
   f32x16 s_a[MT][NT];
   v8 pf[NT][KS2];
   if (ntile > 0) {
     if constexpr (DMA) {
-      for (int t = 0; t < kAhead && t < ntile; ++t) tile_dma(j_lo + t);
-      load_q();
+      if constexpr (!MASK)
+        for (int t = 0; t < kAhead && t < ntile; ++t) tile_dma(j_lo + t, tile_of(j_lo + t));
+      load_q(std::integral_constant<int, MASK ? 2 : 0>{});
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     } else {
-      load_q();
+      load_q(std::integral_constant<int, MASK ? 2 : 0>{});
       for (int t = 0; t < kAhead && t < ntile; ++t) {
-        tile_load(j_lo + t);
+        tile_load(j_lo + t, tile_of(j_lo + t));
         tile_store(j_lo + t);
       }
     }
     ring_barrier();
-    qk(j_lo, s_a, j_lo);
+    qk(Now{}, j_lo, s_a, j_lo);
   }
 
   {
@@ -1062,20 +1159,25 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
     //   group 1: | MFMA(j)     softmax(j+1)  | MFMA(j+1)    ...
     // Both groups touch tiles j and j+1 in interval j, so the ring is the
     // same for both.
-    if (wave >= 4 && ntile > 0) vpart(j_lo, s_a, pf);
+    if (wave >= 4 && ntile > 0) vpart(Now{}, j_lo, s_a, pf);
     auto step = [&](auto last, int j) {
       ring_begin(j);
       if (wave < 4) {
-        vpart(j, s_a, pf);
+        vpart(Now{}, j, s_a, pf);
         ring_mid(j);
         mphase(last, j, pf, s_a);
       } else {
         mphase(last, j, pf, s_a);
         ring_mid(j);
         if constexpr (!decltype(last)::value)
-          if (j + 1 < j_hi) vpart(j + 1, s_a, pf);
+          if (j + 1 < j_hi) vpart(Next{}, j + 1, s_a, pf);
       }
       ring_end(j);
+      if constexpr (MASK) {
+#pragma unroll
+        for (int t = 0; t < kAhead; ++t) ahead[t] = ahead[t + 1];
+        ahead[kAhead] = tile_of(j + 1 + kAhead);
+      }
     };
     // Unrolled by the ring depth, so every stage address is a constant; the
     // last step is peeled at head_dim <= 128.
@@ -1083,6 +1185,9 @@ __device__ __forceinline__ void fa_item(const PrefillParams& p, unsigned char* s
     const std::false_type more{};
     const int nmid = kPeel ? ntile - 1 : ntile;
     for (int t = 0; t < nmid; t += kStages) {
+      // (the steps from t look at most kStages + kAhead ahead of it)
+      if constexpr (MASK && WALK)
+        if (t - walk0 >= 32) fill_walk(t);
       step(more, j_lo + t);
       if (t + 1 < nmid) step(more, j_lo + t + 1);
       if (t + 2 < nmid) step(more, j_lo + t + 2);
@@ -1378,6 +1483,14 @@ int64_t image_bytes(const goda_prefill_args& a) {
   return 2 * (int64_t)a.batch * ntiles * a.heads_kv * bkv * a.head_dim * elem;
 }
 
+// Marks of the caller's mask behind the images.
+int64_t marks_bytes(const goda_prefill_args& a) {
+  if (!a.mask_bits) return 0;
+  const int bkv = kv_tile_for(a.head_dim, a.dtype);
+  const Marks k = marks_of(a, (a.seqlen_k + bkv - 1) / bkv);
+  return (int64_t)k.batch * k.heads * k.blocks * k.words * 8;
+}
+
 // Workgroups of `kern` resident on the whole device at once (cached per
 // device and kernel).
 hipError_t resident_slots(const void* kern, int threads, size_t lds, int* out) {
@@ -1566,7 +1679,14 @@ hipError_t launch_d(PrefillParams p, hipStream_t s) {
   p.ntiles_k = (a.seqlen_k + BKV - 1) / BKV;
   if (p.ntiles_k > 0) {
     dim3 grid(p.ntiles_k, a.heads_kv, a.batch);
-    pack_kv_kernel<T, D, BKV><<<grid, 256, 0, s>>>(p);
+    if (a.mask_bits && a.workspace_bytes >= image_bytes(a) + marks_bytes(a)) {
+      p.marks = reinterpret_cast<uint64_t*>(reinterpret_cast<unsigned char*>(a.workspace) + image_bytes(a));
+      const int64_t waves = marks_bytes(a) / 8 / ((p.ntiles_k + 63) / 64), rows = (int64_t)a.heads_kv * a.batch;
+      grid.x += (unsigned)((waves + 4 * rows - 1) / (4 * rows));
+      pack_kv_kernel<T, D, BKV, true><<<grid, 256, 0, s>>>(p);
+    } else {
+      pack_kv_kernel<T, D, BKV, false><<<grid, 256, 0, s>>>(p);
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
@@ -1601,7 +1721,7 @@ int64_t prefill_mfma_least_bytes(const goda_prefill_args& a) { return image_byte
 
 int64_t prefill_mfma_workspace_bytes(const goda_prefill_args& a) {
   const KeyPieces k = key_pieces(a);
-  return image_bytes(a) + (k.ksplit > 1 ? k.items * k.ksplit * piece_bytes(a.head_dim) : 0);
+  return image_bytes(a) + marks_bytes(a) + (k.ksplit > 1 ? k.items * k.ksplit * piece_bytes(a.head_dim) : 0);
 }
 
 hipError_t launch_prefill_mfma(const PrefillParams& p, hipStream_t s) {

@@ -237,6 +237,40 @@ def test_mask_of_hidden_tiles(dtype, d, causal, alibi, tk):
     assert lse_err(lse, lse_ref) <= (5e-3 if dtype != torch.float32 else 1e-4) * max(1.0, tk / 300 if alibi else 1.0)
 
 
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.float16, 128), (torch.bfloat16, 256), (torch.float32, 128)])
+@pytest.mark.parametrize("alibi", [False, True])  # (the walk downwards)
+@pytest.mark.parametrize("form", ["rows", "per_head", "keys", "window"])
+@pytest.mark.parametrize("hidden", ["first", "all but one", "half", "every"])
+def test_mask_of_many_tiles(dtype, d, alibi, form, hidden):
+    """Lists of more than 64 tiles (several words of marks, several fills of the
+    walk's register), for masks by row, by head and row, and by key alone, from
+    the first tile of the sequence and from one inside a word; the first tiles
+    hidden, one tile left, every second, and none. In a workspace without room
+    for the marks every tile is walked: the same result."""
+    tq, tk, hq, hkv = 72, 8300, 4, 2
+    if dtype == torch.float32:
+        tq, hq = 800, 128  # (more than 3072 tiles of rows: the LDS ring)
+    mq = 1 if form == "keys" or (form == "per_head" and hq > 4) else tq
+    g = torch.Generator().manual_seed(d)
+    q, k, v = (torch.randn(1, t, h, d, generator=g).to(dtype) for t, h in ((tq, hq), (tk, hkv), (tk, hkv)))
+    tile = torch.arange(tk) // 32
+    seen = {"first": tile >= 140, "all but one": tile == 200, "half": tile % 4 < 2, "every": tile < 0}[hidden]
+    mask = seen & (torch.rand(1, hq if form == "per_head" else 1, mq, tk, generator=g) < 0.9)
+    kw = dict(causal=form == "window", window_left=3000 if form == "window" else -1)
+    slopes = torch.tensor([2.0 ** -(4 + i % 8) for i in range(hq)]) if alibi else None
+    plan = ops.plan_prefill(q.to(DEV), k.to(DEV), v.to(DEV), attn_mask=mask.to(DEV),
+                            alibi_slopes=None if slopes is None else slopes.to(DEV), **kw)
+    o = plan().clone()
+    rows = torch.tensor([0, 31, 32, tq - 1])
+    want, _ = ref.attention_rows(q.float(), k.float(), v.float(), rows, base_attn_mask=mask, alibi_slopes=slopes, **kw)
+    assert max_err(o[:, rows.to(DEV)], torch.nan_to_num(want)) <= TOL[dtype]
+    images = 2 * 8320 * hkv * d * q.element_size()
+    assert plan.args.workspace_bytes > images
+    plan.args.workspace_bytes = images
+    plan.result.zero_()
+    assert max_err(plan(), o) <= TOL[dtype]
+
+
 def test_mask_over_more_tiles_than_the_list_holds():
     """Over 4096 key tiles every tile is walked; one key tile in 50 is visible."""
     tk, d = 64 * 4096 + 40, 64
