@@ -429,16 +429,19 @@ __device__ __forceinline__ void grid_item(const PrefillParams& p, const int lin,
   // group, pair after pair, heaviest tile first: every XCD stays within ~3%
   // of the mean, and the XCDs work on the same pair at the same time, so each
   // XCD's L2 still serves one pair's K/V stream to all its workgroups.
-  // XCDs sharing one pair's query tiles: fewer where a pair has fewer (packed_tiles)
-  const int kXg = min(nqt, kVarlenXcdGroup);
+  // XCDs sharing one pair's query tiles (a power of two: shifts): fewer where a
+  // pair has fewer (packed_tiles).
+  static_assert(kVarlenXcdGroup == 8, "log2 below");
+  const int log_xg = nqt >= kVarlenXcdGroup ? 3 : nqt >= 4 ? 2 : nqt >= 2 ? 1 : 0;
+  const int kXg = 1 << log_xg;
   const int npairs = nblk / nqt;
-  if (a.cu_seqlens_q && nblk % 8 == 0 && nqt % kXg == 0 && npairs % (8 / kXg) == 0) {
+  if (a.cu_seqlens_q && nblk % 8 == 0 && (nqt & (kXg - 1)) == 0 && (npairs & ((8 >> log_xg) - 1)) == 0) {
     const int x = lin % 8, s = lin / 8;
-    const int per = nqt / kXg;                 // query tiles of one pair on one XCD
-    pair = s / per * (8 / kXg) + x / kXg;      // place in the walk
+    const int per = nqt >> log_xg;                               // query tiles of one pair on one XCD
+    pair = (s / per << (3 - log_xg)) + (x >> log_xg);            // place in the walk
     // Short sequences: turned by the pair's place in the walk (kRotateTiles).
     const bool rotate = per <= kRotateTiles;
-    qt = (per - 1 - s % per) * kXg + (x + (rotate ? pair : 0)) % kXg;
+    qt = ((per - 1 - s % per) << log_xg) + ((x + (rotate ? pair : 0)) & (kXg - 1));
     if (a.batch <= 64) {
       // Longest sequences first, so the heaviest tiles are not the last ones
       // dispatched: position `pair` in the walk is served by the sequence of
@@ -512,7 +515,7 @@ __device__ __forceinline__ void grid_item(const PrefillParams& p, const int lin,
           return;
         }
         pair = __builtin_ctzll(hit) * per_seq + j % per_seq;
-        qt = (per - 1 - lo) * kXg + x % kXg;
+        qt = ((per - 1 - lo) << log_xg) + (x & (kXg - 1));
       }
     }
   } else {
