@@ -123,6 +123,8 @@ int64_t prefill_mfma_workspace_bytes(const goda_prefill_args& a);
 // all tiles are walked).
 int64_t prefill_mfma_least_bytes(const goda_prefill_args& a);
 hipError_t launch_prefill_mfma(const PrefillParams& p, hipStream_t s);
+// Workgroups of a dense launch (8 waves of 32 query rows each).
+int64_t prefill_mfma_workgroups(const goda_prefill_args& a);
 
 // fp32 prefill on the matrix cores with operands streamed from L2: head_dim
 // 256 (more than two key tiles), and 64 / 128 where the work is small.

@@ -404,14 +404,35 @@ hipError_t launch_d(PrefillParams p, hipStream_t s) {
 //   items 3072  B=3 T=2048 16/16 D=64       319 / 299
 //   items 4096  B=8 T=512 32/8 D=128        177 / 213
 //   items 4096  B=8 T=1024 16/16 D=64       204 / 232
+// Not so where the ring's workgroups are one whole round of equal work and an
+// item's walk here is shared by its waves: full attention over 1024 keys or more
+// (fewer: 148 / 148 at T=512 below, 87 / 84 at T=256):
+//   B=1 T=2048 32/8 D=128    509 / 547        B=1 T=1856 32/8 D=128   461 / 498
+//   B=2 T=8192 4/4 D=64     1021 / 1103       B=1 T=1792 32/8 D=128   445 / 424
+//   B=2 T=1024 32/8 D=128    269 / 286        B=1 T=2304 32/8 D=128  1111 / 688
 // At head_dim 256, which has no ring instance, they replace the vector-ALU
-// kernel (B=8, T=4096, 16/1 heads, ALiBi: 38.0 -> 8.7 ms) but for calls of
-// at most two key tiles, which that one runs without a pre-pass.
+// kernel (B=8, T=4096, 16/1 heads, ALiBi: 38.0 -> 8.7 ms), which has no pre-pass
+// and reads k and v once for 64 rows of a head. It stays for calls of at most
+// two key tiles, and for at most 64 rows of heads with keys of their own, over
+// walks too short to share, where it fills the GPU (512 workgroups at once) as
+// well as this one; us, vector ALUs / here, 16/16 heads:
+//   B=256, 4 rows on 70 keys    614 / 672     B=96, 1 row on 256 keys    1 / 1.06
+//   B=256, 4 on 200            1415 / 1608    B=80, 64 on 896            1 / 0.96
+//   B=64, 64 on 70              170 / 184     B=48, 64 on 256            1 / 0.86
+//   B=64, 64 on 992             1 / 1.14      B=64, 33 on 1024           1 / 0.85
 bool prefill_f32_streams(const goda_prefill_args& a) {
   if (a.dtype != GODA_DTYPE_F32) return false;
-  if (a.head_dim == 256) return a.seqlen_k > 2 * kF32Rows;
   const int64_t items = (int64_t)((a.seqlen_q + kF32Rows - 1) / kF32Rows) * a.heads_q * a.batch;
-  return items <= 3072;
+  const bool shared = f32_key_split(a, items) > 1;
+  if (a.head_dim == 256) {
+    if (a.seqlen_k <= 2 * kF32Rows) return false;
+    if (a.heads_q != a.heads_kv || a.seqlen_q > 64 || shared) return true;
+    const int64_t wgs = (int64_t)a.heads_q * a.batch, rounds = (wgs + 511) / 512;
+    return 8 * wgs < 7 * 512 * rounds;
+  }
+  if (items > 3072) return false;
+  const bool equal = !a.causal && !a.cu_seqlens_q && !a.seqused_k;
+  return !(equal && shared && items > 7 * 256 && prefill_mfma_workgroups(a) <= 256);
 }
 
 int64_t prefill_f32_workspace_bytes(const goda_prefill_args& a) {

@@ -1562,7 +1562,7 @@ KeyPieces key_pieces(const goda_prefill_args& a) {
   const int rows = 8 / hg * 32;
   const int nqt = (a.seqlen_q + rows - 1) / rows;
   const int64_t per_qt = (int64_t)a.batch * a.heads_kv * (group / hg);
-  k.items = per_qt * nqt;
+  k.items = prefill_mfma_workgroups(a);
   // (lengths on the device may all be short: fewer items, so that little is lost)
   const bool long_keys = a.seqlen_k >= 4096;
   if (a.seqused_k ? k.items > (long_keys ? 64 : 48) || a.seqlen_k < 2048
@@ -1718,6 +1718,12 @@ bool prefill_mfma_supported(const goda_prefill_args& a) {
   if (a.dtype == GODA_DTYPE_F32) return a.head_dim == 64 || a.head_dim == 128;
   if (a.dtype != GODA_DTYPE_BF16 && a.dtype != GODA_DTYPE_F16) return false;
   return a.head_dim == 64 || a.head_dim == 128 || a.head_dim == 256;
+}
+
+int64_t prefill_mfma_workgroups(const goda_prefill_args& a) {
+  const int group = a.heads_q / a.heads_kv, hg = gcd_int(group, 8);
+  const int rows = 8 / hg * 32;
+  return (int64_t)((a.seqlen_q + rows - 1) / rows) * a.batch * a.heads_kv * (group / hg);
 }
 
 int64_t prefill_mfma_least_bytes(const goda_prefill_args& a) { return image_bytes(a); }

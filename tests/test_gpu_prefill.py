@@ -462,6 +462,27 @@ def _run_rows(b, tq, tk, hq, hkv, d, causal):
     assert max_err(o[:, rows.to(DEV)], o_ref) <= TOL[torch.float32]
 
 
+@pytest.mark.parametrize("d,b,tq,tk,hq,hkv", [
+    (64, 1, 1024, 1024, 64, 16),  # full attention in one whole round of the ring's workgroups
+    (128, 1, 1024, 1024, 64, 16),
+    (128, 1, 1000, 1050, 56, 14),  # one that is not whole: streamed
+    (256, 128, 40, 70, 4, 4),  # few rows of heads with keys of their own, a whole round: the vector ALUs
+    (256, 8, 64, 900, 64, 64),
+    (256, 8, 65, 200, 64, 64),  # more rows, a longer walk, a round that is not whole: streamed
+    (256, 8, 64, 1024, 64, 64),
+    (256, 5, 40, 70, 64, 64),
+    (256, 128, 20, 70, 4, 4),  # 512 tiles of rows: walks shared by the waves
+])
+def test_prefill_fp32_rounds_of_equal_work(d, b, tq, tk, hq, hkv):
+    """Both sides of the rules for calls that fill the GPU in whole rounds; a
+    workspace is asked for unless the vector ALUs take the call."""
+    _run_rows(b, tq, tk, hq, hkv, d, False)
+    q, k = torch.empty(b, tq, hq, d, device=DEV), torch.empty(b, tk, hkv, d, device=DEV)
+    size = ops.plan_prefill(q, k, k, causal=False).args.workspace_bytes
+    vector = d == 256 and 32 < tq <= 64 and tk < 1024 and b * hq == 512
+    assert (size == 0) == vector
+
+
 @pytest.mark.parametrize("tk", [64, 65, 200])
 def test_prefill_fp32_wide_without_workspace(tk):
     """fp32 at head_dim 256: a call without a workspace gives the same result
