@@ -570,13 +570,14 @@ def test_prefill_split_keys_with_room_for_the_images_alone(d):
 
 
 @pytest.mark.parametrize("dtype,d,hq,hkv", [(torch.float16, 64, 4, 4), (torch.bfloat16, 128, 8, 2), (torch.bfloat16, 256, 8, 1)])
-@pytest.mark.parametrize("tiles", [1, 8, 9, 16, 17])  # query tiles of the longest sequence
-@pytest.mark.parametrize("batch", [1, 5, 65])  # 65: no ranks
+@pytest.mark.parametrize("tiles", [1, 2, 3, 4, 8, 9, 16, 17])  # query tiles of the longest sequence
+@pytest.mark.parametrize("batch", [1, 5, 8, 65, 72])  # over 64: no ranks; 8, 72: pairs for grids of 1, 2 and 4 tiles
 def test_packed_short_sequences_cover_every_tile(dtype, d, hq, hkv, tiles, batch):
     """Packed launches whose query tiles are turned over the XCDs (up to 16 a
-    sequence) and the next size: every row of every sequence against a launch of
-    that sequence alone (the same sums in the same order, or cut along the keys:
-    one rounding of the output apart)."""
+    sequence), grids of 1, 2 and 4 tiles a pair among them, and the next size:
+    every row of every sequence against a launch of that sequence alone (the
+    same sums in the same order, or cut along the keys: one rounding of the
+    output apart)."""
     group = hq // hkv
     rows = 8 // min(group, 8) * 32
     longest = rows * (tiles - 1) + 1
@@ -586,7 +587,7 @@ def test_packed_short_sequences_cover_every_tile(dtype, d, hq, hkv, tiles, batch
     starts = [sum(lens[:i]) for i in range(batch + 1)]
     cu = torch.tensor(starts, dtype=torch.int32, device=DEV)
     o = ops.attention_prefill(q, k, v, causal=True, cu_seqlens_q=cu, cu_seqlens_k=cu, max_seqlen_q=longest, max_seqlen_k=longest)
-    for i in range(min(batch, 12)):
+    for i in range(batch):
         if lens[i] == 0:
             continue
         s = slice(starts[i], starts[i + 1])
