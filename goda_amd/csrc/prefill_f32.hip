@@ -15,7 +15,7 @@
 //
 // An item (32 query rows of one head) is walked by key_split waves of a
 // workgroup of four, wave w taking every key_split-th key tile; they add up in
-// LDS at the end. See launch_attn for its choice.
+// LDS at the end (f32_key_split, launch.h, chooses).
 
 #include "common.h"
 #include "f32_tile.h"

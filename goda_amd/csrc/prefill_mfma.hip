@@ -142,19 +142,19 @@ constexpr int kPieceRows = 256;  // 8 waves of 32 rows
 template <int D>
 constexpr int64_t kPieceBytes = (int64_t)kPieceRows * (D + 2) * 4;
 constexpr int kCus = 256;
+constexpr int kMostPieceBatch = 64;
 
 // Key tiles per piece for this launch: p.piece_tiles, or (lengths on the
-// device) an equal share of all items' tiles, at least what keeps the longest
-// sequence to p.ksplit pieces.
+// device, of at most 64 sequences: key_pieces) an equal share of all items'
+// tiles, at least what keeps the longest sequence to p.ksplit pieces.
 __device__ __forceinline__ int piece_tiles(const PrefillParams& p, int bkv) {
   if (p.piece_tiles > 0) return p.piece_tiles;
   const goda_prefill_args& a = p.a;
   const int lane = threadIdx.x & 63;
-  long long tiles = 0;
-  for (int i = lane; i < a.batch; i += 64) tiles += (max(0, min(a.seqused_k[i], a.seqlen_k)) + bkv - 1) / bkv;
+  int sum = lane < a.batch ? (max(0, min(a.seqused_k[lane], a.seqlen_k)) + bkv - 1) / bkv : 0;
 #pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) tiles += __shfl_xor(tiles, o, 64);
-  tiles *= (long long)p.qtiles * a.heads_kv * (p.group / p.heads_per_wg);
+  for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, 64);
+  const long long tiles = (long long)sum * p.qtiles * a.heads_kv * (p.group / p.heads_per_wg);
   const int share = (int)min((long long)p.ntiles_k, (tiles + kCus - 1) / kCus);
   return max(max(share, p.min_piece), (p.ntiles_k + p.ksplit - 1) / p.ksplit);
 }
@@ -1563,9 +1563,13 @@ KeyPieces key_pieces(const goda_prefill_args& a) {
   const int nqt = (a.seqlen_q + rows - 1) / rows;
   const int64_t per_qt = (int64_t)a.batch * a.heads_kv * (group / hg);
   k.items = prefill_mfma_workgroups(a);
-  // (lengths on the device may all be short: fewer items, so that little is lost)
+  // Lengths on the device, seen by the host as the capacity alone: where they are
+  // all short nothing is cut, and the second launch and the reading of the
+  // lengths cost 3 to 4 us a call (capacity 8192: 8 x 16 rows on 256 keys 26 / 30,
+  // on 1024 44 / 48, on 2048 68 / 60), so fewer items.
   const bool long_keys = a.seqlen_k >= 4096;
-  if (a.seqused_k ? k.items > (long_keys ? 64 : 48) || a.seqlen_k < 2048
+  static_assert(kMostPieceBatch == 64, "piece_tiles reads the lengths of 64 sequences, and an item is of one");
+  if (a.seqused_k ? k.items > (long_keys ? kMostPieceBatch : 48) || a.seqlen_k < 2048
                   : k.items > (a.head_dim == 64 ? 64 : long_keys ? 128 : 96))
     return k;
   const int diag = a.seqlen_k - a.seqlen_q;

@@ -432,8 +432,7 @@ def _norm_case(b, tq, tk, hq, hkv, d, dtype, *, rope, seed, varlen_lens=None):
 def test_backward_fused_qk_norm(dtype, d, rope):
     """The fused QK-RMSNorm (goda's RMSNorm before RoPE, mint/nn/attn.py:57-60)
     through the backward: dq / dk of the rows before the norm and both scales'
-    gradients against the oracle's autograd (fp32 at head_dim 256 runs the
-    generic kernels over materialized normalized rows)."""
+    gradients against the oracle's autograd."""
     _norm_case(2, 96, 96, 8, 2, d, dtype, rope=rope, seed=41)
 
 

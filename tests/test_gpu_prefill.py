@@ -192,7 +192,7 @@ def test_prefill_varlen(dtype, d, hq, hkv):
 def test_prefill_alibi_varlen_window(dtype, d, hq, hkv, window):
     """ALiBi walks each item's key tiles from the last down; with packed
     sequences and a left window the walk starts and ends away from tile 0.
-    (fp32 at head_dim 256 takes the generic kernel, checked the same way.)"""
+    (fp32 at head_dim 256 streams its operands, checked the same way.)"""
     lens = [1, 37, 64, 65, 300, 129, 5]
     cu = torch.zeros(len(lens) + 1, dtype=torch.int32)
     cu[1:] = torch.cumsum(torch.tensor(lens), 0)
@@ -525,7 +525,12 @@ def test_prefill_fp32_wide_large_values(tk):
 ])
 def test_prefill_split_keys(dtype, d, b, tq, tk, hq, hkv, causal, window, alibi):
     """Batches of few items, whose keys are cut into pieces added up by a second
-    launch."""
+    launch; the workspace has room for them."""
+    q, k = torch.empty(b, tq, hq, d, dtype=dtype, device=DEV), torch.empty(b, tk, hkv, d, dtype=dtype, device=DEV)
+    plan = ops.plan_prefill(q, k, k, causal=causal, window_left=window)
+    tile = 64 if d <= 128 else 32
+    images = 2 * b * (-(-tk // tile) * tile) * hkv * d * 2
+    assert (plan.args.workspace_bytes > images) == (window != 40)
     _run_case(b, tq, tk, hq, hkv, d, dtype, causal, seed=tq, window=window, alibi=alibi, rope=not alibi)
 
 
@@ -533,11 +538,15 @@ def test_prefill_split_keys(dtype, d, b, tq, tk, hq, hkv, causal, window, alibi)
 @pytest.mark.parametrize("lens", [[1500, 3, 700, 0, 1499], [2000], [40, 40, 40], [1025] + [17] * 69])
 def test_prefill_split_keys_lengths_on_the_device(dtype, d, hq, hkv, lens):
     """Key counts read on the device: sequences cut into several pieces, one, or
-    none, an empty one, and more than 64 of them; rows with no key give 0."""
+    none, and an empty one; rows with no key give 0. 70 sequences are too many
+    items to cut, whatever their lengths."""
     b, tq, tk = len(lens), 33, 2048
     q, k, v = _rand((b, tq, hq, d), dtype, 1), _rand((b, tk, hkv, d), dtype, 2), _rand((b, tk, hkv, d), dtype, 3)
     used = torch.tensor(lens, dtype=torch.int32)
-    o, lse = ops.attention_prefill(q.to(DEV), k.to(DEV), v.to(DEV), causal=True, seqused_k=used.to(DEV), return_lse=True)
+    plan = ops.plan_prefill(q.to(DEV), k.to(DEV), v.to(DEV), causal=True, seqused_k=used.to(DEV), return_lse=True)
+    images = 2 * b * tk * hkv * d * 2
+    assert (plan.args.workspace_bytes > images) == (b <= 5)  # (cut, where a length asks for it)
+    o, lse = plan()
     for i, n in enumerate(lens):
         first = max(0, tq - n)  # bottom-right: these rows see no key
         assert torch.count_nonzero(o[i, :first]) == 0 and bool(torch.isneginf(lse[i, :, :first]).all())
